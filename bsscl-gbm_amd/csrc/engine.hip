@@ -257,6 +257,14 @@ using namespace bsscl;
 namespace {
 constexpr int32_t kNoAllocMaxNodes = 1 << 17;   // nodes of all trees of a call
 constexpr int32_t kNoAllocMaxTrees = 1 << 14;
+constexpr int32_t kNoAllocMaxCols = 4096;       // columns the walk can renumber
+// What launch_walk_pack and launch_walk read beside the nodes, one class.
+struct WalkLists {
+  int32_t first[kNoAllocMaxTrees + 8], count[kNoAllocMaxTrees + 8];
+  int32_t class_slots[2];
+  int32_t cols[kWalkMaxCols + 1];
+  uint8_t remap[kNoAllocMaxCols];
+};
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t kScrNodes = 0;
 constexpr size_t kScrFeat = kScrNodes + align256(sizeof(TreeNodeDev) * kNoAllocMaxNodes);
@@ -265,8 +273,12 @@ constexpr size_t kScrVal = kScrThr + align256(sizeof(int64_t) * kNoAllocMaxNodes
 constexpr size_t kScrLeft = kScrVal + align256(sizeof(double) * kNoAllocMaxNodes);
 constexpr size_t kScrRight = kScrLeft + align256(sizeof(int32_t) * kNoAllocMaxNodes);
 constexpr size_t kScrOffs = kScrRight + align256(sizeof(int32_t) * kNoAllocMaxNodes);
-constexpr size_t kScrChunks = kScrOffs + align256(sizeof(int32_t) * (kNoAllocMaxTrees + 1));
-constexpr size_t kScratchBytes = kScrChunks + align256(sizeof(int32_t) * (kNoAllocMaxTrees + 1));
+constexpr size_t kScrLists = kScrOffs + align256(sizeof(int32_t) * (kNoAllocMaxTrees + 1));
+constexpr size_t kScratchBytes = kScrLists + align256(sizeof(WalkLists));
+// The packed arrays are dead once the traversal nodes are made: the walk's
+// values and words take their place.
+constexpr size_t kScrWalk = kScrFeat;
+constexpr int64_t kNoAllocWalkSlots = (int64_t)((kScrOffs - kScrWalk) / 12 / 2 * 2);
 static_assert(kScratchBytes <= (7u << 20), "noalloc scratch stays under 7 MiB");
 constexpr int kMaxDevices = 64;
 }  // namespace
@@ -452,7 +464,12 @@ struct bsscl_engine {
   bool pipeline = false;   // enqueue the next round before returning one
   int32_t ahead = -1;      // slot of a round enqueued ahead, or -1
   uint64_t round_seq = 0;
-  DevBuf<int32_t> offsets_d;
+  // An ensemble's nodes and lists (upload_ensemble), and its packed form for
+  // the walk in LDS.
+  TempBuf<char> ens_d;
+  std::vector<uint8_t> child_marks;  // host work space of its checks
+  TempBuf<uint32_t> walk_words;
+  TempBuf<double> walk_vals;
   DevBuf<double> partials_d, loss_d, out_d, proba_d;
   PinnedArena pin;
   // Large host transfers go through these pinned chunks (host_upload,
@@ -2878,86 +2895,242 @@ hipStream_t copy_stream(int device) {
 namespace bsscl {
 namespace {
 
-// The ensemble's F of matrix `slot` into E->out_d (est:863-884).
-// The packed trees (est:2192-2216) on the device in the engine's columns of
-// matrices with M's features and tiers: tree_d, and offsets_d with, for the
-// LDS-staged walk (*staged), its *n_chunks runs of whole trees after them.
-int upload_trees(bsscl_engine *E, const Matrix &M, const int16_t *features,
-                 const int64_t *thresholds, const double *values, const int32_t *left,
-                 const int32_t *right, const int32_t *offsets, int32_t n_trees, bool *staged_out,
-                 int32_t *n_chunks_out) {
-  const int32_t total = n_trees > 0 ? offsets[n_trees] : 0;
-  std::vector<TreeNodeDev> nodes((size_t)std::max(total, 1));
-  bool adjacent = true;  // every right child is its left child + 1
-  for (int32_t t = 0; t < n_trees; ++t) {
-    const int32_t a = offsets[t], b = offsets[t + 1];
-    if (a < 0 || b <= a || b > total) return set_error(BSSCL_EINVAL, "predict: bad offsets");
-    for (int32_t i = a; i < b; ++i) {
-      TreeNodeDev &d = nodes[(size_t)i];
-      d.value = values[i];
-      d.feature = features[i];
-      if (d.feature >= 0) {
-        const int32_t l = left[i], r = right[i];
-        if (d.feature >= M.F || l < 0 || r < 0 || l >= b - a || r >= b - a || l <= i - a || r <= i - a)
-          return set_error(BSSCL_EINVAL, "predict: malformed tree " + std::to_string(t));
-        adjacent = adjacent && r == l + 1;
-        int64_t thr = thresholds[i];
-        split_to_engine(M, d.feature, thr);
-        d.threshold = (int32_t)std::max<int64_t>(-1, std::min<int64_t>(thr, 1 << 20));
-        d.left = l;
-        d.right = r;
-      } else {
-        d.feature = -1;
-        d.threshold = 0;
-        d.left = d.right = 0;
-      }
+// Packed trees (est:2192-2216) of K classes, class k's arrays at index k.
+struct PackedTrees {
+  int32_t K;
+  const int16_t *const *features;
+  const int64_t *const *thresholds;
+  const double *const *values;
+  const int32_t *const *left;
+  const int32_t *const *right;
+  const int32_t *const *offsets;
+  const int32_t *n_trees;
+};
+
+// What the walk needs to know of an ensemble: its largest tree, the columns
+// it splits on, and whether every node has one parent (then a tree has as
+// many nodes breadth first as in its arrays).
+struct TreeShape {
+  int32_t max_nodes = 1;
+  bool proper = true;
+  std::vector<uint8_t> used;  // by engine column
+  int32_t n_used = 0;
+  void use(int32_t col) {
+    n_used += used[(size_t)col] ? 0 : 1;
+    used[(size_t)col] = 1;
+  }
+  // The used columns in ascending order (at least one) and every column's
+  // index among them.
+  void columns(int32_t *cols, uint8_t *remap) const {
+    int32_t k = 0;
+    cols[0] = 0;
+    for (size_t c = 0; c < used.size(); ++c) {
+      remap[c] = (uint8_t)k;
+      if (used[c]) cols[k++] = (int32_t)c;
     }
   }
-  CHK(E->pin.reserve(std::max<size_t>(E->pin.cap, 8u << 20)));
-  // The offsets, then (for the LDS-staged kernel) the runs of whole trees it
-  // stages at a time.
-  int32_t max_nodes = 0;
-  for (int32_t t = 0; t < n_trees; ++t) max_nodes = std::max(max_nodes, offsets[t + 1] - offsets[t]);
-  // (Test hook BSSCL_TEST_PREDICT_GLOBAL=1: every row walks the trees in HBM.)
-  const bool staged = n_trees > 0 && predict_staged_ok(M.cols(), max_nodes, adjacent) &&
-                      !std::getenv("BSSCL_TEST_PREDICT_GLOBAL");
-  // (A model without trees may pass no arrays at all: offsets is read only
-  // when there are trees.)
-  std::vector<int32_t> offs((size_t)n_trees + 1, 0);
-  if (n_trees > 0) std::copy(offsets, offsets + n_trees + 1, offs.begin());
-  int32_t n_chunks = 0;
-  if (staged) {
-    offs.resize(2 * ((size_t)n_trees + 1));
-    n_chunks = predict_chunks(offsets, n_trees, offs.data() + n_trees + 1);
+};
+
+// (Test hook BSSCL_TEST_PREDICT_GLOBAL=1: every row walks the trees in HBM.)
+bool plan_walk(const TreeShape &sh, int64_t n, WalkPlan *plan) {
+  return sh.proper && !std::getenv("BSSCL_TEST_PREDICT_GLOBAL") &&
+         walk_plan(n, std::max(1, sh.n_used), sh.max_nodes, plan);
+}
+
+// An ensemble on the device: the nodes in the engine's columns, class k's
+// tree t at offsets[first_tree[k] + t]; for the walk in LDS also its plan,
+// lists and packed words and values (E->walk_words, E->walk_vals).
+struct Ensemble {
+  int32_t K = 0;
+  double lr = 0.0;
+  bool walk = false;
+  WalkPlan plan{};
+  std::vector<int32_t> first_tree;
+  const TreeNodeDev *nodes = nullptr;
+  const int32_t *offsets = nullptr;
+  const int32_t *cols = nullptr, *class_slots = nullptr;
+};
+
+// Checks the trees for matrices with M's features and tiers, uploads them
+// with their lists in one copy and packs them for a walk of n rows.
+int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, double lr, int64_t n,
+                    Ensemble *out) {
+  size_t total = 0, trees = 0;
+  for (int32_t k = 0; k < P.K; ++k) {
+    // (Offsets first: the arrays' sizes follow from them.)
+    for (int32_t t = 0; t < P.n_trees[k]; ++t)
+      if (P.offsets[k][t] < 0 || P.offsets[k][t + 1] <= P.offsets[k][t])
+        return set_error(BSSCL_EINVAL, "predict: bad offsets");
+    if (P.n_trees[k] > 0) total += (size_t)P.offsets[k][P.n_trees[k]];
+    trees += (size_t)P.n_trees[k];
   }
-  CHK(upload(E, E->tree_d, nodes.data(), nodes.size()));
-  CHK(upload(E, E->offsets_d, offs.data(), offs.size()));
-  *staged_out = staged;
-  *n_chunks_out = n_chunks;
+  Ensemble &en = *out;
+  en.K = P.K;
+  en.lr = lr;
+  TreeShape sh;
+  sh.used.assign((size_t)M.cols(), 0);
+  // Built in pinned memory and copied from there: nodes, tree offsets, then
+  // the walk's lists (first node and node count of every slot, the classes'
+  // slots, the staged columns, every column's index among them).
+  const size_t off_b = std::max<size_t>(total, 1) * sizeof(TreeNodeDev);
+  const size_t list_b = off_b + (trees + 1) * 4;
+  const size_t slots_max = trees + (size_t)P.K * (kWalkMaxGroup + kWalkMaxTpl);
+  const size_t cols_max = (size_t)M.cols();
+  const size_t bytes_max =
+      list_b + (2 * slots_max + 2 * (size_t)P.K + cols_max + 1) * 4 + cols_max;
+  const size_t pin_b = std::max<size_t>(bytes_max + 512, 8u << 20);
+  if (pin_b > E->pin.cap) HIPCHK(hipStreamSynchronize(E->st));
+  CHK(E->pin.reserve(std::max(E->pin.cap, pin_b)));
+  char *stage = E->pin.take<char>(bytes_max);
+  if (!stage) {  // the arena's earlier copies first
+    CHK(sync(E));
+    stage = E->pin.take<char>(bytes_max);
+  }
+  TreeNodeDev *nodes = reinterpret_cast<TreeNodeDev *>(stage);
+  int32_t *offs = reinterpret_cast<int32_t *>(stage + off_b);
+  std::vector<uint8_t> &child = E->child_marks;
+  child.assign(std::max<size_t>(total, 1), 0);
+  en.first_tree.assign((size_t)P.K + 1, 0);
+  size_t base = 0;   // class k's first node
+  int32_t tree = 0;  // and tree
+  for (int32_t k = 0; k < P.K; ++k) {
+    const int32_t nt = P.n_trees[k];
+    const int32_t *offsets = P.offsets ? P.offsets[k] : nullptr;
+    // (A class without trees may pass no arrays at all.)
+    const int32_t tot = nt > 0 ? offsets[nt] : 0;
+    for (int32_t t = 0; t < nt; ++t) {
+      const int32_t a = offsets[t], b = offsets[t + 1];
+      offs[(size_t)tree++] = (int32_t)base + a;
+      sh.max_nodes = std::max(sh.max_nodes, b - a);
+      for (int32_t i = a; i < b; ++i) {
+        TreeNodeDev d;
+        d.value = P.values[k][i];
+        d.feature = P.features[k][i];
+        if (d.feature >= 0) {
+          const int32_t l = P.left[k][i], r = P.right[k][i];
+          if (d.feature >= M.F || l < 0 || r < 0 || l >= b - a || r >= b - a || l <= i - a ||
+              r <= i - a)
+            return set_error(BSSCL_EINVAL, "predict: malformed tree " + std::to_string(t));
+          uint8_t &lc = child[base + (size_t)(a + l)], &rc = child[base + (size_t)(a + r)];
+          sh.proper = sh.proper && !lc && !rc && l != r;
+          lc = rc = 1;
+          int64_t thr = P.thresholds[k][i];
+          split_to_engine(M, d.feature, thr);
+          d.threshold = (int32_t)std::max<int64_t>(-1, std::min<int64_t>(thr, 1 << 20));
+          d.left = l;
+          d.right = r;
+          sh.use(d.feature);
+        } else {
+          d.feature = -1;
+          d.threshold = 0;
+          d.left = d.right = 0;
+        }
+        nodes[base + (size_t)i] = d;
+      }
+    }
+    base += (size_t)tot;
+    en.first_tree[(size_t)k + 1] = tree;
+  }
+  offs[(size_t)tree] = (int32_t)base;
+  en.walk = tree > 0 && plan_walk(sh, n, &en.plan);
+
+  int32_t *first = reinterpret_cast<int32_t *>(stage + list_b);
+  int32_t *count = nullptr, *slots = nullptr, *cols = nullptr;
+  uint8_t *remap = nullptr;
+  size_t n_slots = 0, bytes = list_b;
+  if (en.walk) {
+    // Each class's slots from a multiple of per_group on; the slots between
+    // the classes and up to a multiple of tpl are empty.
+    const WalkPlan &p = en.plan;
+    for (int32_t k = 0; k < P.K; ++k)
+      n_slots = (size_t)round_up(round_up((int64_t)n_slots, p.per_group) +
+                                     P.n_trees[k], p.tpl);
+    count = first + n_slots;
+    slots = count + n_slots;
+    cols = slots + 2 * (size_t)P.K;
+    remap = reinterpret_cast<uint8_t *>(cols + std::max(1, sh.n_used));
+    bytes = (size_t)(reinterpret_cast<char *>(remap) - stage) + cols_max;
+    std::memset(first, 0, 2 * n_slots * 4);
+    size_t at = 0;
+    for (int32_t k = 0; k < P.K; ++k) {
+      at = (size_t)round_up((int64_t)at, p.per_group);
+      slots[2 * (size_t)k] = (int32_t)at;
+      const int32_t t0 = en.first_tree[(size_t)k];
+      for (int32_t t = 0; t < P.n_trees[k]; ++t, ++at) {
+        first[at] = offs[(size_t)(t0 + t)];
+        count[at] = P.offsets[k][t + 1] - P.offsets[k][t];
+      }
+      at = (size_t)round_up((int64_t)at, p.tpl);
+      slots[2 * (size_t)k + 1] = (int32_t)at;
+    }
+    sh.columns(cols, remap);
+  }
+  CHK(E->ens_d.ensure(bytes));
+  HIPCHK(hipMemcpyAsync(E->ens_d.p, stage, bytes, hipMemcpyHostToDevice, E->st));
+  auto dev = [&](const void *host) {
+    return E->ens_d.p + (static_cast<const char *>(host) - stage);
+  };
+  en.nodes = reinterpret_cast<const TreeNodeDev *>(E->ens_d.p);
+  en.offsets = reinterpret_cast<const int32_t *>(dev(offs));
+  if (!en.walk) return BSSCL_OK;
+  en.class_slots = reinterpret_cast<const int32_t *>(dev(slots));
+  en.cols = reinterpret_cast<const int32_t *>(dev(cols));
+  CHK(E->walk_words.ensure(n_slots * (size_t)en.plan.slot));
+  CHK(E->walk_vals.ensure(n_slots * (size_t)en.plan.slot));
+  HIPCHK(launch_walk_pack(E->st, en.nodes, reinterpret_cast<const int32_t *>(dev(first)),
+                          reinterpret_cast<const int32_t *>(dev(count)), (int32_t)n_slots,
+                          reinterpret_cast<const uint8_t *>(dev(remap)), lr, en.plan,
+                          E->walk_words.p, E->walk_vals.p));
   return BSSCL_OK;
 }
 
+// F of every class over n rows of `codes` (class k's at out + k *
+// out_stride), or with proba (K = 1) the probabilities of F + base_score;
+// then out is where F goes when the walk cannot write them itself.
+int run_ensemble(bsscl_engine *E, const Ensemble &en, const uint8_t *codes, int64_t ld, int64_t n,
+                 double *out, int64_t out_stride, double *proba = nullptr,
+                 double base_score = 0.0) {
+  hipEvent_t start, stop;
+  if (en.walk) {
+    CHK(prof_kernel(E, 4, &start, &stop));
+    WalkArgs a{codes,        ld,         n,          en.cols,
+               en.plan.n_cols, E->walk_words.p, E->walk_vals.p, en.class_slots,
+               en.plan.slot, en.plan.per_group, out, out_stride,
+               reinterpret_cast<double2 *>(proba), base_score};
+    HIPCHK(launch_walk(E->st, en.plan, a, en.K, start, stop));
+    return BSSCL_OK;
+  }
+  for (int32_t k = 0; k < en.K; ++k) {
+    CHK(prof_kernel(E, 4, &start, &stop));
+    const int32_t t0 = en.first_tree[(size_t)k];
+    HIPCHK(launch_predict(E->st, codes, ld, n, en.nodes, en.offsets + t0,
+                          en.first_tree[(size_t)k + 1] - t0, en.lr, out + k * out_stride, start,
+                          stop));
+  }
+  if (proba) HIPCHK(launch_binary_proba(E->st, out, n, base_score, proba));
+  return BSSCL_OK;
+}
+
+// The ensemble's F of matrix `slot` into E->out_d (est:863-884), or its
+// binary probabilities into E->proba_d.
 int predict_to_device(bsscl_engine *E, int32_t slot, const int16_t *features,
                       const int64_t *thresholds, const double *values,
                       const int32_t *left, const int32_t *right,
-                      const int32_t *offsets, int32_t n_trees, double learning_rate) {
+                      const int32_t *offsets, int32_t n_trees, double learning_rate,
+                      bool proba, double base_score) {
   if (!E || (n_trees > 0 && (!features || !thresholds || !values || !left || !right || !offsets)))
     return set_error(BSSCL_EINVAL, "predict: null argument");
   CHK(check_matrix(E, slot));
   if (n_trees < 0) return set_error(BSSCL_EINVAL, "predict: negative tree count");
   HIPCHK(hipSetDevice(E->device));
   const Matrix &M = E->mat[slot];
-  bool staged = false;
-  int32_t n_chunks = 0;
-  CHK(upload_trees(E, M, features, thresholds, values, left, right, offsets, n_trees, &staged,
-                   &n_chunks));
+  const PackedTrees P{1, &features, &thresholds, &values, &left, &right, &offsets, &n_trees};
+  Ensemble en;
+  CHK(upload_ensemble(E, M, P, learning_rate, M.n, &en));
   CHK(E->out_d.ensure((size_t)M.n));
-  hipEvent_t start, stop;
-  CHK(prof_kernel(E, 4, &start, &stop));
-  HIPCHK(launch_predict(E->st, M.codes.p, M.ld, M.n, M.cols(), E->tree_d.p, E->offsets_d.p,
-                        n_trees, staged ? E->offsets_d.p + n_trees + 1 : nullptr, n_chunks,
-                        learning_rate, E->out_d.p, start, stop));
-  return BSSCL_OK;
+  if (proba) CHK(E->proba_d.ensure(2 * (size_t)M.n));
+  return run_ensemble(E, en, M.codes.p, M.ld, M.n, E->out_d.p, M.n,
+                      proba ? E->proba_d.p : nullptr, base_score);
 }
 
 }  // namespace
@@ -3100,7 +3273,9 @@ void bsscl_engine_destroy(bsscl_engine *E) {
     if (E->rtable_pin[b]) (void)hipHostFree(E->rtable_pin[b]);
     if (E->rslot[b].done) (void)hipEventDestroy(E->rslot[b].done);
   }
-  E->offsets_d.release();
+  E->ens_d.release();
+  E->walk_words.release();
+  E->walk_vals.release();
   E->partials_d.release();
   E->ktime_d.release();
   E->loss_d.release();
@@ -3867,7 +4042,7 @@ int bsscl_predict(bsscl_engine *E, int32_t slot, const int16_t *features,
                   double learning_rate, double *out_F) {
   if (!out_F) return set_error(BSSCL_EINVAL, "predict: null argument");
   CHK(predict_to_device(E, slot, features, thresholds, values, left, right, offsets, n_trees,
-                        learning_rate));
+                        learning_rate, false, 0.0));
   CHK(host_download(E, out_F, E->out_d.p, (size_t)E->mat[slot].n * 8));
   CHK(sync(E));
   return BSSCL_OK;
@@ -3880,11 +4055,8 @@ int bsscl_predict_proba(bsscl_engine *E, int32_t slot, const int16_t *features,
                         double base_score, double *out_proba) {
   if (!out_proba) return set_error(BSSCL_EINVAL, "predict_proba: null argument");
   CHK(predict_to_device(E, slot, features, thresholds, values, left, right, offsets, n_trees,
-                        learning_rate));
-  const int64_t n = E->mat[slot].n;
-  CHK(E->proba_d.ensure(2 * (size_t)n));
-  HIPCHK(launch_binary_proba(E->st, E->out_d.p, n, base_score, E->proba_d.p));
-  CHK(host_download(E, out_proba, E->proba_d.p, (size_t)n * 16));
+                        learning_rate, true, base_score));
+  CHK(host_download(E, out_proba, E->proba_d.p, (size_t)E->mat[slot].n * 16));
   CHK(sync(E));
   return BSSCL_OK;
 }
@@ -3922,10 +4094,9 @@ int bsscl_predict_proba_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, i
   view.F = F;
   view.tiers = tiers;
   CHK(E->pcodes.ensure((size_t)view.ld * view.cols()));
-  bool staged = false;
-  int32_t n_chunks = 0;
-  CHK(upload_trees(E, view, features, thresholds, values, left, right, offsets, n_trees, &staged,
-                   &n_chunks));
+  const PackedTrees P{1, &features, &thresholds, &values, &left, &right, &offsets, &n_trees};
+  Ensemble en;
+  CHK(upload_ensemble(E, view, P, learning_rate, std::min(n, rows_c), &en));
   CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id));
   CHK(E->out_d.ensure((size_t)n));
   CHK(E->proba_d.ensure(2 * (size_t)n));
@@ -3961,17 +4132,11 @@ int bsscl_predict_proba_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, i
       e = launch_bin(E->st, xb, x_is_f64, rows, F, E->edges_d.p, edge_stride, E->nbins_d.p,
                      E->nanid_d.p, has_any_nan, E->pcodes.p, view.ld, tiers);
     if (e == hipSuccess && !one_chunk) e = hipEventRecord(E->pipe_ev[2 + b], E->st);
-    hipEvent_t start = nullptr, stop = nullptr;
     if (e == hipSuccess) {
-      rc = prof_kernel(E, 4, &start, &stop);
+      rc = run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p + r0, n,
+                        E->proba_d.p + 2 * r0, base_score);
       if (rc != BSSCL_OK) break;
     }
-    if (e == hipSuccess)
-      e = launch_predict(E->st, E->pcodes.p, view.ld, rows, view.cols(), E->tree_d.p,
-                         E->offsets_d.p, n_trees, staged ? E->offsets_d.p + n_trees + 1 : nullptr,
-                         n_chunks, learning_rate, E->out_d.p + r0, start, stop);
-    if (e == hipSuccess)
-      e = launch_binary_proba(E->st, E->out_d.p + r0, rows, base_score, E->proba_d.p + 2 * r0);
     if (e == hipSuccess && !one_chunk) {
       hipEvent_t ev = nullptr;
       e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
@@ -4016,37 +4181,23 @@ int bsscl_predict_proba_mc(bsscl_engine *E, int32_t slot, int32_t K,
     return set_error(BSSCL_EINVAL, "predict_proba_mc: K must be in [2, " +
                                        std::to_string(kMcMaxK) + "]");
   CHK(check_matrix(E, slot));
-  int32_t max_total = 1, max_trees = 0;
   for (int32_t k = 0; k < K; ++k) {
     if (n_trees[k] < 0) return set_error(BSSCL_EINVAL, "predict_proba_mc: negative tree count");
     if (n_trees[k] > 0 && (!features[k] || !thresholds[k] || !values[k] || !left[k] ||
                            !right[k] || !offsets[k]))
       return set_error(BSSCL_EINVAL, "predict_proba_mc: null tree array");
-    if (n_trees[k] > 0) max_total = std::max(max_total, offsets[k][n_trees[k]]);
-    max_trees = std::max(max_trees, n_trees[k]);
   }
   HIPCHK(hipSetDevice(E->device));
   const Matrix &M = E->mat[slot];
   const int64_t n = M.n;
-  // Every class's trees fit the tree buffers, so that no class's upload
-  // reallocates them under the walk of the class before.
-  CHK(E->tree_d.ensure((size_t)max_total));
-  CHK(E->offsets_d.ensure(2 * ((size_t)max_trees + 1)));
   CHK(E->out_d.ensure((size_t)K * n));
   CHK(E->proba_d.ensure((size_t)K * n));
-  // F[k] accumulated tree by tree from 0.0 (est:3293-3315), one walk per
-  // class, then the softmax of each row and one readback.
-  for (int32_t k = 0; k < K; ++k) {
-    bool staged = false;
-    int32_t n_chunks = 0;
-    CHK(upload_trees(E, M, features[k], thresholds[k], values[k], left[k], right[k], offsets[k],
-                     n_trees[k], &staged, &n_chunks));
-    hipEvent_t start, stop;
-    CHK(prof_kernel(E, 4, &start, &stop));
-    HIPCHK(launch_predict(E->st, M.codes.p, M.ld, n, M.cols(), E->tree_d.p, E->offsets_d.p,
-                          n_trees[k], staged ? E->offsets_d.p + n_trees[k] + 1 : nullptr,
-                          n_chunks, learning_rate, E->out_d.p + (size_t)k * n, start, stop));
-  }
+  // F[k] accumulated tree by tree from 0.0 (est:3293-3315), every class in
+  // one walk, then the softmax of each row and one readback.
+  const PackedTrees P{K, features, thresholds, values, left, right, offsets, n_trees};
+  Ensemble en;
+  CHK(upload_ensemble(E, M, P, learning_rate, n, &en));
+  CHK(run_ensemble(E, en, M.codes.p, M.ld, n, E->out_d.p, n));
   HIPCHK(launch_mc_softmax(E->st, E->out_d.p, n, K, E->proba_d.p));
   CHK(host_download(E, out_proba, E->proba_d.p, (size_t)n * K * 8));
   CHK(sync(E));
@@ -4075,17 +4226,26 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
                                        " nodes exceed the fixed scratch (at most " +
                                        std::to_string(kNoAllocMaxNodes) + ")");
   // The same checks as bsscl_predict: every traversal stays in its tree.
-  bool adjacent = true;  // every right child is its left child + 1
+  TreeShape sh;
+  sh.used.assign((size_t)M.cols(), 0);
+  std::vector<uint8_t> child((size_t)std::max(total, 1), 0);
   for (int32_t t = 0; t < n_trees; ++t) {
     const int32_t a = offsets[t], b = offsets[t + 1];
     if (a < 0 || b <= a || b > total) return set_error(BSSCL_EINVAL, "predict_noalloc: bad offsets");
+    sh.max_nodes = std::max(sh.max_nodes, b - a);
     for (int32_t i = a; i < b; ++i) {
       if (features[i] < 0) continue;
       const int32_t l = left[i], r = right[i];
       if (features[i] >= M.F || l < 0 || r < 0 || l >= b - a || r >= b - a || l <= i - a ||
           r <= i - a)
         return set_error(BSSCL_EINVAL, "predict_noalloc: malformed tree " + std::to_string(t));
-      adjacent = adjacent && r == l + 1;
+      uint8_t &lc = child[(size_t)(a + l)], &rc = child[(size_t)(a + r)];
+      sh.proper = sh.proper && !lc && !rc && l != r;
+      lc = rc = 1;
+      int32_t col = features[i];
+      int64_t thr = thresholds[i];
+      split_to_engine(M, col, thr);
+      sh.use(col);
     }
   }
   HIPCHK(hipSetDevice(E->device));
@@ -4116,26 +4276,34 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
                              reinterpret_cast<const int32_t *>(S + kScrRight), total,
                              M.F, M.tiers, nodes));
   }
-  // The LDS-staged kernel's runs of whole trees (host list on the stack; the
-  // copy has finished when the call returns).
-  int32_t max_nodes = 0;
-  for (int32_t t = 0; t < n_trees; ++t) max_nodes = std::max(max_nodes, offsets[t + 1] - offsets[t]);
-  const bool staged = n_trees > 0 && predict_staged_ok(M.cols(), max_nodes, adjacent) &&
-                      !std::getenv("BSSCL_TEST_PREDICT_GLOBAL");
-  int32_t n_chunks = 0;
-  int32_t *chunks_d = reinterpret_cast<int32_t *>(S + kScrChunks);
-  if (staged) {
-    std::array<int32_t, kNoAllocMaxTrees + 1> chunks;
-    n_chunks = predict_chunks(offsets, n_trees, chunks.data());
-    HIPCHK(hipMemcpyAsync(chunks_d, chunks.data(), ((size_t)n_chunks + 1) * 4,
-                          hipMemcpyHostToDevice, E->st));
-    HIPCHK(launch_predict(E->st, M.codes.p, M.ld, M.n, M.cols(), nodes, offs, n_trees, chunks_d,
-                          n_chunks, learning_rate, out_F_dev));
+  // The walk in LDS where its lists and packed trees fit the scratch (host
+  // lists on the stack; the copy has finished when the call returns).
+  WalkPlan plan;
+  if (n_trees > 0 && M.cols() <= kNoAllocMaxCols && plan_walk(sh, M.n, &plan) &&
+      round_up(n_trees, plan.tpl) * plan.slot <= kNoAllocWalkSlots) {
+    WalkLists L;
+    const int32_t n_slots = (int32_t)round_up(n_trees, plan.tpl);
+    for (int32_t t = 0; t < n_slots; ++t) {
+      L.first[t] = t < n_trees ? offsets[t] : 0;
+      L.count[t] = t < n_trees ? offsets[t + 1] - offsets[t] : 0;
+    }
+    L.class_slots[0] = 0;
+    L.class_slots[1] = n_slots;
+    sh.columns(L.cols, L.remap);
+    WalkLists *D = reinterpret_cast<WalkLists *>(S + kScrLists);
+    double *vals = reinterpret_cast<double *>(S + kScrWalk);
+    uint32_t *words = reinterpret_cast<uint32_t *>(vals + kNoAllocWalkSlots);
+    HIPCHK(hipMemcpyAsync(D, &L, sizeof(L), hipMemcpyHostToDevice, E->st));
+    HIPCHK(launch_walk_pack(E->st, nodes, D->first, D->count, n_slots, D->remap, learning_rate,
+                            plan, words, vals));
+    const WalkArgs a{M.codes.p, M.ld, M.n, D->cols, plan.n_cols, words, vals, D->class_slots,
+                     plan.slot, plan.per_group, out_F_dev, M.n, nullptr, 0.0};
+    HIPCHK(launch_walk(E->st, plan, a, 1));
     HIPCHK(hipStreamSynchronize(E->st));
     return BSSCL_OK;
   }
-  HIPCHK(launch_predict(E->st, M.codes.p, M.ld, M.n, M.cols(), nodes, offs, n_trees, nullptr, 0,
-                        learning_rate, out_F_dev));
+  HIPCHK(launch_predict(E->st, M.codes.p, M.ld, M.n, nodes, offs, n_trees, learning_rate,
+                        out_F_dev));
   HIPCHK(hipStreamSynchronize(E->st));
   return BSSCL_OK;
 }

@@ -458,25 +458,68 @@ hipError_t launch_predict_tree(hipStream_t st, const uint8_t *codes,
 hipError_t launch_pack_trees(hipStream_t st, const int16_t *features, const int64_t *thresholds,
                              const double *values, const int32_t *left, const int32_t *right,
                              int32_t total, int32_t F, int32_t tiers, TreeNodeDev *nodes);
-// Ensemble prediction.  With `chunks` (predict_chunks' list of n_chunks
-// runs of whole trees; only when predict_staged_ok) the rows' codes and the
-// trees are staged in LDS; otherwise each row walks the trees in HBM.
-int32_t predict_chunk_nodes();
-// (right_follows_left: every split node's right child is its left child + 1.)
-bool predict_staged_ok(int32_t n_cols, int32_t max_tree_nodes, bool right_follows_left);
-// Greedy runs of whole trees of at most predict_chunk_nodes() nodes: writes
-// the first tree of each run and n_trees after the last (n_trees + 1 entries
-// at most); returns the number of runs.
-int32_t predict_chunks(const int32_t *offsets, int32_t n_trees, int32_t *chunks);
-// out[2i], out[2i + 1] = 1 - p, p with p = 1 / (1 + exp(-clip(F[i] + base,
-// -500, 500))); out 16-byte aligned.
+// Ensemble prediction in HBM: each row walks the trees one node load after
+// another (any tree and column count; the walk in LDS is below).
+hipError_t launch_predict(hipStream_t st, const uint8_t *codes, int64_t ld, int64_t n,
+                          const TreeNodeDev *nodes, const int32_t *offsets, int32_t n_trees,
+                          double lr, double *out, hipEvent_t ev_start = nullptr,
+                          hipEvent_t ev_stop = nullptr);
+
+// A binary model's (1 - p, p) of F + base_score (est:3318-3324, 3335-3336):
+// p = 1 / (1 + exp(-clip(F, -500, 500))), each operation rounded separately
+// as NumPy's are (clip keeps a NaN).
+#pragma clang fp contract(off)
+__device__ __forceinline__ double2 binary_proba(double F, double base_score) {
+  const double f = __dadd_rn(F, base_score);
+  const double fc = isnan(f) ? f : fmin(fmax(f, -500.0), 500.0);
+  const double p = __ddiv_rn(1.0, __dadd_rn(1.0, exp(-fc)));
+  return make_double2(__dsub_rn(1.0, p), p);
+}
+#pragma clang fp contract(on)
+// binary_proba of F[0..n); out 16-byte aligned.
 hipError_t launch_binary_proba(hipStream_t st, const double *F, int64_t n, double base,
                                double *out);
-hipError_t launch_predict(hipStream_t st, const uint8_t *codes, int64_t ld,
-                          int64_t n, int32_t n_cols, const TreeNodeDev *nodes,
-                          const int32_t *offsets, int32_t n_trees, const int32_t *chunks,
-                          int32_t n_chunks, double lr, double *out,
-                          hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
+
+// Ensemble prediction in LDS (walk.hip), for trees of at most 1023 nodes
+// that split on at most kWalkMaxCols distinct columns.
+constexpr int32_t kWalkMaxCols = 208;  // 256 rows' codes and a group of trees: 64 KB of LDS
+// From kWalkRows4 rows of at most kWalkCols4 columns on (1,024 rows' codes
+// and a group of trees: 64 KB) a lane walks four rows, else one.
+constexpr int64_t kWalkRows4 = 400000;
+constexpr int32_t kWalkCols4 = 52;
+constexpr int32_t kWalkMaxGroup = 256, kWalkMaxTpl = 8;  // limits of per_group and tpl below
+struct WalkPlan {
+  int32_t slot;       // node slots of a tree: a power of two above the largest tree's nodes
+  int32_t per_group;  // trees staged in LDS at a time
+  int32_t n_cols;     // columns staged per row
+  int32_t rpl, tpl;   // rows of a lane, trees walked at once
+  int32_t win;        // log2 bytes of the window of LDS that a tree's offsets are relative to
+};
+// The plan for n rows, n_cols distinct columns and trees of at most
+// max_nodes nodes; false when they do not fit.  A class's trees take slots
+// from a multiple of per_group on, their count rounded up to a multiple of
+// tpl (the rest of them with count 0 in launch_walk_pack).
+bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan);
+hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int32_t *first,
+                            const int32_t *count, int32_t n_slots, const uint8_t *remap,
+                            double lr, const WalkPlan &p, uint32_t *words, double *vals);
+struct WalkArgs {
+  const uint8_t *codes;  // feature-major, ld a multiple of 256
+  int64_t ld, n;
+  const int32_t *cols;  // the staged columns (null: 0 .. n_cols - 1)
+  int32_t n_cols;
+  const uint32_t *words;  // launch_walk_pack's outputs, slot entries a tree
+  const double *vals;
+  const int32_t *class_slots;  // class k has slots [class_slots[2k], class_slots[2k + 1])
+  int32_t slot, per_group;
+  double *out;  // F of class k at out + k * out_stride
+  int64_t out_stride;
+  double2 *proba;  // when not null: binary_proba(F, base_score) instead
+  double base_score;
+};
+// F (or the probabilities) of n rows for K classes in one launch.
+hipError_t launch_walk(hipStream_t st, const WalkPlan &p, const WalkArgs &a, int32_t K,
+                       hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
 
 int update_F_blocks(int64_t n);
 

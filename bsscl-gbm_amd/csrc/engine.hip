@@ -859,11 +859,16 @@ int host_download(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
   return host_download_on(E, E->st, dst, src, bytes);
 }
 
-// Code tiers and NaN presence of binning with these bin counts (checked).
-int bin_layout(int32_t F, int32_t edge_stride, const int32_t *bin_counts,
-               const int32_t *nan_bin_id, int32_t *tiers, int32_t *has_any_nan) {
+// Code tiers and NaN presence of binning with these bin counts (checked),
+// and launch_bin's levels: 0 when some feature's edges do not ascend (a
+// column with infinities can have NaN edges) or it has too many bins.
+int bin_layout(int32_t F, const double *edges_2d, int32_t edge_stride, const int32_t *bin_counts,
+               const int32_t *nan_bin_id, int32_t *tiers, int32_t *has_any_nan,
+               int32_t *levels) {
   *tiers = 1;
   *has_any_nan = 0;
+  int32_t most = 2;
+  bool ascend = true;
   for (int32_t j = 0; j < F; ++j) {
     if (bin_counts[j] < 1 || bin_counts[j] >= edge_stride)
       return set_error(BSSCL_EINVAL, "bin_features: bin_counts must be in [1, edge_stride)");
@@ -872,7 +877,15 @@ int bin_layout(int32_t F, int32_t edge_stride, const int32_t *bin_counts,
     // Training codes are at most nb - 1, which these tiers hold exactly.
     *tiers = std::max(*tiers, tiers_for_bins(bin_counts[j]));
     if (nan_bin_id[j] >= 0) *has_any_nan = 1;
+    most = std::max(most, bin_counts[j]);
+    const double *e = edges_2d + (size_t)j * edge_stride;
+    bool up = true;
+    for (int32_t k = 0; k < bin_counts[j]; ++k) up &= e[k] <= e[k + 1];
+    ascend = ascend && up;
   }
+  *levels = 1;
+  while (*levels <= kBinMaxLevels && (1 << *levels) < most) ++*levels;
+  if (!ascend || *levels > kBinMaxLevels) *levels = 0;
   return BSSCL_OK;
 }
 
@@ -3317,8 +3330,9 @@ int bsscl_bin_features(bsscl_engine *E, int32_t slot, const void *X,
   if (staged && (!E->xstage.p || E->xs_n != n || E->xs_F != F || E->xs_f64 != (x_is_f64 ? 1 : 0)))
     return set_error(BSSCL_EINVAL,
                      "bin_features: X is NULL but no staged matrix of this shape and dtype");
-  int32_t has_any_nan = 0, tiers = 1;
-  CHK(bin_layout(F, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan));
+  int32_t has_any_nan = 0, tiers = 1, levels = 0;
+  CHK(bin_layout(F, edges_2d, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan,
+                 &levels));
   HIPCHK(hipSetDevice(E->device));
   CHK(alloc_matrix(E, slot, n, F, tiers));
   CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id));
@@ -3328,7 +3342,7 @@ int bsscl_bin_features(bsscl_engine *E, int32_t slot, const void *X,
   const size_t esz = x_is_f64 ? 8 : 4;
   if (staged) {
     hipError_t e = launch_bin(E->st, E->xstage.p, x_is_f64, n, F, ed, edge_stride, nb, nid,
-                              has_any_nan, M.codes.p, M.ld, tiers);
+                              has_any_nan, M.codes.p, M.ld, tiers, levels);
     if (e == hipSuccess) e = hipStreamSynchronize(E->st);
     if (e != hipSuccess)
       return set_error(BSSCL_EDEVICE, std::string("binning: ") + hipGetErrorString(e));
@@ -3345,7 +3359,7 @@ int bsscl_bin_features(bsscl_engine *E, int32_t slot, const void *X,
       CHK(host_upload(E, xd.p, (const unsigned char *)X + (size_t)r0 * F * esz,
                       (size_t)rows * F * esz));
       hipError_t e = launch_bin(E->st, xd.p, x_is_f64, rows, F, ed, edge_stride, nb, nid,
-                                has_any_nan, M.codes.p + r0, M.ld, tiers);
+                                has_any_nan, M.codes.p + r0, M.ld, tiers, levels);
       if (e == hipSuccess) e = hipStreamSynchronize(E->st);
       if (e != hipSuccess)
         return set_error(BSSCL_EDEVICE, std::string("binning: ") + hipGetErrorString(e));
@@ -4074,8 +4088,9 @@ int bsscl_predict_proba_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, i
   if (n <= 0 || n > INT32_MAX || F <= 0)
     return set_error(BSSCL_EINVAL, "predict_proba_rows: bad shape");
   if (n_trees < 0) return set_error(BSSCL_EINVAL, "predict_proba_rows: negative tree count");
-  int32_t tiers = 1, has_any_nan = 0;
-  CHK(bin_layout(F, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan));
+  int32_t tiers = 1, has_any_nan = 0, levels = 0;
+  CHK(bin_layout(F, edges_2d, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan,
+                 &levels));
   HIPCHK(hipSetDevice(E->device));
   const size_t esz = x_is_f64 ? 8 : 4;
   // Rows per chunk: about 256 MB of X, in whole blocks of the walk (512
@@ -4130,7 +4145,7 @@ int bsscl_predict_proba_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, i
     if (e == hipSuccess && !one_chunk) e = hipStreamWaitEvent(E->st, E->pipe_ev[b], 0);
     if (e == hipSuccess)
       e = launch_bin(E->st, xb, x_is_f64, rows, F, E->edges_d.p, edge_stride, E->nbins_d.p,
-                     E->nanid_d.p, has_any_nan, E->pcodes.p, view.ld, tiers);
+                     E->nanid_d.p, has_any_nan, E->pcodes.p, view.ld, tiers, levels);
     if (e == hipSuccess && !one_chunk) e = hipEventRecord(E->pipe_ev[2 + b], E->st);
     if (e == hipSuccess) {
       rc = run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p + r0, n,

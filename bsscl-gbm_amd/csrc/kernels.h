@@ -244,7 +244,11 @@ constexpr int kReplaySlots = 1024;  // candidate slots the device replay holds
 hipError_t launch_bin(hipStream_t st, const void *X, int is_f64, int64_t n,
                       int32_t F, const double *edges, int32_t stride,
                       const int32_t *nb, const int32_t *nan_id,
-                      int32_t has_any_nan, uint8_t *codes, int64_t ld, int32_t tiers);
+                      int32_t has_any_nan, uint8_t *codes, int64_t ld, int32_t tiers,
+                      int32_t levels);
+// (levels > 0: every feature's edges ascend and nb <= 1 << levels, at most
+// kBinMaxLevels; 0: any edges.)
+constexpr int32_t kBinMaxLevels = 9;
 hipError_t launch_load_codes(hipStream_t st, const void *src, int is_u16,
                              int64_t n, int32_t F, uint8_t *codes, int64_t ld, int32_t tiers);
 hipError_t launch_get_codes(hipStream_t st, const uint8_t *codes, int64_t ld,

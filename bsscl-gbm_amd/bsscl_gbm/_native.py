@@ -58,6 +58,8 @@ _SIGS = {
     "bsscl_predict_proba_rows": [_P, _P, _i32, _i64, _i32, _P, _i32, _P, _P, _P, _P, _P, _P,
                                  _P, _P, _i32, _f64, _f64, _P],
     "bsscl_predict_proba_mc": [_P, _i32, _i32, _P, _P, _P, _P, _P, _P, _P, _f64, _P],
+    "bsscl_predict_proba_mc_rows": [_P, _P, _i32, _i64, _i32, _P, _i32, _P, _P, _i32, _P, _P,
+                                    _P, _P, _P, _P, _P, _f64, _P],
     "bsscl_predict_tree": [_P, _i32, _P, _P, _P, _P, _P, _i32, _P],
     "bsscl_predict_noalloc": [_P, _i32, _P, _P, _P, _P, _P, _P, _i32, _f64, _P],
     "bsscl_node_split": [_P, _P, _P, _P, _i64, _P, _i32, _P, _f64, _f64, _P, _P,
@@ -450,26 +452,51 @@ class Engine:
             float(learning_rate), float(base_score), ptr(out)))
         return out
 
+    @staticmethod
+    def _class_tables(packs, n_trees):
+        """(tables of K array pointers in the ABI's order, tree counts, the
+        arrays themselves, which must outlive the call)."""
+        names = ("features", "thresholds", "values", "left", "right", "offsets")
+        dtypes = (np.int16, np.int64, np.float64, np.int32, np.int32, np.int32)
+        keep, tables = [], []
+        for name, dt in zip(names, dtypes):
+            arrs = [np.ascontiguousarray(p[name], dt) if p is not None else None for p in packs]
+            keep.append(arrs)
+            tables.append(ctypes.cast(
+                (ctypes.c_void_p * len(packs))(*[a.ctypes.data if a is not None else None
+                                                 for a in arrs]), ctypes.c_void_p))
+        nt = np.ascontiguousarray([int(t) if p is not None else 0
+                                   for p, t in zip(packs, n_trees)], np.int32)
+        return tables, nt, keep
+
     def predict_proba_mc(self, slot, n, packs, n_trees, learning_rate):
         """bsscl_predict_proba_mc: a multiclass model's softmax probabilities
         of matrix `slot`, shape (n, K); packs[k] is class k's packed trees
         (None for a class without trees)."""
-        K = len(packs)
-        names = ("features", "thresholds", "values", "left", "right", "offsets")
-        dtypes = (np.int16, np.int64, np.float64, np.int32, np.int32, np.int32)
-        keep = []
-        tables = []
-        for name, dt in zip(names, dtypes):
-            arrs = [np.ascontiguousarray(p[name], dt) if p is not None else None for p in packs]
-            keep.append(arrs)
-            tables.append((ctypes.c_void_p * K)(*[a.ctypes.data if a is not None else None
-                                                 for a in arrs]))
-        nt = np.ascontiguousarray([int(t) if p is not None else 0
-                                   for p, t in zip(packs, n_trees)], np.int32)
-        out = np.empty((n, K), np.float64)
-        check(lib().bsscl_predict_proba_mc(self.handle, int(slot), K,
-                                           *[ctypes.cast(t, ctypes.c_void_p) for t in tables],
-                                           ptr(nt), float(learning_rate), ptr(out)))
+        tables, nt, keep = self._class_tables(packs, n_trees)
+        out = np.empty((n, len(packs)), np.float64)
+        check(lib().bsscl_predict_proba_mc(self.handle, int(slot), len(packs), *tables, ptr(nt),
+                                           float(learning_rate), ptr(out)))
+        del keep
+        return out
+
+    def predict_proba_mc_rows(self, X, edges_2d, bin_counts, nan_bin_id, packs, n_trees,
+                              learning_rate):
+        """bsscl_predict_proba_mc_rows: predict_proba_mc of host rows X,
+        binned and walked on the device in overlapped row chunks; matrix
+        slots are left as they were."""
+        X = np.ascontiguousarray(X)
+        if X.dtype not in (np.float32, np.float64):
+            X = X.astype(np.float64)
+        n, F = X.shape
+        e = np.ascontiguousarray(edges_2d, dtype=np.float64)
+        bc = np.ascontiguousarray(bin_counts, dtype=np.int32)
+        ni = np.ascontiguousarray(nan_bin_id, dtype=np.int32)
+        tables, nt, keep = self._class_tables(packs, n_trees)
+        out = np.empty((n, len(packs)), np.float64)
+        check(lib().bsscl_predict_proba_mc_rows(
+            self.handle, ptr(X), int(X.dtype == np.float64), n, F, ptr(e), e.shape[1], ptr(bc),
+            ptr(ni), len(packs), *tables, ptr(nt), float(learning_rate), ptr(out)))
         del keep
         return out
 

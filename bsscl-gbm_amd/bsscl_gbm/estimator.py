@@ -979,30 +979,31 @@ class HybridHistGBMNumbaV1_0_1:
         if X.ndim != 2 or X.shape[1] != self.n_features_in_:
             raise ValueError(f"X must have {self.n_features_in_} features")
         eng = _engine(self._device_index())
-        if proba and not self._is_multiclass:
-            # Binning, walk and probabilities in one call, its row chunks'
-            # uploads overlapping the device's work on the chunk before.
-            packed = {'features': self._packed_features, 'thresholds': self._packed_thresholds,
-                      'values': self._packed_values, 'left': self._packed_left,
-                      'right': self._packed_right, 'offsets': self._tree_offsets}
+        if proba:
+            # Binning, walk and probabilities (est:3318-3336; multiclass
+            # est:3293-3315 and the softmax of est:2327-2332) in one call, its
+            # row chunks' uploads overlapping the device's work on the chunk
+            # before.
             with eng.lock:
                 t0 = time.perf_counter()
-                out = eng.predict_proba_rows(X, self.bin_edges, self.feature_bin_counts,
-                                             self._nan_bin_id, packed, len(self.trees),
-                                             self.learning_rate,
-                                             getattr(self, 'base_score_', 0.0))
+                if self._is_multiclass:
+                    out = eng.predict_proba_mc_rows(
+                        X, self.bin_edges, self.feature_bin_counts, self._nan_bin_id,
+                        self._mc_packed, [len(t) for t in self.mc_trees], self.learning_rate)
+                else:
+                    packed = {'features': self._packed_features,
+                              'thresholds': self._packed_thresholds,
+                              'values': self._packed_values, 'left': self._packed_left,
+                              'right': self._packed_right, 'offsets': self._tree_offsets}
+                    out = eng.predict_proba_rows(X, self.bin_edges, self.feature_bin_counts,
+                                                 self._nan_bin_id, packed, len(self.trees),
+                                                 self.learning_rate,
+                                                 getattr(self, 'base_score_', 0.0))
                 self.times['inference'] = (time.perf_counter() - t0) * 1000
             return out
         with eng.lock:  # matrix slot 1 holds this call's codes until it returns
             eng.bin_features(1, X, self.bin_edges, self.feature_bin_counts, self._nan_bin_id)
             t0 = time.perf_counter()
-            if self._is_multiclass and proba:
-                # est:3293-3315 and the softmax (est:2327-2332) on the
-                # device, read back once.
-                out = eng.predict_proba_mc(1, X.shape[0], self._mc_packed,
-                                           [len(t) for t in self.mc_trees], self.learning_rate)
-                self.times['inference'] = (time.perf_counter() - t0) * 1000
-                return out
             if self._is_multiclass:
                 # est:3293-3315: per class, sum its trees from 0.0.
                 F = np.zeros((X.shape[0], self.n_classes_), dtype=np.float64)

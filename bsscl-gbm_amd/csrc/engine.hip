@@ -307,6 +307,12 @@ int scratch_for_device(int device, unsigned char **out) {
 }
 }  // namespace
 
+namespace {
+constexpr int kXferPins = 6;
+constexpr int kOutPins = 3;
+constexpr size_t kOutPinBytes = 16u << 20;
+}  // namespace
+
 struct bsscl_engine {
   int32_t device = 0;
   hipStream_t st = nullptr;
@@ -472,20 +478,27 @@ struct bsscl_engine {
   TempBuf<double> walk_vals;
   DevBuf<double> partials_d, loss_d, out_d, proba_d;
   PinnedArena pin;
-  // Large host transfers go through these pinned chunks (host_upload,
-  // host_download), and binning of a host matrix through xchunk.
-  char *xfer_pin[3] = {nullptr, nullptr, nullptr};
-  hipEvent_t xfer_ev[3] = {nullptr, nullptr, nullptr};
-  int xfer_next = 0;  // the pinned chunk the next piece goes through
+  // Large host transfers go through these pinned buffers and, every second
+  // piece, their own stream (host_upload, host_download); binning of a host
+  // matrix through xchunk.
+  char *xfer_pin[kXferPins] = {};
+  hipEvent_t xfer_ev[kXferPins] = {};
+  int xfer_next = 0;  // the pinned buffer the next piece goes through
+  hipStream_t st_xfer = nullptr;
+  hipEvent_t xfer_fork = nullptr;
   TempBuf<unsigned char> xchunk;
   // bsscl_predict_proba_rows: the second row chunk of X, one chunk's codes,
   // and its events (chunk uploaded, chunk binned; two of each).
   TempBuf<unsigned char> xchunk2;
   TempBuf<uint8_t> pcodes;
   hipEvent_t pipe_ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  // Probabilities on their way to pageable memory (predict_rows): at most
+  // kOutPinBytes each.
+  size_t out_pin_b = 0;
+  char *out_pin[kOutPins] = {};
+  hipEvent_t out_ev[kOutPins] = {};
   // The bin edges, bin counts and NaN bins of the last binning call.
-  TempBuf<double> edges_d;
-  TempBuf<int32_t> nbins_d, nanid_d;
+  TempBuf<char> edges_d;
 
   // Feature matrix staged by bsscl_stage_features (row-major, as given) and
   // its columns sorted by bsscl_sort_columns (keys [F][col_ld]).
@@ -678,12 +691,26 @@ int upload(bsscl_engine *E, DevBuf<T> &dst, const T *src, size_t count) {
   return BSSCL_OK;
 }
 
+// `bytes` of the pinned arena for a copy on E->st, waiting for its earlier
+// copies when they leave no room.
+int take_pinned(bsscl_engine *E, size_t bytes, char **out) {
+  // (16 MB, as the tree builder's first call takes: growing it later would
+  // free and pin again, about 1 ms.)
+  const size_t want = std::max<size_t>(2 * bytes + 512, 16u << 20);
+  *out = bytes + 512 <= E->pin.cap ? E->pin.take<char>(bytes) : nullptr;
+  if (*out) return BSSCL_OK;
+  CHK(sync(E));
+  CHK(E->pin.reserve(std::max(E->pin.cap, want)));
+  *out = E->pin.take<char>(bytes);
+  return BSSCL_OK;
+}
+
 // ---------------------------------------------------------------------------
 // Large host <-> device transfers.  A copy from pageable memory makes HIP
 // stage it through its own pinned buffers, one after the other (about
 // 19 GB/s for a 112 MB matrix, 27-29 GB/s for 2 GB).  Here host threads
-// copy chunks into three pinned buffers while the DMA engine moves the
-// chunk before, so both run at once, and the DMA engine sets the rate.
+// copy pieces into pinned buffers while the DMA engine moves the pieces
+// before, so both run at once, and the DMA engine sets the rate.
 // ---------------------------------------------------------------------------
 
 // A few host threads that split a memcpy with the caller.  One pool per
@@ -771,92 +798,128 @@ class CopyPool {
   size_t bytes_ = 0;
 };
 
-// Chunks of 8 MB keep small transfers pipelined; from 512 MB on, 32 MB
-// chunks reach 55 GB/s host to device against 52 (10M x 50 float32: 36 ms;
-// HIP's own pageable copy 69-73 ms).
-constexpr size_t kXferChunkMax = 32u << 20;
-size_t xfer_chunk(size_t bytes) { return bytes >= (512u << 20) ? kXferChunkMax : 8u << 20; }
+// Large transfers go piece by piece through kXferPins pinned buffers,
+// alternating between the caller's stream and a second one: consecutive
+// copies of one stream are about 14 us apart (4 MB pieces: 47 GB/s host to
+// device), which the other stream's copy fills (55-57 GB/s from 2 MB on; one
+// stream reaches 53 with 8 MB pieces and 55 with 32 MB ones).
+// Up to 1 MB HIP's own pageable copy is as fast.
+constexpr size_t kXferPiece = 4u << 20, kXferSmall = 1u << 20;
+size_t xfer_piece(size_t bytes) {
+  return std::min(kXferPiece, std::max<size_t>(256u << 10, bytes / 4 / 4096 * 4096));
+}
 
 int ensure_xfer(bsscl_engine *E) {
-  for (int b = 0; b < 3; ++b) {
+  for (int b = 0; b < kXferPins; ++b) {
     if (!E->xfer_pin[b])
-      HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&E->xfer_pin[b]), kXferChunkMax,
+      HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&E->xfer_pin[b]), kXferPiece,
                            hipHostMallocDefault));
     if (!E->xfer_ev[b]) HIPCHK(hipEventCreateWithFlags(&E->xfer_ev[b], hipEventDisableTiming));
   }
+  if (!E->st_xfer) HIPCHK(hipStreamCreateWithFlags(&E->st_xfer, hipStreamNonBlocking));
+  if (!E->xfer_fork)
+    HIPCHK(hipEventCreateWithFlags(&E->xfer_fork, hipEventDisableTiming));
   return BSSCL_OK;
 }
 
-// Enqueues dst (device) = src (host, pageable) on stream `st` in pieces of
-// `piece` bytes through the pinned chunks, and returns once the last piece
-// has been copied into its pinned chunk; the copies complete on `st`.  A
-// pinned chunk is refilled only after the copy that last read it, whichever
-// call or stream enqueued that one.
-int host_upload_async(bsscl_engine *E, hipStream_t st, void *dst, const void *src, size_t bytes,
-                      size_t piece) {
-  if (bytes < 2 * piece) {
+int ensure_out_pins(bsscl_engine *E, size_t bytes) {
+  for (int b = 0; b < kOutPins; ++b) {
+    if (E->out_pin_b < bytes && E->out_pin[b]) {
+      HIPCHK(hipHostFree(E->out_pin[b]));
+      E->out_pin[b] = nullptr;
+    }
+    if (!E->out_pin[b])
+      HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&E->out_pin[b]), std::max(bytes, E->out_pin_b),
+                           hipHostMallocDefault));
+    if (!E->out_ev[b]) HIPCHK(hipEventCreateWithFlags(&E->out_ev[b], hipEventDisableTiming));
+  }
+  E->out_pin_b = std::max(bytes, E->out_pin_b);
+  return BSSCL_OK;
+}
+
+// The pinned buffer of the next piece, once the copy that last used it (of
+// whichever call or stream) has gone; `ev` is recorded after the piece's.
+int next_piece(bsscl_engine *E, char **pin, hipEvent_t *ev) {
+  const int b = E->xfer_next;
+  E->xfer_next = (b + 1) % kXferPins;
+  HIPCHK(hipEventSynchronize(E->xfer_ev[b]));
+  *pin = E->xfer_pin[b];
+  *ev = E->xfer_ev[b];
+  return BSSCL_OK;
+}
+
+// Enqueues dst (device) = src (host, pageable) after the work already on
+// stream `st`, and returns once the last piece has been copied into its
+// pinned buffer; later work on `st` sees the whole copy.
+int host_upload_async(bsscl_engine *E, hipStream_t st, void *dst, const void *src, size_t bytes) {
+  if (bytes <= kXferSmall) {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     return BSSCL_OK;
   }
   CHK(ensure_xfer(E));
   CopyPool &pool = CopyPool::get();
-  for (size_t off = 0; off < bytes; off += piece) {
-    const int b = E->xfer_next;
-    E->xfer_next = (b + 1) % 3;
+  HIPCHK(hipEventRecord(E->xfer_fork, st));
+  HIPCHK(hipStreamWaitEvent(E->st_xfer, E->xfer_fork, 0));
+  const size_t piece = xfer_piece(bytes);
+  hipEvent_t last = nullptr;
+  bool second = false;
+  for (size_t off = 0; off < bytes; off += piece, second = !second) {
     const size_t len = std::min(piece, bytes - off);
-    HIPCHK(hipEventSynchronize(E->xfer_ev[b]));  // its previous piece has gone
-    pool.copy(E->xfer_pin[b], static_cast<const char *>(src) + off, len);
-    HIPCHK(hipMemcpyAsync(static_cast<char *>(dst) + off, E->xfer_pin[b], len,
-                          hipMemcpyHostToDevice, st));
-    HIPCHK(hipEventRecord(E->xfer_ev[b], st));
+    char *pin;
+    hipEvent_t ev;
+    CHK(next_piece(E, &pin, &ev));
+    pool.copy(pin, static_cast<const char *>(src) + off, len);
+    hipStream_t on = second ? E->st_xfer : st;
+    HIPCHK(hipMemcpyAsync(static_cast<char *>(dst) + off, pin, len, hipMemcpyHostToDevice, on));
+    HIPCHK(hipEventRecord(ev, on));
+    if (second) last = ev;
   }
+  if (last) HIPCHK(hipStreamWaitEvent(st, last, 0));
   return BSSCL_OK;
 }
 
 // dst (device) = src (host, pageable) on E->st; returns once the copy is
 // complete.
 int host_upload(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
-  CHK(host_upload_async(E, E->st, dst, src, bytes, xfer_chunk(bytes)));
+  CHK(host_upload_async(E, E->st, dst, src, bytes));
   HIPCHK(hipStreamSynchronize(E->st));
   return BSSCL_OK;
 }
 
-// dst (host, pageable) = src (device) after the work already on stream
-// `st`; returns once dst holds it.
-int host_download_on(bsscl_engine *E, hipStream_t st, void *dst, const void *src, size_t bytes) {
-  const size_t chunk = xfer_chunk(bytes);
-  if (bytes < 2 * chunk) {
-    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+// dst (host, pageable) = src (device) after the work already on E->st;
+// returns once dst holds it.
+int host_download(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
+  if (bytes <= kXferSmall) {
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, E->st));
+    HIPCHK(hipStreamSynchronize(E->st));
     return BSSCL_OK;
   }
   CHK(ensure_xfer(E));
   CopyPool &pool = CopyPool::get();
-  const size_t n_chunks = (bytes + chunk - 1) / chunk;
+  HIPCHK(hipEventRecord(E->xfer_fork, E->st));
+  HIPCHK(hipStreamWaitEvent(E->st_xfer, E->xfer_fork, 0));
+  const size_t piece = xfer_piece(bytes);
+  const size_t n = (bytes + piece - 1) / piece;
+  char *pin[kXferPins];
+  hipEvent_t ev[kXferPins];
   auto enqueue = [&](size_t c) -> int {
-    const int b = (int)(c % 3);
-    const size_t off = c * chunk;
-    HIPCHK(hipEventSynchronize(E->xfer_ev[b]));  // no upload still reads the chunk
-    HIPCHK(hipMemcpyAsync(E->xfer_pin[b], static_cast<const char *>(src) + off,
-                          std::min(chunk, bytes - off), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipEventRecord(E->xfer_ev[b], st));
+    CHK(next_piece(E, &pin[c % kXferPins], &ev[c % kXferPins]));
+    hipStream_t on = c & 1 ? E->st_xfer : E->st;
+    HIPCHK(hipMemcpyAsync(pin[c % kXferPins], static_cast<const char *>(src) + c * piece,
+                          std::min(piece, bytes - c * piece), hipMemcpyDeviceToHost, on));
+    HIPCHK(hipEventRecord(ev[c % kXferPins], on));
     return BSSCL_OK;
   };
-  // Two chunks in flight ahead of the one being copied out.
-  for (size_t c = 0; c < std::min<size_t>(2, n_chunks); ++c) CHK(enqueue(c));
-  for (size_t c = 0; c < n_chunks; ++c) {
-    if (c + 2 < n_chunks) CHK(enqueue(c + 2));
-    const int b = (int)(c % 3);
-    HIPCHK(hipEventSynchronize(E->xfer_ev[b]));
-    const size_t off = c * chunk;
-    pool.copy(static_cast<char *>(dst) + off, E->xfer_pin[b], std::min(chunk, bytes - off));
+  // All but one of the buffers in flight ahead of the one being copied out.
+  const size_t ahead = kXferPins - 1;
+  for (size_t c = 0; c < std::min(ahead, n); ++c) CHK(enqueue(c));
+  for (size_t c = 0; c < n; ++c) {
+    if (c + ahead < n) CHK(enqueue(c + ahead));
+    HIPCHK(hipEventSynchronize(ev[c % kXferPins]));
+    pool.copy(static_cast<char *>(dst) + c * piece, pin[c % kXferPins],
+              std::min(piece, bytes - c * piece));
   }
   return BSSCL_OK;
-}
-
-// dst (host, pageable) = src (device) after the work already on E->st.
-int host_download(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
-  return host_download_on(E, E->st, dst, src, bytes);
 }
 
 // Code tiers and NaN presence of binning with these bin counts (checked),
@@ -889,17 +952,26 @@ int bin_layout(int32_t F, const double *edges_2d, int32_t edge_stride, const int
   return BSSCL_OK;
 }
 
-// A binning call's edges [F][edge_stride], bin counts and NaN bins into
-// E->edges_d, nbins_d and nanid_d (on E->st).
+// A binning call's edges [F][edge_stride], bin counts and NaN bins on the
+// device (E->edges_d), in one copy from pinned memory on E->st.
+struct DevEdges {
+  const double *edges;
+  const int32_t *nb, *nan_id;
+};
+
 int upload_edges(bsscl_engine *E, int32_t F, const double *edges_2d, int32_t edge_stride,
-                 const int32_t *bin_counts, const int32_t *nan_bin_id) {
-  CHK(E->edges_d.ensure((size_t)F * edge_stride));
-  CHK(E->nbins_d.ensure((size_t)F));
-  CHK(E->nanid_d.ensure((size_t)F));
-  HIPCHK(hipMemcpyAsync(E->edges_d.p, edges_2d, (size_t)F * edge_stride * 8,
-                        hipMemcpyHostToDevice, E->st));
-  HIPCHK(hipMemcpyAsync(E->nbins_d.p, bin_counts, (size_t)F * 4, hipMemcpyHostToDevice, E->st));
-  HIPCHK(hipMemcpyAsync(E->nanid_d.p, nan_bin_id, (size_t)F * 4, hipMemcpyHostToDevice, E->st));
+                 const int32_t *bin_counts, const int32_t *nan_bin_id, DevEdges *out) {
+  const size_t eb = (size_t)F * edge_stride * 8, fb = (size_t)F * 4;
+  char *stage = nullptr;
+  CHK(take_pinned(E, eb + 2 * fb, &stage));
+  std::memcpy(stage, edges_2d, eb);
+  std::memcpy(stage + eb, bin_counts, fb);
+  std::memcpy(stage + eb + fb, nan_bin_id, fb);
+  CHK(E->edges_d.ensure(eb + 2 * fb));
+  HIPCHK(hipMemcpyAsync(E->edges_d.p, stage, eb + 2 * fb, hipMemcpyHostToDevice, E->st));
+  out->edges = reinterpret_cast<const double *>(E->edges_d.p);
+  out->nb = reinterpret_cast<const int32_t *>(E->edges_d.p + eb);
+  out->nan_id = out->nb + F;
   return BSSCL_OK;
 }
 
@@ -2920,6 +2992,24 @@ struct PackedTrees {
   const int32_t *n_trees;
 };
 
+// The class count and arrays of a multiclass prediction.
+int check_classes(const PackedTrees &P) {
+  if (!P.n_trees || !P.features || !P.thresholds || !P.values || !P.left || !P.right ||
+      !P.offsets)
+    return set_error(BSSCL_EINVAL, "predict_proba_mc: null argument");
+  if (P.K < 2 || P.K > kMcMaxK)
+    return set_error(BSSCL_EINVAL,
+                     "predict_proba_mc: K must be in [2, " + std::to_string(kMcMaxK) + "]");
+  for (int32_t k = 0; k < P.K; ++k) {
+    if (P.n_trees[k] < 0)
+      return set_error(BSSCL_EINVAL, "predict_proba_mc: negative tree count");
+    if (P.n_trees[k] > 0 && (!P.features[k] || !P.thresholds[k] || !P.values[k] || !P.left[k] ||
+                             !P.right[k] || !P.offsets[k]))
+      return set_error(BSSCL_EINVAL, "predict_proba_mc: null tree array");
+  }
+  return BSSCL_OK;
+}
+
 // What the walk needs to know of an ensemble: its largest tree, the columns
 // it splits on, and whether every node has one parent (then a tree has as
 // many nodes breadth first as in its arrays).
@@ -2991,14 +3081,8 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   const size_t cols_max = (size_t)M.cols();
   const size_t bytes_max =
       list_b + (2 * slots_max + 2 * (size_t)P.K + cols_max + 1) * 4 + cols_max;
-  const size_t pin_b = std::max<size_t>(bytes_max + 512, 8u << 20);
-  if (pin_b > E->pin.cap) HIPCHK(hipStreamSynchronize(E->st));
-  CHK(E->pin.reserve(std::max(E->pin.cap, pin_b)));
-  char *stage = E->pin.take<char>(bytes_max);
-  if (!stage) {  // the arena's earlier copies first
-    CHK(sync(E));
-    stage = E->pin.take<char>(bytes_max);
-  }
+  char *stage = nullptr;
+  CHK(take_pinned(E, bytes_max, &stage));
   TreeNodeDev *nodes = reinterpret_cast<TreeNodeDev *>(stage);
   int32_t *offs = reinterpret_cast<int32_t *>(stage + off_b);
   std::vector<uint8_t> &child = E->child_marks;
@@ -3144,6 +3228,129 @@ int predict_to_device(bsscl_engine *E, int32_t slot, const int16_t *features,
   if (proba) CHK(E->proba_d.ensure(2 * (size_t)M.n));
   return run_ensemble(E, en, M.codes.p, M.ld, M.n, E->out_d.p, M.n,
                       proba ? E->proba_d.p : nullptr, base_score);
+}
+
+// The whole predict_proba of host rows: binning, the walk and the
+// probabilities, (1 - p, p) per row for one class, the softmax over the
+// classes for more.
+//
+// X streams through the device in row chunks: while chunk c goes up on the
+// rows stream (host copies into the pinned pieces, then DMA), the engine's
+// stream bins, walks and reads back chunk c - 1 and the host copies chunk
+// c - 2's probabilities out.  The upload sets the rate (57 GB/s here), so a
+// chunk only has to be short enough that the last one's tail is short, and
+// long enough to fill the chip: an eighth of X between 8 and 64 MB.  Up to
+// 16 MB go as one chunk.  1M x 28 float32, 100 trees: 3.6 ms in one chunk,
+// 2.65 so (2.12 of them the upload); 10M x 50, 500 trees: 44.0 ms in 256 MB
+// chunks read back at the end, 39.2 so.  (More copy threads, or a thread for
+// the results alone, change neither.)
+int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, int32_t F,
+                 const double *edges_2d, int32_t edge_stride, const int32_t *bin_counts,
+                 const int32_t *nan_bin_id, const PackedTrees &P, double lr, double base_score,
+                 double *out_proba) {
+  int32_t tiers = 1, has_any_nan = 0, levels = 0;
+  CHK(bin_layout(F, edges_2d, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan,
+                 &levels));
+  HIPCHK(hipSetDevice(E->device));
+  const size_t row_b = (size_t)F * (x_is_f64 ? 8 : 4), total_b = row_b * (size_t)n;
+  const size_t out_w = P.K > 1 ? (size_t)P.K : 2;  // doubles per row
+  size_t chunk_b = std::min<size_t>(std::max<size_t>(total_b / 8, 8u << 20), 64u << 20);
+  if (total_b <= (16u << 20)) chunk_b = total_b;
+  // (A chunk's probabilities fit a pinned buffer.)
+  int64_t rows_c = (int64_t)std::min(chunk_b / row_b, kOutPinBytes / (8 * out_w));
+  // (Test hook BSSCL_TEST_PREDICT_CHUNK_ROWS: another count.)
+  if (const char *t = std::getenv("BSSCL_TEST_PREDICT_CHUNK_ROWS"))
+    rows_c = std::min<int64_t>(std::strtoll(t, nullptr, 10), rows_c);
+  rows_c = std::min<int64_t>(std::max<int64_t>(1024, rows_c / 1024 * 1024), round_up(n, 1024));
+  if (rows_c >= n) rows_c = n;
+  const bool one_chunk = rows_c >= n;
+  // One chunk's codes, in the layout of a matrix of rows_c rows.
+  Matrix view;
+  view.n = rows_c;
+  view.ld = round_up(rows_c + 8, 256);
+  view.F = F;
+  view.tiers = tiers;
+  CHK(E->pcodes.ensure((size_t)view.ld * view.cols()));
+  CHK(E->out_d.ensure((size_t)P.K * rows_c));
+  CHK(E->proba_d.ensure(out_w * (size_t)rows_c));
+  const size_t xbytes = (size_t)rows_c * row_b;
+  CHK(E->xchunk.ensure(xbytes));
+  if (!one_chunk) CHK(E->xchunk2.ensure(xbytes));
+  CHK(ensure_out_pins(E, std::min(kOutPinBytes, out_w * 8 * (size_t)rows_c)));
+  for (hipEvent_t &ev : E->pipe_ev)
+    if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  const unsigned char *xs = static_cast<const unsigned char *>(X);
+  const int64_t n_chunks = (n + rows_c - 1) / rows_c;
+  auto rows_of = [&](int64_t c) { return std::min(rows_c, n - c * rows_c); };
+  // Chunk c's probabilities from their pinned buffer.
+  auto finish = [&](int64_t c) -> int {
+    const int b = (int)(c % kOutPins);
+    HIPCHK(hipEventSynchronize(E->out_ev[b]));
+    CopyPool::get().copy(out_proba + out_w * (size_t)(c * rows_c), E->out_pin[b],
+                         out_w * 8 * (size_t)rows_of(c));
+    return BSSCL_OK;
+  };
+  Ensemble en;
+  DevEdges de;
+  auto enqueue = [&](int64_t c) -> int {
+    const int64_t r0 = c * rows_c, rows = rows_of(c);
+    const int b = (int)(c & 1);
+    unsigned char *xb = b ? E->xchunk2.p : E->xchunk.p;
+    const size_t xc = (size_t)rows * row_b;
+    if (one_chunk) {
+      // Nothing to overlap: through the arena when small, else as pieces.
+      char *stage = nullptr;
+      if (xc <= (1u << 20)) {
+        CHK(take_pinned(E, xc, &stage));
+        std::memcpy(stage, xs, xc);
+        HIPCHK(hipMemcpyAsync(xb, stage, xc, hipMemcpyHostToDevice, E->st));
+      } else {
+        CHK(host_upload_async(E, E->st, xb, xs, xc));
+      }
+    } else {
+      // (Its buffer is free once chunk c - 2 has been binned.)
+      if (c >= 2) HIPCHK(hipStreamWaitEvent(E->st_rows, E->pipe_ev[2 + b], 0));
+      CHK(host_upload_async(E, E->st_rows, xb, xs + (size_t)r0 * row_b, xc));
+      HIPCHK(hipEventRecord(E->pipe_ev[b], E->st_rows));
+    }
+    if (c == 0) {  // the model, while the first rows are on their way
+      CHK(upload_ensemble(E, view, P, lr, rows_c, &en));
+      CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id, &de));
+    }
+    if (!one_chunk) HIPCHK(hipStreamWaitEvent(E->st, E->pipe_ev[b], 0));
+    HIPCHK(launch_bin(E->st, xb, x_is_f64, rows, F, de.edges, edge_stride, de.nb, de.nan_id,
+                      has_any_nan, E->pcodes.p, view.ld, tiers, levels));
+    if (!one_chunk) HIPCHK(hipEventRecord(E->pipe_ev[2 + b], E->st));
+    if (P.K == 1) {
+      CHK(run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p, rows_c, E->proba_d.p,
+                       base_score));
+    } else {
+      CHK(run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p, rows));
+      HIPCHK(launch_mc_softmax(E->st, E->out_d.p, rows, P.K, E->proba_d.p));
+    }
+    const int o = (int)(c % kOutPins);
+    HIPCHK(hipMemcpyAsync(E->out_pin[o], E->proba_d.p, out_w * 8 * (size_t)rows,
+                          hipMemcpyDeviceToHost, E->st));
+    HIPCHK(hipEventRecord(E->out_ev[o], E->st));
+    return BSSCL_OK;
+  };
+  int rc = BSSCL_OK;
+  for (int64_t c = 0; c < n_chunks && rc == BSSCL_OK; ++c) {
+    rc = enqueue(c);
+    if (rc == BSSCL_OK && c >= 2) rc = finish(c - 2);
+  }
+  for (int64_t c = std::max<int64_t>(0, n_chunks - 2); c < n_chunks && rc == BSSCL_OK; ++c)
+    rc = finish(c);
+  if (rc != BSSCL_OK) {  // the buffers can be used again once both streams drain
+    (void)hipStreamSynchronize(E->st_rows);
+    (void)hipStreamSynchronize(E->st);
+    return rc;
+  }
+  // (The last chunk's event followed everything on both streams: they need
+  // no wait of their own, 17 us of a 64-row call.)
+  CHK(prof_collect(E));
+  E->pin.reset();
+  return BSSCL_OK;
 }
 
 }  // namespace
@@ -3295,16 +3502,20 @@ void bsscl_engine_destroy(bsscl_engine *E) {
   E->out_d.release();
   E->proba_d.release();
   E->pin.release();
-  for (int b = 0; b < 3; ++b) {
+  for (int b = 0; b < kXferPins; ++b) {
     if (E->xfer_pin[b]) (void)hipHostFree(E->xfer_pin[b]);
     if (E->xfer_ev[b]) (void)hipEventDestroy(E->xfer_ev[b]);
   }
+  if (E->xfer_fork) (void)hipEventDestroy(E->xfer_fork);
+  if (E->st_xfer) (void)hipStreamDestroy(E->st_xfer);
   E->xchunk.release();
   E->xchunk2.release();
   E->pcodes.release();
   E->edges_d.release();
-  E->nbins_d.release();
-  E->nanid_d.release();
+  for (int b = 0; b < kOutPins; ++b) {
+    if (E->out_pin[b]) (void)hipHostFree(E->out_pin[b]);
+    if (E->out_ev[b]) (void)hipEventDestroy(E->out_ev[b]);
+  }
   for (hipEvent_t ev : E->pipe_ev)
     if (ev) (void)hipEventDestroy(ev);
   release_staging(E);
@@ -3335,9 +3546,10 @@ int bsscl_bin_features(bsscl_engine *E, int32_t slot, const void *X,
                  &levels));
   HIPCHK(hipSetDevice(E->device));
   CHK(alloc_matrix(E, slot, n, F, tiers));
-  CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id));
-  const double *ed = E->edges_d.p;
-  const int32_t *nb = E->nbins_d.p, *nid = E->nanid_d.p;
+  DevEdges de;
+  CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id, &de));
+  const double *ed = de.edges;
+  const int32_t *nb = de.nb, *nid = de.nan_id;
   Matrix &M = E->mat[slot];
   const size_t esz = x_is_f64 ? 8 : 4;
   if (staged) {
@@ -3347,8 +3559,7 @@ int bsscl_bin_features(bsscl_engine *E, int32_t slot, const void *X,
     if (e != hipSuccess)
       return set_error(BSSCL_EDEVICE, std::string("binning: ") + hipGetErrorString(e));
   } else {
-    // Stream X through the device in row chunks of at most 512 MB (each
-    // chunk's upload then takes the 32 MB pieces of host_upload).
+    // Stream X through the device in row chunks of at most 512 MB.
     int64_t chunk = std::max<int64_t>(64, (int64_t)((512u << 20) / (esz * (size_t)F)) / 64 * 64);
     chunk = std::min<int64_t>(chunk, round_up(n, 64));
     // (The chunk buffer stays allocated for the next host matrix.)
@@ -4088,100 +4299,27 @@ int bsscl_predict_proba_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, i
   if (n <= 0 || n > INT32_MAX || F <= 0)
     return set_error(BSSCL_EINVAL, "predict_proba_rows: bad shape");
   if (n_trees < 0) return set_error(BSSCL_EINVAL, "predict_proba_rows: negative tree count");
-  int32_t tiers = 1, has_any_nan = 0, levels = 0;
-  CHK(bin_layout(F, edges_2d, edge_stride, bin_counts, nan_bin_id, &tiers, &has_any_nan,
-                 &levels));
-  HIPCHK(hipSetDevice(E->device));
-  const size_t esz = x_is_f64 ? 8 : 4;
-  // Rows per chunk: about 256 MB of X, in whole blocks of the walk (512
-  // rows).  The walk hides its LDS latency only with many blocks per CU:
-  // 1M x 28 in eighths took 1.46 ms of walk against 0.36 ms in one launch,
-  // and 10M x 50 in 9 chunks 33 ms against 30 ms in 8.  (Test hook
-  // BSSCL_TEST_PREDICT_CHUNK_ROWS: another count.)
-  int64_t rows_c = (int64_t)((256u << 20) / (esz * (size_t)F));
-  if (const char *t = std::getenv("BSSCL_TEST_PREDICT_CHUNK_ROWS"))
-    rows_c = std::strtoll(t, nullptr, 10);
-  rows_c = std::min<int64_t>(std::max<int64_t>(512, rows_c / 512 * 512), round_up(n, 512));
-  // One chunk's codes, in the layout of a matrix of rows_c rows.
-  Matrix view;
-  view.n = rows_c;
-  view.ld = round_up(rows_c + 8, 256);
-  view.F = F;
-  view.tiers = tiers;
-  CHK(E->pcodes.ensure((size_t)view.ld * view.cols()));
   const PackedTrees P{1, &features, &thresholds, &values, &left, &right, &offsets, &n_trees};
-  Ensemble en;
-  CHK(upload_ensemble(E, view, P, learning_rate, std::min(n, rows_c), &en));
-  CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id));
-  CHK(E->out_d.ensure((size_t)n));
-  CHK(E->proba_d.ensure(2 * (size_t)n));
-  const bool one_chunk = n <= rows_c;
-  const size_t xbytes = (size_t)rows_c * F * esz;
-  CHK(E->xchunk.ensure(xbytes));
-  if (!one_chunk) CHK(E->xchunk2.ensure(xbytes));
-  for (hipEvent_t &ev : E->pipe_ev)
-    if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  // Chunk c goes up on the rows stream into buffer c % 2 (after the binning
-  // of chunk c - 2 has read it); the engine's stream bins it, walks it and
-  // turns its F into probabilities, while chunk c + 1 goes up.  (A single
-  // chunk goes up on the engine's stream, with nothing to overlap.)
-  hipStream_t up = one_chunk ? E->st : E->st_rows;
-  const size_t piece = xfer_chunk((size_t)n * F * esz);
-  const unsigned char *xs = static_cast<const unsigned char *>(X);
-  std::vector<hipEvent_t> done;  // chunk c's probabilities are written
-  int rc = BSSCL_OK;
-  int c = 0;
-  for (int64_t r0 = 0; r0 < n && rc == BSSCL_OK; r0 += rows_c, ++c) {
-    const int64_t rows = std::min(rows_c, n - r0);
-    const int b = c & 1;
-    unsigned char *xb = b ? E->xchunk2.p : E->xchunk.p;
-    hipError_t e = hipSuccess;
-    if (c >= 2) e = hipStreamWaitEvent(up, E->pipe_ev[2 + b], 0);
-    if (e == hipSuccess) {
-      rc = host_upload_async(E, up, xb, xs + (size_t)r0 * F * esz, (size_t)rows * F * esz, piece);
-      if (rc != BSSCL_OK) break;
-      if (!one_chunk) e = hipEventRecord(E->pipe_ev[b], up);
-    }
-    if (e == hipSuccess && !one_chunk) e = hipStreamWaitEvent(E->st, E->pipe_ev[b], 0);
-    if (e == hipSuccess)
-      e = launch_bin(E->st, xb, x_is_f64, rows, F, E->edges_d.p, edge_stride, E->nbins_d.p,
-                     E->nanid_d.p, has_any_nan, E->pcodes.p, view.ld, tiers, levels);
-    if (e == hipSuccess && !one_chunk) e = hipEventRecord(E->pipe_ev[2 + b], E->st);
-    if (e == hipSuccess) {
-      rc = run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p + r0, n,
-                        E->proba_d.p + 2 * r0, base_score);
-      if (rc != BSSCL_OK) break;
-    }
-    if (e == hipSuccess && !one_chunk) {
-      hipEvent_t ev = nullptr;
-      e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-      if (e == hipSuccess) {
-        done.push_back(ev);
-        e = hipEventRecord(ev, E->st);
-      }
-    }
-    if (e != hipSuccess)
-      rc = set_error(BSSCL_EDEVICE, std::string("predict_proba_rows: ") + hipGetErrorString(e));
-  }
-  // The probabilities come back chunk by chunk on the rows stream, each as
-  // soon as its chunk is done, while the device works on the later chunks.
-  if (rc == BSSCL_OK && one_chunk) rc = host_download(E, out_proba, E->proba_d.p, (size_t)n * 16);
-  for (size_t k = 0; rc == BSSCL_OK && k < done.size(); ++k) {
-    const int64_t r0 = (int64_t)k * rows_c, rows = std::min(rows_c, n - r0);
-    if (hipStreamWaitEvent(E->st_rows, done[k], 0) != hipSuccess) {
-      rc = set_error(BSSCL_EDEVICE, "predict_proba_rows: stream wait failed");
-      break;
-    }
-    rc = host_download_on(E, E->st_rows, out_proba + 2 * r0, E->proba_d.p + 2 * r0,
-                          (size_t)rows * 16);
-  }
-  // (Both streams drain before the buffers can be used again, on every path.)
-  (void)hipStreamSynchronize(E->st_rows);
-  (void)hipStreamSynchronize(E->st);
-  for (hipEvent_t ev : done) (void)hipEventDestroy(ev);
-  if (rc != BSSCL_OK) return rc;
-  CHK(sync(E));
-  return BSSCL_OK;
+  return predict_rows(E, X, x_is_f64, n, F, edges_2d, edge_stride, bin_counts, nan_bin_id, P,
+                      learning_rate, base_score, out_proba);
+}
+
+int bsscl_predict_proba_mc_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n,
+                                int32_t F, const double *edges_2d, int32_t edge_stride,
+                                const int32_t *bin_counts, const int32_t *nan_bin_id, int32_t K,
+                                const int16_t *const *features, const int64_t *const *thresholds,
+                                const double *const *values, const int32_t *const *left,
+                                const int32_t *const *right, const int32_t *const *offsets,
+                                const int32_t *n_trees, double learning_rate,
+                                double *out_proba) {
+  if (!E || !X || !edges_2d || !bin_counts || !nan_bin_id || !out_proba)
+    return set_error(BSSCL_EINVAL, "predict_proba_mc_rows: null argument");
+  if (n <= 0 || n > INT32_MAX || F <= 0)
+    return set_error(BSSCL_EINVAL, "predict_proba_mc_rows: bad shape");
+  const PackedTrees P{K, features, thresholds, values, left, right, offsets, n_trees};
+  CHK(check_classes(P));
+  return predict_rows(E, X, x_is_f64, n, F, edges_2d, edge_stride, bin_counts, nan_bin_id, P,
+                      learning_rate, 0.0, out_proba);
 }
 
 int bsscl_predict_proba_mc(bsscl_engine *E, int32_t slot, int32_t K,
@@ -4189,19 +4327,10 @@ int bsscl_predict_proba_mc(bsscl_engine *E, int32_t slot, int32_t K,
                            const double *const *values, const int32_t *const *left,
                            const int32_t *const *right, const int32_t *const *offsets,
                            const int32_t *n_trees, double learning_rate, double *out_proba) {
-  if (!E || !out_proba || !n_trees || !features || !thresholds || !values || !left || !right ||
-      !offsets)
-    return set_error(BSSCL_EINVAL, "predict_proba_mc: null argument");
-  if (K < 2 || K > kMcMaxK)
-    return set_error(BSSCL_EINVAL, "predict_proba_mc: K must be in [2, " +
-                                       std::to_string(kMcMaxK) + "]");
+  if (!E || !out_proba) return set_error(BSSCL_EINVAL, "predict_proba_mc: null argument");
+  const PackedTrees P{K, features, thresholds, values, left, right, offsets, n_trees};
+  CHK(check_classes(P));
   CHK(check_matrix(E, slot));
-  for (int32_t k = 0; k < K; ++k) {
-    if (n_trees[k] < 0) return set_error(BSSCL_EINVAL, "predict_proba_mc: negative tree count");
-    if (n_trees[k] > 0 && (!features[k] || !thresholds[k] || !values[k] || !left[k] ||
-                           !right[k] || !offsets[k]))
-      return set_error(BSSCL_EINVAL, "predict_proba_mc: null tree array");
-  }
   HIPCHK(hipSetDevice(E->device));
   const Matrix &M = E->mat[slot];
   const int64_t n = M.n;
@@ -4209,7 +4338,6 @@ int bsscl_predict_proba_mc(bsscl_engine *E, int32_t slot, int32_t K,
   CHK(E->proba_d.ensure((size_t)K * n));
   // F[k] accumulated tree by tree from 0.0 (est:3293-3315), every class in
   // one walk, then the softmax of each row and one readback.
-  const PackedTrees P{K, features, thresholds, values, left, right, offsets, n_trees};
   Ensemble en;
   CHK(upload_ensemble(E, M, P, learning_rate, n, &en));
   CHK(run_ensemble(E, en, M.codes.p, M.ld, n, E->out_d.p, n));

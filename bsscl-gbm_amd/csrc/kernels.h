@@ -491,12 +491,15 @@ constexpr int32_t kWalkMaxCols = 208;  // 256 rows' codes and a group of trees: 
 // and a group of trees: 64 KB) a lane walks four rows, else one.
 constexpr int64_t kWalkRows4 = 400000;
 constexpr int32_t kWalkCols4 = 52;
+// Up to this many rows the waves of a block share out the trees.
+constexpr int64_t kWalkSplitRows = 65536;
 constexpr int32_t kWalkMaxGroup = 256, kWalkMaxTpl = 8;  // limits of per_group and tpl below
 struct WalkPlan {
   int32_t slot;       // node slots of a tree: a power of two above the largest tree's nodes
   int32_t per_group;  // trees staged in LDS at a time
   int32_t n_cols;     // columns staged per row
   int32_t rpl, tpl;   // rows of a lane, trees walked at once
+  bool split;         // a block's waves walk different trees
   int32_t win;        // log2 bytes of the window of LDS that a tree's offsets are relative to
 };
 // The plan for n rows, n_cols distinct columns and trees of at most

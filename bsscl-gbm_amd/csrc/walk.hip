@@ -252,12 +252,112 @@ __global__ __launch_bounds__((1 << kTileLog2) / kRpl) void k_walk(WalkArgs a) {
 }
 #pragma clang fp contract(on)
 
+// The walk of few rows: the kSplitWaves waves of a block take 64 rows through
+// eight trees each at a time, so a request of some rows is not one wave's
+// walk of every tree (28 columns, 100 trees: 11 us at 64 rows and 20 at 65,000,
+// against 27 and 28 in k_walk's blocks; 50 columns, 500 trees: 37 and 77
+// against 120 and 125; from about 100,000 rows on the rows alone fill the
+// chip).
+// The leaves' values wait in LDS, in place of the words they were reached
+// by, and the first wave adds them in tree order.
+constexpr int kSplitWaves = 8, kSplitTrees = 8 * kSplitWaves;
+
+#pragma clang fp contract(off)
+template <bool kProba>
+__global__ __launch_bounds__(64 * kSplitWaves) void k_walk_split(WalkArgs a) {
+  constexpr int kWin = kWinSmall, kTpl = 8;
+  constexpr uint32_t kChildMask = (1u << kWin) - 4u;
+  constexpr uint32_t kColMask = 0xFFFFFFu & ~((1u << kWin) - 1u);
+  constexpr int kWaveBytes = kGroupNodes * 4;  // words of eight trees; then [8][64] values
+  constexpr int kCodes = kSplitWaves * kWaveBytes;
+  static_assert(kTpl * 64 * 8 <= kWaveBytes, "the values fit in place of the words");
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int32_t cls = (int32_t)blockIdx.y;
+  const int64_t row0 = (int64_t)blockIdx.x * 64;
+  for (int k = (int)threadIdx.x; k < a.n_cols * 4; k += 64 * kSplitWaves) {
+    const int64_t col = a.cols ? a.cols[k >> 2] : k >> 2;
+    lds_put(kCodes + 16 * k,
+            *reinterpret_cast<const Quad *>(a.codes + col * a.ld + row0 + 16 * (k & 3)));
+  }
+  const uint32_t mine = (uint32_t)(wave * kWaveBytes);
+  auto code_at = [&](uint32_t w) {
+    return kCodes + (((w & kColMask) >> (kWin - 6)) | (uint32_t)lane);
+  };
+  const int32_t t_end = a.class_slots[2 * cls + 1];
+  double F = 0.0;
+  for (int32_t g = a.class_slots[2 * cls]; g < t_end; g += kSplitTrees) {
+    // This wave's trees: slots [t0, t0 + nt), nt a multiple of kTpl or 0.  A
+    // tree's words are relative to its window, and a group of trees starts
+    // at a window.
+    const int32_t t0 = g + wave * kTpl;
+    const bool any = t0 < t_end;
+    uint32_t p[kTpl];
+    if (any) {
+      const Quad *src = reinterpret_cast<const Quad *>(a.words + (int64_t)t0 * a.slot);
+      const int nq = kTpl * a.slot / 4;
+      for (int q = lane; q < nq; q += 64) lds_put(mine + 16 * q, src[q]);
+    }
+    __syncthreads();
+    if (any) {
+      int32_t steps = 2;
+      uint32_t w[kTpl], win[kTpl];
+      // Where the wave's trees start in their first window.
+      const uint32_t lead = ((uint32_t)(t0 % a.per_group) * (uint32_t)a.slot * 4u) &
+                            ((1u << kWin) - 1u);
+#pragma unroll
+      for (int j = 0; j < kTpl; ++j) {
+        const uint32_t at = (uint32_t)(j * a.slot * 4);
+        win[j] = mine + ((lead + at) & ~((1u << kWin) - 1u)) - lead;
+        const Quad top = lds_get<Quad>(mine + at);
+        steps = max(steps, __builtin_amdgcn_readfirstlane((int)top.y));
+        w[j] = lds_get<uint8_t>(code_at(top.x)) > (top.x >> 24) ? top.w : top.z;
+      }
+      for (int32_t d = 1; d < steps; ++d) {
+#pragma unroll
+        for (int j = 0; j < kTpl; ++j) p[j] = lds_get<uint8_t>(code_at(w[j]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kTpl; ++j)
+          p[j] = win[j] + ((w[j] & kChildMask) | (p[j] > (w[j] >> 24) ? 4u : 0u));
+        if (d + 1 < steps) {
+#pragma unroll
+          for (int j = 0; j < kTpl; ++j) w[j] = lds_get<uint32_t>(p[j]);
+        }
+      }
+      double v[kTpl];
+#pragma unroll
+      for (int j = 0; j < kTpl; ++j)
+        v[j] = a.vals[(int64_t)t0 * a.slot + (p[j] - mine) / 4];
+      // (The wave's own words are read no more.)
+#pragma unroll
+      for (int j = 0; j < kTpl; ++j) lds_put(mine + (uint32_t)(j * 64 + lane) * 8, v[j]);
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int32_t nt = min(t_end - g, kSplitTrees);
+      for (int32_t t = 0; t < nt; t += kTpl) {
+#pragma unroll
+        for (int j = 0; j < kTpl; ++j)
+          F = F + lds_get<double>((uint32_t)(t / kTpl * kWaveBytes + (j * 64 + lane) * 8));
+      }
+    }
+    __syncthreads();
+  }
+  const int64_t i = row0 + lane;
+  if (wave == 0 && i < a.n) {
+    if constexpr (kProba) a.proba[i] = binary_proba(F, a.base_score);
+    else a.out[cls * a.out_stride + i] = F;
+  }
+}
+#pragma clang fp contract(on)
+
 bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
   if (n_cols < 1 || n_cols > kWalkMaxCols || max_nodes >= kGroupNodes) return false;
   WalkPlan &p = *plan;
   p.slot = 4;
   while (p.slot <= max_nodes) p.slot *= 2;  // (slot 1 holds no node)
   p.n_cols = n_cols;
+  p.split = false;
   p.win = p.slot * 4 <= 1 << kWinSmall ? kWinSmall : kWinLarge;
   // Four rows per lane conflict least but need a full chip of 1,024-row
   // tiles, two of them per CU (28 columns, 100 trees: 67 us at 100,000 rows
@@ -270,6 +370,7 @@ bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
   } else {
     p.rpl = 1;
     p.tpl = p.slot <= kGroupNodes / 8 ? 8 : p.slot <= kGroupNodes / 2 ? 2 : 1;
+    p.split = n <= kWalkSplitRows && p.tpl == 8;
   }
   p.per_group = kGroupNodes / p.slot;
   return true;
@@ -306,6 +407,15 @@ hipError_t run_walk(hipStream_t st, const WalkArgs &a, int32_t K, hipEvent_t ev_
 hipError_t launch_walk(hipStream_t st, const WalkPlan &p, const WalkArgs &a, int32_t K,
                        hipEvent_t ev_start, hipEvent_t ev_stop) {
   if (a.n <= 0) return hipSuccess;
+  if (p.split) {
+    const dim3 grid((unsigned)((a.n + 63) / 64), (unsigned)K), block(64 * kSplitWaves);
+    const size_t lds = (size_t)kSplitWaves * kGroupNodes * 4 + ((size_t)a.n_cols << 6);
+    if (a.proba)
+      hipExtLaunchKernelGGL(k_walk_split<true>, grid, block, lds, st, ev_start, ev_stop, 0, a);
+    else
+      hipExtLaunchKernelGGL(k_walk_split<false>, grid, block, lds, st, ev_start, ev_stop, 0, a);
+    return hipGetLastError();
+  }
   if (p.rpl == 4) return run_walk<4, 2, 10, kWinSmall>(st, a, K, ev_start, ev_stop);
   if (p.tpl == 8) return run_walk<1, 8, 8, kWinSmall>(st, a, K, ev_start, ev_stop);
   if (p.win == kWinSmall) return run_walk<1, 2, 8, kWinSmall>(st, a, K, ev_start, ev_stop);

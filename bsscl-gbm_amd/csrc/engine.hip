@@ -402,6 +402,10 @@ struct bsscl_engine {
   DevBuf<int32_t> round_rows[2];  // in-bag rows of round slot s, ascending
   DevBuf<int64_t> rows64;
   DevBuf<int32_t> rows_in, sort_tmp;
+  // bsscl_build_tree's rows sorted (load_grad_hess), and what it found.
+  TempBuf<uint8_t> tree_flags;
+  TempBuf<int32_t> tree_sort_tmp, tree_rows32;
+  TempBuf<char> checks_d;
   // Row permutation of a device-rows sampler (cumulative over its rounds)
   // and the Fisher-Yates work arrays.
   DevBuf<int32_t> perm[2];
@@ -2062,27 +2066,87 @@ inline void split_to_engine(const Matrix &X, int32_t &feature, int64_t &threshol
   }
 }
 
+// A caller's gradients, hessians and (for a tree) rows are checked and their
+// largest magnitudes found on the device from this many rows on: host passes
+// over them took as long as their upload (1M rows: 1.0 ms).  Below, the
+// passes are short and a device round trip is not.
+constexpr int64_t kDeviceCheckRows = 65536;
+
+// The int64 row ids of bsscl_build_tree as the device found them.
+struct TreeRows {
+  const int64_t *rows;
+  int64_t m;
+  bool sorted = false;  // distinct: E->tree_rows32 holds them in ascending order
+};
+
 // Uploads host gradients/hessians and quantizes them with scales from their
-// largest magnitudes.
+// largest magnitudes.  With `tr`, its rows too (E->rows64), checked; distinct
+// rows are also sorted, by flags and a compaction, so that the root gather
+// streams through the columns (1M x 28, shuffled rows: 113 us, sorted 28).
 int load_grad_hess(bsscl_engine *E, const double *grad, const double *hess,
-                   int64_t n, int64_t rows_summed) {
+                   int64_t n, int64_t rows_summed, TreeRows *tr = nullptr) {
   double gmax = 0.0, hmax = 0.0;
-  for (int64_t i = 0; i < n; ++i) {
-    const double a = std::fabs(grad[i]), b = std::fabs(hess[i]);
-    if (!std::isfinite(a) || !std::isfinite(b))
-      return set_error(BSSCL_EINVAL, "grad/hess must be finite");
-    gmax = std::max(gmax, a);
-    hmax = std::max(hmax, b);
+  CHK(E->g64.ensure((size_t)n));
+  CHK(E->h64.ensure((size_t)n));
+  CHK(E->ghq.ensure((size_t)n));
+  const char *bad_row = "build_tree: sample index out of range";
+  const char *not_finite = "grad/hess must be finite";
+  if (n < kDeviceCheckRows) {
+    if (tr) {
+      for (int64_t k = 0; k < tr->m; ++k)
+        if (tr->rows[k] < 0 || tr->rows[k] >= n) return set_error(BSSCL_EINVAL, bad_row);
+      CHK(E->rows64.ensure((size_t)tr->m));
+      CHK(host_upload_async(E, E->st, E->rows64.p, tr->rows, (size_t)tr->m * 8));
+    }
+    for (int64_t i = 0; i < n; ++i) {
+      const double a = std::fabs(grad[i]), b = std::fabs(hess[i]);
+      if (!std::isfinite(a) || !std::isfinite(b)) return set_error(BSSCL_EINVAL, not_finite);
+      gmax = std::max(gmax, a);
+      hmax = std::max(hmax, b);
+    }
+    CHK(host_upload_async(E, E->st, E->g64.p, grad, (size_t)n * 8));
+    CHK(host_upload_async(E, E->st, E->h64.p, hess, (size_t)n * 8));
+  } else {
+    struct Found {
+      unsigned long long mx[2];
+      int32_t bad, distinct;
+    };
+    CHK(E->checks_d.ensure(sizeof(Found)));
+    Found *d = reinterpret_cast<Found *>(E->checks_d.p);
+    HIPCHK(hipMemsetAsync(d, 0, sizeof(Found), E->st));
+    if (tr) {
+      CHK(E->rows64.ensure((size_t)tr->m));
+      CHK(host_upload_async(E, E->st, E->rows64.p, tr->rows, (size_t)tr->m * 8));
+      // (One tile of flags past the rows: its offset in the compaction is
+      // the number of distinct rows.)
+      const int64_t n_pad = sort_rows_flag_bytes(n) + 4096;
+      CHK(E->tree_flags.ensure((size_t)n_pad));
+      CHK(E->tree_sort_tmp.ensure((size_t)(n_pad / 4096 + 1)));
+      CHK(E->tree_rows32.ensure((size_t)tr->m));
+      HIPCHK(hipMemsetAsync(E->tree_flags.p, 0, (size_t)n_pad, E->st));
+      HIPCHK(launch_mark_checked(E->st, E->rows64.p, tr->m, n, E->tree_flags.p, &d->bad));
+      HIPCHK(launch_sort_rows(E->st, nullptr, tr->m, E->tree_flags.p, n_pad, E->tree_sort_tmp.p,
+                              E->tree_rows32.p, true));
+      HIPCHK(hipMemcpyAsync(&d->distinct, E->tree_sort_tmp.p + n_pad / 4096 - 1, 4,
+                            hipMemcpyDeviceToDevice, E->st));
+    }
+    CHK(host_upload_async(E, E->st, E->g64.p, grad, (size_t)n * 8));
+    CHK(host_upload_async(E, E->st, E->h64.p, hess, (size_t)n * 8));
+    HIPCHK(launch_abs_max(E->st, E->g64.p, E->h64.p, n, d->mx));
+    Found f;
+    HIPCHK(hipMemcpyAsync(&f, d, sizeof(f), hipMemcpyDeviceToHost, E->st));
+    HIPCHK(hipStreamSynchronize(E->st));
+    if (f.bad) return set_error(BSSCL_EINVAL, bad_row);
+    constexpr unsigned long long kInf = 0x7ff0000000000000ull;
+    if (f.mx[0] >= kInf || f.mx[1] >= kInf) return set_error(BSSCL_EINVAL, not_finite);
+    std::memcpy(&gmax, &f.mx[0], 8);
+    std::memcpy(&hmax, &f.mx[1], 8);
+    if (tr) tr->sorted = f.distinct == tr->m;
   }
   const double gm = fixed_mul(gmax, rows_summed), hm = fixed_mul(hmax, rows_summed);
   E->g_scale = 1.0 / gm;
   E->h_scale = 1.0 / hm;
   E->h_bound = hmax;
-  CHK(E->g64.ensure((size_t)n));
-  CHK(E->h64.ensure((size_t)n));
-  CHK(E->ghq.ensure((size_t)n));
-  HIPCHK(hipMemcpyAsync(E->g64.p, grad, (size_t)n * 8, hipMemcpyHostToDevice, E->st));
-  HIPCHK(hipMemcpyAsync(E->h64.p, hess, (size_t)n * 8, hipMemcpyHostToDevice, E->st));
   HIPCHK(launch_quantize(E->st, E->g64.p, E->h64.p, n, gm, hm, E->ghq.p));
   return BSSCL_OK;
 }
@@ -3449,6 +3513,10 @@ void bsscl_engine_destroy(bsscl_engine *E) {
   E->rows64.release();
   E->rows_in.release();
   E->sort_tmp.release();
+  E->tree_flags.release();
+  E->tree_sort_tmp.release();
+  E->tree_rows32.release();
+  E->checks_d.release();
   for (int s = 0; s < 2; ++s) E->perm[s].release();
   E->fy_head.release();
   E->fy_next.release();
@@ -3799,23 +3867,19 @@ int bsscl_build_tree(bsscl_engine *E, const double *grad, const double *hess,
   (void)max_bins;
   const Matrix &X = E->mat[0];
   if (n_samples <= 0) return set_error(BSSCL_EINVAL, "build_tree: no samples");
-  for (int64_t k = 0; k < n_samples; ++k)
-    if (sample_indices[k] < 0 || sample_indices[k] >= X.n)
-      return set_error(BSSCL_EINVAL, "build_tree: sample index out of range");
   TreeOut out{out_features, out_thresholds, out_values, out_left, out_right,
               out_node_count, out_split_gains};
   std::vector<int32_t> feats, nb_sel;
   HIPCHK(hipSetDevice(E->device));
   CHK(validate_tree_args(E, feature_indices, n_selected, max_leaves,
                          min_samples_leaf, bin_counts, out, feats, nb_sel));
-  CHK(load_grad_hess(E, grad, hess, X.n, n_samples));
-  CHK(E->rows64.ensure((size_t)n_samples));
-  HIPCHK(hipMemcpyAsync(E->rows64.p, sample_indices, (size_t)n_samples * 8,
-                        hipMemcpyHostToDevice, E->st));
+  TreeRows tr{sample_indices, n_samples};
+  CHK(load_grad_hess(E, grad, hess, X.n, n_samples, &tr));
   TreeParams tp{max_leaves, max_depth, min_samples_leaf, min_child_weight,
                 reg_lambda, gamma};
   E->set_base = 0;
-  CHK(build_tree_core(E, nullptr, n_samples, feats, nb_sel, tp, out));
+  CHK(build_tree_core(E, tr.sorted ? E->tree_rows32.p : nullptr, n_samples, feats, nb_sel, tp,
+                      out));
   tree_to_reference(X, out);
   return BSSCL_OK;
 }

@@ -264,6 +264,12 @@ hipError_t launch_grad_hess(hipStream_t st, const double *F, const uint8_t *y,
 hipError_t launch_grad_hess_f64(hipStream_t st, const double *F,
                                 const uint8_t *y, int64_t n, double w0,
                                 double w1, double *g, double *h);
+// The flags of a caller's m row ids; *bad = 1 when one is outside [0, n).
+hipError_t launch_mark_checked(hipStream_t st, const int64_t *rows, int64_t m, int64_t n,
+                               uint8_t *flags, int32_t *bad);
+// out[0], out[1] raised to the bits of max |a|, max |b|.
+hipError_t launch_abs_max(hipStream_t st, const double *a, const double *b, int64_t n,
+                          unsigned long long *out);
 hipError_t launch_sort_rows(hipStream_t st, const int32_t *rows, int64_t m,
                             uint8_t *flags, int64_t n_pad, int32_t *block_tmp,
                             int32_t *out, bool marked = false);

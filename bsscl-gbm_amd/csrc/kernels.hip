@@ -512,6 +512,44 @@ hipError_t launch_grad_hess_f64(hipStream_t st, const double *F,
   return hipGetLastError();
 }
 
+// The largest |a| and |b| over n values, as bits (of non-negative doubles,
+// which order as unsigned integers; those of an infinity or a NaN are above
+// every finite value's), raised into out[0] and out[1].
+__global__ __launch_bounds__(256) void k_abs_max(const double *__restrict__ a,
+                                                 const double *__restrict__ b, int64_t n,
+                                                 unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long red[2][4];
+  unsigned long long m[2] = {0, 0};
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(fabs(a[i]));
+    const unsigned long long y = (unsigned long long)__double_as_longlong(fabs(b[i]));
+    m[0] = x > m[0] ? x : m[0];
+    m[1] = y > m[1] ? y : m[1];
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    for (int o = 32; o >= 1; o >>= 1) {
+      const unsigned long long t = __shfl_xor(m[k], o, 64);
+      m[k] = t > m[k] ? t : m[k];
+    }
+    if (lane_id() == 0) red[k][threadIdx.x >> 6] = m[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned long long v = 0;
+    for (int w = 0; w < 4; ++w) v = red[threadIdx.x][w] > v ? red[threadIdx.x][w] : v;
+    (void)__hip_atomic_fetch_max(out + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+hipError_t launch_abs_max(hipStream_t st, const double *a, const double *b, int64_t n,
+                          unsigned long long *out) {
+  if (n <= 0) return hipSuccess;
+  const unsigned nb = (unsigned)std::min<int64_t>((n + 1023) / 1024, 1024);
+  hipLaunchKernelGGL(k_abs_max, dim3(nb), dim3(256), 0, st, a, b, n, out);
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // In-bag rows in ascending order.  The sampler hands over the reference's
 // sample_idx (distinct row ids in shuffled order); a byte flag per row and a
@@ -526,6 +564,26 @@ __global__ __launch_bounds__(256) void k_mark(const int32_t *__restrict__ rows,
                                               int64_t m, uint8_t *__restrict__ flags) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < m) flags[rows[i]] = 1;
+}
+
+// k_mark of a caller's row ids, which may be any: *bad becomes 1 when one is
+// outside [0, n).
+__global__ __launch_bounds__(256) void k_mark_checked(const int64_t *__restrict__ rows, int64_t m,
+                                                      int64_t n, uint8_t *__restrict__ flags,
+                                                      int32_t *__restrict__ bad) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const int64_t r = rows[i];
+  if (r >= 0 && r < n) flags[r] = 1;
+  else *bad = 1;
+}
+
+hipError_t launch_mark_checked(hipStream_t st, const int64_t *rows, int64_t m, int64_t n,
+                               uint8_t *flags, int32_t *bad) {
+  if (m <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_mark_checked, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, rows, m,
+                     n, flags, bad);
+  return hipGetLastError();
 }
 
 __device__ __forceinline__ uint32_t byte_sum(uint4 v) {

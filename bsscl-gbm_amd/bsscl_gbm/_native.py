@@ -36,6 +36,8 @@ _SIGS = {
     "bsscl_build_tree": [_P, _P, _P, _P, _i64, _P, _i32, _i32, _i32, _i32, _f64,
                          _P, _i32, _f64, _f64, _P, _P, _P, _P, _P, _P, _P],
     "bsscl_boost_begin": [_P, _P, _i64, _f64, _f64, _f64],
+    "bsscl_boost_val_begin": [_P, _P, _i64, _f64],
+    "bsscl_boost_val_loss": [_P, _P],
     "bsscl_boost_round": [_P, _P, _i32, _i32, _i32, _f64, _P, _i32, _f64, _f64,
                           _f64, _P, _P, _P, _P, _P, _P, _P, _P],
     "bsscl_boost_get_F": [_P, _P],
@@ -381,6 +383,17 @@ class Engine:
             ptr(tf), ptr(tt), ptr(tv), ptr(tl), ptr(tr), ptr(nc), ptr(sg),
             ptr(loss)))
         return (tf, tt, tv, tl, tr, int(nc[0]), sg), float(loss[0])
+
+    def boost_val_begin(self, y, base_score):
+        """The rows of matrix 1, with labels y, as the run's validation rows."""
+        y = np.ascontiguousarray(y, np.int64)
+        check(lib().bsscl_boost_val_begin(self.handle, ptr(y), len(y), float(base_score)))
+
+    def boost_val_loss(self):
+        """Validation log-loss after the last round returned."""
+        out = np.zeros(1, np.float64)
+        check(lib().bsscl_boost_val_loss(self.handle, ptr(out)))
+        return float(out[0])
 
     def boost_get_F(self, n):
         out = np.empty(n, np.float64)

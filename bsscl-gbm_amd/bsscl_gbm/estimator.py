@@ -99,10 +99,6 @@ def _as_float(X):
     return X
 
 
-def _sigmoid(F):
-    return 1.0 / (1.0 + np.exp(-np.clip(F, -500, 500)))
-
-
 # Rows from which the estimator's label, count and lookup passes (one
 # memory pass each) run in row blocks on a few threads: NumPy's loops
 # release the GIL, and each element, or each block's count, is NumPy's own.
@@ -727,15 +723,16 @@ class HybridHistGBMNumbaV1_0_1:
 
     def _fit_binary(self, eng, y, n_val, y_val, sampler, binary_start):
         w0, w1, self.base_score_ = binary_start
-        F_val = np.full(n_val, self.base_score_) if n_val else None
         eng.boost_begin(y, w0, w1, self.base_score_)
+        if n_val:
+            eng.boost_val_begin(y_val, self.base_score_)
         best_val_loss = np.inf
         rounds_no_improve = 0
         hook = getattr(self, '_round_hook', None)
         self._live_sampler = sampler  # read by profiling hooks during the fit
-        # Without an eval set every round runs: the engine may enqueue the
-        # next round while this one is returned.
-        eng.set_pipeline(not n_val and getattr(self, '_pipeline_rounds', True))
+        # The engine may enqueue the next round while this one is returned.
+        # (Early stopping drops the round that is then in flight.)
+        eng.set_pipeline(getattr(self, '_pipeline_rounds', True))
         try:
             for m in range(self.n_estimators):
                 if hook is not None:
@@ -749,9 +746,7 @@ class HybridHistGBMNumbaV1_0_1:
                 self.train_loss_history_.append(train_loss)
                 val_loss = None
                 if n_val:
-                    F_val += self.learning_rate * eng.predict_tree(1, n_val, tree)
-                    pv = np.clip(_sigmoid(F_val), 1e-15, 1 - 1e-15)
-                    val_loss = -np.mean(y_val * np.log(pv) + (1 - y_val) * np.log(1 - pv))
+                    val_loss = eng.boost_val_loss()
                     self.val_loss_history_.append(val_loss)
                 if self.verbose and ((m + 1) % 20 == 0 or m == 0):
                     msg = f"  ✓ Tree {m+1:>3}/{self.n_estimators}  |  train-loss: {train_loss:.6f}"

@@ -180,6 +180,17 @@ int bsscl_boost_round(bsscl_engine *eng, bsscl_sampler *sampler,
  * round enqueued ahead: turn pipelining off before destroying it. */
 int bsscl_boost_set_pipeline(bsscl_engine *eng, int32_t on);
 
+/*
+ * Validation rows of the boosting run (est:2898-2903): matrix 1, binned as
+ * matrix 0, with labels y int64[n] in {0,1} and scores starting at
+ * base_score.  Called after bsscl_boost_begin and before its first round;
+ * each round then also adds learning_rate * tree to these scores and takes
+ * their log-loss (est:2320-2325), which bsscl_boost_val_loss returns for the
+ * last round returned.  Matrix 1 must stay as it is until the last round.
+ */
+int bsscl_boost_val_begin(bsscl_engine *eng, const int64_t *y, int64_t n, double base_score);
+int bsscl_boost_val_loss(bsscl_engine *eng, double *out);
+
 /* F of the boosting run (float64[n]). */
 int bsscl_boost_get_F(bsscl_engine *eng, double *F_out);
 

@@ -542,6 +542,7 @@ struct bsscl_engine {
   int32_t hist_copies_span = 1;
   // Partition tile of the current tree: 256 threads x part_rows rows.
   int32_t part_rows = 4;
+  int32_t part_parts = 1;  // blocks that share a scatter tile's features
   int32_t part_tile = 1024;
   int32_t hist_blocks_per_cu = 8;
   int32_t hist_rows_per_flush = 10240;       // the root's tiles
@@ -1413,6 +1414,15 @@ int prepare_tree_buffers(bsscl_engine *E, int64_t m, int32_t F_sel, int32_t leve
   E->part_rows = 16;
   while (E->part_rows > 4 && m / ((int64_t)kPartThreads * E->part_rows) < 512) E->part_rows >>= 1;
   E->part_tile = kPartThreads * E->part_rows;
+  // A tile's features are shared out over blocks until about 1,024 blocks
+  // move rows: with few tiles one block walked every batch of four features
+  // alone (a scatter of 75,000 rows x 70 features 36 us, 14 shared; 214,000 x
+  // 48 28 and 17; 8,000 x 16 15.6 and 11).  Twice as many blocks repeat the
+  // routing too often (17 and 18 us; 750,000 x 22, one block per tile, 23 us,
+  // 27 with two).
+  E->part_parts = (int32_t)std::min<int64_t>(
+      (F_sel + 3) / 4,
+      std::max<int64_t>(1, 1024 / std::max<int64_t>(1, (m + E->part_tile - 1) / E->part_tile)));
   // (A level counts the tiles of every candidate or previous parent: at most
   // m / part_tile plus two partial tiles per candidate.)
   const int64_t tcap = m / E->part_tile + 2 * (int64_t)cap + 4;
@@ -1694,7 +1704,7 @@ int launch_partition(bsscl_engine *E, int src, int dst, const PartParent *parent
                                E->track_rid ? E->rid_c[dst & 1].p : nullptr, parents, groups,
                                tiles, plan, max_tiles, E->part_rows, tile_begin,
                                E->tile_cnt_d.p, E->nleft_d.p, E->segs.p, E->hist_node_d.p,
-                               min_samples_leaf, F_sel));
+                               min_samples_leaf, F_sel, E->part_parts));
   CHK(prof_end(E, stop));
   return BSSCL_OK;
 }

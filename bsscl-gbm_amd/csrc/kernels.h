@@ -358,7 +358,7 @@ hipError_t launch_part_scatter(hipStream_t st, const uint8_t *codes_src,
                                int32_t max_tiles, int32_t part_rows,
                                const int32_t *tile_begin, const int32_t *tile_cnt,
                                int64_t *parent_nleft, NodeSeg *segs, int32_t *hist_node,
-                               int32_t min_samples_leaf, int32_t F_sel);
+                               int32_t min_samples_leaf, int32_t F_sel, int32_t parts);
 // Histogram reduction and split search of one level (parents == nullptr:
 // the root, node 0, whose tasks hist_begin[0] .. hist_begin[1] built it).
 // span_parents: the tasks of parent p tiled its own segment (an in-place

@@ -1572,7 +1572,11 @@ void k_part_scatter(
     const LevelPlan *__restrict__ plan, const int32_t *__restrict__ tile_begin,
     const int32_t *__restrict__ tile_cnt, int64_t *__restrict__ parent_nleft,
     NodeSeg *__restrict__ segs, int32_t *__restrict__ hist_node, int32_t min_samples_leaf,
-    int32_t F_sel) {
+    int32_t F_all, int32_t f_part) {
+  // This block's features: part blockIdx.y of the tile's; the first part
+  // moves the (g,h) and writes the children's segments.
+  const int32_t f_first = (int32_t)blockIdx.y * f_part, F_sel = min(F_all, f_first + f_part);
+  const bool first_part = blockIdx.y == 0;
   __shared__ unsigned long long tmp[kPartBlock / 64];
   __shared__ unsigned long long red[kPartBlock / 64][4];
   constexpr int kTile = kPartBlock * R;
@@ -1641,7 +1645,7 @@ void k_part_scatter(
     // left child, its right child, then side 1's.
     const int64_t base[4] = {Pa.start + gpre[0], Pa.start + gtot[0] + gpre[1],
                              Pb.start + gpre[2], Pb.start + gtot[2] + gpre[3]};
-    if (ti == tb0 && tid == 0) {
+    if (first_part && ti == tb0 && tid == 0) {
       if (G.par[0] >= 0)
         write_children(Pa, G.par[0], gtot[0], gtot[1], min_samples_leaf, parent_nleft, segs,
                        hist_node);
@@ -1676,7 +1680,7 @@ void k_part_scatter(
     __syncthreads();
     // (g,h) and row ids: slot s -> its destination row.  (An empty run's
     // offset equals the next one's, so the count below skips it.)
-    for (int sl = tid; sl < vtot; sl += kPartBlock) {
+    for (int sl = first_part ? tid : vtot; sl < vtot; sl += kPartBlock) {
       const int r = (sl >= off[1] ? 1 : 0) + (sl >= off[2] ? 1 : 0) + (sl >= off[3] ? 1 : 0);
       const int64_t d = sel4(r, base[0], base[1], base[2], base[3]) +
                         (sl - sel4(r, off[0], off[1], off[2], off[3]));
@@ -1718,9 +1722,10 @@ void k_part_scatter(
       CodeWords<R> nxt[Q];
 #pragma unroll
       for (int u = 0; u < Q; ++u)
-        nxt[u] = u < F_sel ? load_codes<R>(codes_src + (int64_t)u * ld_c, row, lo, hi)
-                           : zero_codes<R>();
-      for (int f0 = 0, b = 0; f0 < F_sel; f0 += Q, b ^= 1) {
+        nxt[u] = f_first + u < F_sel
+                     ? load_codes<R>(codes_src + (int64_t)(f_first + u) * ld_c, row, lo, hi)
+                     : zero_codes<R>();
+      for (int f0 = f_first, b = 0; f0 < F_sel; f0 += Q, b ^= 1) {
 #pragma unroll
         for (int u = 0; u < Q; ++u) cs[b][u * kPartBlock + tid] = nxt[u].v;
 #pragma unroll
@@ -1798,14 +1803,14 @@ void k_part_scatter(
       CodeWords<R> cur[kQuad];
 #pragma unroll
       for (int u = 0; u < kQuad; ++u) {
-        if (u < F_sel) {
-          cur[u] = load_codes<R>(codes_src + (int64_t)u * ld_c, row, lo, hi);
+        if (f_first + u < F_sel) {
+          cur[u] = load_codes<R>(codes_src + (int64_t)(f_first + u) * ld_c, row, lo, hi);
         } else {
 #pragma unroll
           for (int k = 0; k < R / 4; ++k) cur[u].w[k] = 0u;
         }
       }
-      for (int f0 = 0, b = 0; f0 < F_sel; f0 += kQuad, b ^= 1) {
+      for (int f0 = f_first, b = 0; f0 < F_sel; f0 += kQuad, b ^= 1) {
 #pragma unroll
         for (int g = 0; g < R / 4; ++g) {
           uint4 r;
@@ -1867,14 +1872,17 @@ hipError_t launch_part_scatter(hipStream_t st, const uint8_t *codes_src,
                                int32_t max_tiles, int32_t part_rows,
                                const int32_t *tile_begin, const int32_t *tile_cnt,
                                int64_t *parent_nleft, NodeSeg *segs, int32_t *hist_node,
-                               int32_t min_samples_leaf, int32_t F_sel) {
+                               int32_t min_samples_leaf, int32_t F_sel, int32_t parts) {
   if (max_tiles <= 0) return hipSuccess;
+  // (Whole batches of four features per part.)
+  const int32_t f_part = (F_sel + 4 * parts - 1) / (4 * parts) * 4;
+  const unsigned n_parts = (unsigned)std::max(1, (F_sel + f_part - 1) / f_part);
 #define BSSCL_SCATTER(R, Q)                                                                   \
-  hipLaunchKernelGGL((k_part_scatter<R, Q>), dim3((unsigned)max_tiles), dim3(kPartBlock), 0, st, \
+  hipLaunchKernelGGL((k_part_scatter<R, Q>), dim3((unsigned)max_tiles, n_parts), dim3(kPartBlock), 0, st, \
                      codes_src, codes_dst, ld_c, gh_src, gh_dst, rid_src, rid_dst, parents,      \
                      groups, tiles, plan, tile_begin, tile_cnt, parent_nleft, segs,            \
                      hist_node,                                                                \
-                     min_samples_leaf, F_sel)
+                     min_samples_leaf, F_sel, f_part)
   switch (part_rows) {
     case 4: BSSCL_SCATTER(4, ScatterQ<4>::value); break;
     case 8: BSSCL_SCATTER(8, ScatterQ<8>::value); break;

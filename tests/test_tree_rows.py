@@ -59,3 +59,24 @@ def test_bad_rows_and_gradients_are_refused(engine, size):
     got = engine.build_tree(g, h, rows, feats, *ARGS.values())
     want = om.build_tree(codes, g, h, rows, feats, *ARGS.values())
     assert treecmp.compare(want, got) == "equal"
+
+
+@pytest.mark.parametrize("F", [1, 4, 5, 8, 33])
+@pytest.mark.parametrize("n", [900, 5003, 140_001])
+def test_scatter_shares_a_tiles_features(engine, n, F):
+    """The partition's rows move with every feature of a tile, whichever
+    blocks share them: batches of four, a last one of one, one block each."""
+    print(f"[case] scatter {n} x {F}", flush=True)
+    rng = np.random.default_rng(n + F)
+    # (Few enough bins that no node has an empty one: splits on its two sides
+    # part the same rows and their gains tie.)
+    bins = 4 if n < 2000 else 12 if n < 50_000 else 60
+    codes = rng.integers(0, bins, (n, F)).astype(np.uint8)
+    g, h = rng.standard_normal(n) + 0.02 * codes.sum(1), rng.random(n) + 0.1
+    args = dict(ARGS, max_leaves=31, max_depth=6, min_samples_leaf=20,
+                bin_counts=np.full(F, bins, np.int32), max_bins=bins)
+    feats = np.arange(F, dtype=np.int32)
+    engine.load_codes(0, codes)
+    got = engine.build_tree(g, h, np.arange(n), feats, *args.values())
+    want = om.build_tree(codes, g, h, np.arange(n), feats, *args.values())
+    assert treecmp.compare(want, got) == "equal"

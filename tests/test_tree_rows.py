@@ -80,3 +80,26 @@ def test_scatter_shares_a_tiles_features(engine, n, F):
     got = engine.build_tree(g, h, np.arange(n), feats, *args.values())
     want = om.build_tree(codes, g, h, np.arange(n), feats, *args.values())
     assert treecmp.compare(want, got) == "equal"
+
+
+@pytest.mark.parametrize("F", [64, 65, 80, 113, 128, 129])
+def test_planner_takes_every_feature(engine, F):
+    """The planner's waves take four or eight features each up to 128: the
+    best split may lie in any of them, and of two equal columns the first
+    wins."""
+    print(f"[case] planner {F} features", flush=True)
+    n, bins = 6007, 10
+    rng = np.random.default_rng(F)
+    codes = rng.integers(0, bins, (n, F)).astype(np.uint8)
+    codes[:, F - 1] = codes[:, 3]
+    codes[:, F - 2] = codes[:, F // 2]
+    steer = codes[:, [3, F // 2, F - 3, 4, 60]].astype(np.float64)
+    g = rng.standard_normal(n) + steer @ [0.2, -0.15, 0.1, 0.05, -0.05]
+    h = rng.random(n) + 0.1
+    args = dict(ARGS, max_leaves=31, max_depth=6, min_samples_leaf=20,
+                bin_counts=np.full(F, bins, np.int32), max_bins=bins)
+    feats = np.arange(F, dtype=np.int32)
+    engine.load_codes(0, codes)
+    got = engine.build_tree(g, h, np.arange(n), feats, *args.values())
+    want = om.build_tree(codes, g, h, np.arange(n), feats, *args.values())
+    assert treecmp.compare(want, got) == "equal"

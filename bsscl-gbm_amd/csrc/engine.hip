@@ -309,9 +309,75 @@ int scratch_for_device(int device, unsigned char **out) {
 }  // namespace
 
 namespace {
+constexpr int kMcLanesMax = 2;
 constexpr int kXferPins = 6;
 constexpr int kOutPins = 3;
 constexpr size_t kOutPinBytes = 16u << 20;
+}  // namespace
+
+// What the enqueued work of one tree writes, and its stream.  A multiclass
+// round builds its classes' trees in several lanes at once: lane 0 is the
+// engine's own members of these names, and the others change places with
+// them while their trees are enqueued (TreeLanes).
+struct TreeLane {
+  hipStream_t st = nullptr;
+  hipEvent_t done = nullptr;
+  DevBuf<uint8_t> codes_c[2];
+  DevBuf<GH> gh_c[3];
+  DevBuf<unsigned long long> pool, part_d;
+  int32_t node_alloc = 0, node_cap = 0;
+  int64_t node_stride = 0;
+  DevBuf<NodeSeg> segs;
+  DevBuf<SplitCand> cand;
+  DevBuf<long long> totals;
+  DevBuf<char> table_d;
+  char *table_pin = nullptr;
+  size_t table_pin_bytes = 0;
+  LevelPlan *plan_d = nullptr;
+  NodeOut *nodes_d = nullptr;
+  DevBuf<PartParent> parents_d[2];
+  DevBuf<PartGroup> groups_d;
+  DevBuf<int32_t> tile_begin_d, hist_begin_d, work_flag_d, hist_node_d;
+  DevBuf<double> work_e_d, kept_e_d, parent_e_d[2];
+  DevBuf<int64_t> nleft_d;
+  DevBuf<PartTile> tiles_d;
+  DevBuf<int32_t> tile_cnt_d, level_args_d;
+  DevBuf<HistTask> hist_tasks_d;
+  DevBuf<TreeNodeDev> tree_d;
+};
+
+namespace {
+
+// Calls f with each buffer of a and the same one of b.
+template <typename A, typename B, typename Fn>
+void lane_buffers(A &a, B &b, Fn f) {
+  for (int s = 0; s < 2; ++s) {
+    f(a.codes_c[s], b.codes_c[s]);
+    f(a.parents_d[s], b.parents_d[s]);
+    f(a.parent_e_d[s], b.parent_e_d[s]);
+  }
+  for (int s = 0; s < 3; ++s) f(a.gh_c[s], b.gh_c[s]);
+  f(a.pool, b.pool);
+  f(a.part_d, b.part_d);
+  f(a.segs, b.segs);
+  f(a.cand, b.cand);
+  f(a.totals, b.totals);
+  f(a.table_d, b.table_d);
+  f(a.groups_d, b.groups_d);
+  f(a.tile_begin_d, b.tile_begin_d);
+  f(a.hist_begin_d, b.hist_begin_d);
+  f(a.work_flag_d, b.work_flag_d);
+  f(a.hist_node_d, b.hist_node_d);
+  f(a.work_e_d, b.work_e_d);
+  f(a.kept_e_d, b.kept_e_d);
+  f(a.nleft_d, b.nleft_d);
+  f(a.tiles_d, b.tiles_d);
+  f(a.tile_cnt_d, b.tile_cnt_d);
+  f(a.level_args_d, b.level_args_d);
+  f(a.hist_tasks_d, b.hist_tasks_d);
+  f(a.tree_d, b.tree_d);
+}
+
 }  // namespace
 
 struct bsscl_engine {
@@ -385,6 +451,10 @@ struct bsscl_engine {
   char *mc_out_pin = nullptr;
   size_t mc_out_pin_bytes = 0;
 
+  // A multiclass round's further lanes (buffers are released with the engine).
+  TreeLane mc_lane[kMcLanesMax - 1];
+  hipEvent_t mc_fork = nullptr;
+
   // Tree workspace.
   // Compact row sets: a tree uses sets set_base and set_base + 1 (levels
   // alternate); a boosting round in slot s uses base 2s, so the next round's
@@ -395,10 +465,8 @@ struct bsscl_engine {
   int32_t set_base = 0;
   // A tree's root rows in another set than set_base (-1: set_base).  Its
   // levels then never write it, so the root codes of a multiclass round,
-  // gathered once, serve all its classes (root_codes_ready: the root's
-  // gather brings the (g,h) alone).
+  // gathered once, serve all its classes.
   int32_t root_set = -1;
-  bool root_codes_ready = false;
   // A boosting round's root inputs (RootPack), uploaded by the rows stream
   // into the slot's own arena.
   DevBuf<char> root_d[2];
@@ -683,6 +751,10 @@ int prof_collect(bsscl_engine *E, uint64_t upto = UINT64_MAX) {
 int sync(bsscl_engine *E) {
   HIPCHK(hipStreamSynchronize(E->st_rows));
   HIPCHK(hipStreamSynchronize(E->st));
+  // (The pinned arena serves every lane; one of these is the engine's own
+  // stream while a lane is in its place.)
+  for (TreeLane &l : E->mc_lane)
+    if (l.st) HIPCHK(hipStreamSynchronize(l.st));
   CHK(prof_collect(E));
   E->pin.reset();
   return BSSCL_OK;
@@ -1556,13 +1628,10 @@ int launch_root(bsscl_engine *E, const int32_t *rows32, int64_t m,
   E->feat_d = feat_d;
   E->nb_sel_d = reinterpret_cast<const int32_t *>(dv[kPackNbHot]);
   E->hot_sel_d = E->nb_sel_d + F_sel;
-  // (A boosting round's root rows are already in set b: launch_gather_codes
-  // and launch_gather_gh.)
-  // (With the root's codes already in place, the gather brings the (g,h)
-  // alone: no feature columns.)
+  // (A round's root rows are already in set b: launch_gather_codes and
+  // launch_gather_gh or launch_gather_quantized.)
   if (!gathered)
-    HIPCHK(launch_gather_root(E->st, X.codes.p, X.ld, feat_d, E->root_codes_ready ? 0 : F_sel,
-                              rows32, rows32 ? nullptr : E->rows64.p, m, E->ghq.p,
+    HIPCHK(launch_gather_root(E->st, X.codes.p, X.ld, feat_d, F_sel, rows32, rows32 ? nullptr : E->rows64.p, m, E->ghq.p,
                               E->codes_c[b].p, E->ld_c, E->gh_c[b].p,
                               E->track_rid && b == 0 ? E->rid_c[0].p : nullptr,
                               E->ld_c, E->segs.p, E->hist_node_d.p));
@@ -2962,13 +3031,95 @@ int mc_tree_host(bsscl_engine *E, int32_t k, const std::vector<int32_t> &feats,
   return BSSCL_OK;
 }
 
-// The round's K trees back to back with no host wait between them: per
-// class its quantized gradients, the tree, the tree's replay on the device
-// and F[:, k] += lr * tree(X) (k_mc_apply skips it when the replay failed);
-// then one readback of the K trees.  The classes' gradients all come from
-// the scores before the round (est:3013-3019), so the order of the K
-// updates does not enter any tree, and a class whose device replay failed
-// is built again on the host-driven path from its unchanged gradients.
+// Lanes for the K trees of a multiclass round over m rows.  A tree of one
+// class is a chain of small launches that leaves most of the chip idle, so
+// the classes' chains run beside each other.  Whole fits of 20 (10) rounds
+// with one lane and two: 200,003 x 24, 5 classes 30.5 and 23.4 ms; 20,000 x
+// 20, 3 classes 16.1 and 13.2; 5,000 x 12, 8 classes (10) 16.1 and 11.2; 1M
+// x 28, 5 classes (10) 40.4 and 36.2; 3M x 30, 5 classes (6) 82 and 78.7.
+// Three and four lanes take 23.9 and 24.3 ms at 200,003 rows (the process's
+// four hardware queues also serve the rows, the copies and the caller), and
+// so does the rows stream as the third (24.5).  A tree of more than
+// kLevelsPerCheck levels reads its plan back on the way and a profiled one is
+// timed by itself: one lane.  (Test hook BSSCL_TEST_MC_LANES=1: one lane.)
+int32_t mc_lanes(const bsscl_engine *E, int32_t K, const TreeParams &tp) {
+  if (E->prof > 0 || tp.max_depth > kLevelsPerCheck) return 1;
+  const char *t = std::getenv("BSSCL_TEST_MC_LANES");
+  return t && t[0] == '1' ? 1 : std::min(K, kMcLanesMax);
+}
+
+// The lanes of one round: `use` puts lane i's stream and buffers in the
+// engine's place, `fork` lets every lane start after the work enqueued so far
+// in lane 0, and `join` lets lane 0 go on after all of them.  Lane 0 is back
+// in place when the object goes, and the lanes idle if they were not joined.
+class TreeLanes {
+ public:
+  explicit TreeLanes(bsscl_engine *E, int32_t n) : E_(E), n_(n) {}
+  TreeLanes(const TreeLanes &) = delete;
+  TreeLanes &operator=(const TreeLanes &) = delete;
+  ~TreeLanes() {
+    use(0);
+    if (forked_)
+      for (int32_t i = 1; i < n_; ++i) (void)hipStreamSynchronize(lane(i).st);
+  }
+  void use(int32_t i) {
+    if (cur_ > 0) exchange(lane(cur_));
+    cur_ = i;
+    if (cur_ > 0) exchange(lane(cur_));
+  }
+  int create() {
+    for (int32_t i = 1; i < n_; ++i) {
+      TreeLane &l = lane(i);
+      if (!l.st) HIPCHK(hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking));
+      if (!l.done) HIPCHK(hipEventCreateWithFlags(&l.done, hipEventDisableTiming));
+    }
+    if (n_ > 1 && !E_->mc_fork)
+      HIPCHK(hipEventCreateWithFlags(&E_->mc_fork, hipEventDisableTiming));
+    return BSSCL_OK;
+  }
+  int fork() {
+    if (n_ < 2) return BSSCL_OK;
+    use(0);
+    HIPCHK(hipEventRecord(E_->mc_fork, E_->st));
+    forked_ = true;
+    for (int32_t i = 1; i < n_; ++i) HIPCHK(hipStreamWaitEvent(lane(i).st, E_->mc_fork, 0));
+    return BSSCL_OK;
+  }
+  int join() {
+    use(0);
+    for (int32_t i = 1; i < n_; ++i) {
+      HIPCHK(hipEventRecord(lane(i).done, lane(i).st));
+      HIPCHK(hipStreamWaitEvent(E_->st, lane(i).done, 0));
+    }
+    forked_ = false;
+    return BSSCL_OK;
+  }
+
+ private:
+  TreeLane &lane(int32_t i) { return E_->mc_lane[i - 1]; }
+  void exchange(TreeLane &l) {
+    lane_buffers(*E_, l, [](auto &a, auto &b) { std::swap(a, b); });
+    std::swap(E_->st, l.st);
+    std::swap(E_->node_alloc, l.node_alloc);
+    std::swap(E_->node_cap, l.node_cap);
+    std::swap(E_->node_stride, l.node_stride);
+    std::swap(E_->table_pin, l.table_pin);
+    std::swap(E_->table_pin_bytes, l.table_pin_bytes);
+    std::swap(E_->plan_d, l.plan_d);
+    std::swap(E_->nodes_d, l.nodes_d);
+  }
+  bsscl_engine *E_;
+  int32_t n_, cur_ = 0;
+  bool forked_ = false;
+};
+
+// The round's K trees with no host wait between them, in turn over the
+// lanes: per class its quantized gradients, the tree, the tree's replay on
+// the device and F[:, k] += lr * tree(X) (k_mc_apply skips it when the
+// replay failed); then one readback of the K trees.  The classes' gradients
+// all come from the scores before the round (est:3013-3019), so the order of
+// the K updates does not enter any tree, and a class whose device replay
+// failed is built again on the host-driven path from its unchanged gradients.
 // `out(k)` gives class k's output arrays.
 template <typename OutFn>
 int mc_trees_device(bsscl_engine *E, const std::vector<int32_t> &feats,
@@ -2981,50 +3132,68 @@ int mc_trees_device(bsscl_engine *E, const std::vector<int32_t> &feats,
   const size_t per = round_out_bytes(M);
   // (mc_out_d is released only when no copy reads it: the previous call
   // ended with a synchronisation.)
-  CHK(E->tree_d.ensure((size_t)M));
   CHK(E->mc_out_d.ensure(per * (size_t)K));
   CHK(ensure_host_pinned(E, E->mc_out_pin, E->mc_out_pin_bytes, per * (size_t)K));
-  // The K trees share their rows and features: the round's root codes are
-  // gathered once into set 2, which the trees' levels never write (they
-  // alternate between sets 0 and 1), and each class's root gathers its
-  // (g,h) alone.
+  // The K trees share their rows and features: the round's root codes and
+  // root inputs are made once, the codes in set 2, which the trees' levels
+  // never write (they alternate between sets 0 and 1), and each class's root
+  // gathers its (g,h) alone.
   // (Rows given as int64 by bsscl_mc_round have no int32 list for that
-  // gather: each class then gathers its root itself.)
+  // gather: each class then gathers its root itself, one after the other.)
   const bool shared_root = E->mc_rows32 != nullptr;
   E->set_base = 0;
   E->root_set = shared_root ? 2 : -1;
   struct RootReset {
     bsscl_engine *e;
-    ~RootReset() {
-      e->root_set = -1;
-      e->root_codes_ready = false;
-    }
+    ~RootReset() { e->root_set = -1; }
   } root_reset{E};
-  CHK(prepare_tree_buffers(E, m, F_sel, std::max(1, tp.max_depth), tp.max_leaves));
+  const int32_t n_lanes = shared_root ? mc_lanes(E, K, tp) : 1;
+  TreeLanes lanes(E, n_lanes);
+  CHK(lanes.create());
+  for (int32_t i = 0; i < n_lanes; ++i) {
+    lanes.use(i);
+    CHK(E->tree_d.ensure((size_t)M));
+    CHK(prepare_tree_buffers(E, m, F_sel, std::max(1, tp.max_depth), tp.max_leaves));
+  }
+  lanes.use(0);
+  PreRoot pre;
   if (shared_root) {
     CHK(upload(E, E->mc_feat_d, feats.data(), feats.size()));
     HIPCHK(launch_gather_codes(E->st, X.codes.p, X.ld, E->mc_feat_d.p, F_sel, E->mc_rows32, m,
                                E->codes_c[2].p, E->ld_c, E->ld_c));
-    E->root_codes_ready = true;
+    RootPack R;
+    build_root_pack(E, m, feats, nb_sel, R);
+    CHK(upload_pack(E, R.pk, pre.dev));
+    pre.n_hist = R.rp.n_hist;
+    CHK(lanes.fork());
   }
   for (int32_t k = 0; k < K; ++k) {
+    lanes.use(k % n_lanes);
     // The class's fixed point: from the maxima the host read back, or from
     // those on the device (the same multipliers, dev_fixed_mul), with the
     // hessian bound max weight / 4 for the planner's kept-split rule.
     DevScale dv{nullptr, 0, 0};
+    double gm = 1.0, hm = 1.0;
     if (E->mc_scales_host) {
       CHK(mc_class_scales(E, k));
+      gm = E->mc_gm[(size_t)k];
+      hm = E->mc_hm[(size_t)k];
     } else {
       dv = DevScale{E->mc_max.p + 2 * k, fixed_bits(m), 0};
       E->g_scale = E->h_scale = 1.0;  // (the kernels take dv's)
       E->h_bound = E->mc_hbound;
     }
-    HIPCHK(launch_quantize(E->st, E->mc_G.p + (size_t)k * n, E->mc_H.p + (size_t)k * n, n,
-                           dv.max ? 1.0 : E->mc_gm[(size_t)k], dv.max ? 1.0 : E->mc_hm[(size_t)k],
-                           E->ghq.p, dv));
+    const double *g = E->mc_G.p + (size_t)k * n, *h = E->mc_H.p + (size_t)k * n;
+    if (shared_root)
+      HIPCHK(launch_gather_quantized(
+          E->st, g, h, E->mc_rows32, m, gm, hm, dv, E->gh_c[2].p, E->ld_c, E->segs.p,
+          E->hist_node_d.p, reinterpret_cast<const LevelPlan *>(pre.dev[kPackPlan]), E->plan_d));
+    else
+      HIPCHK(launch_quantize(E->st, g, h, n, gm, hm, E->ghq.p, dv));
     int32_t run = 0;
     E->round_dev = dv;
-    const int trc = launch_tree(E, E->mc_rows32, m, feats, nb_sel, tp, &run);
+    const int trc = launch_tree(E, E->mc_rows32, m, feats, nb_sel, tp, &run, true, shared_root,
+                                shared_root ? &pre : nullptr);
     E->round_dev = DevScale{nullptr, 0, 0};
     CHK(trc);
     char *base = E->mc_out_d.p + (size_t)k * per;
@@ -3036,12 +3205,12 @@ int mc_trees_device(bsscl_engine *E, const std::vector<int32_t> &feats,
     HIPCHK(launch_mc_apply(E->st, X.codes.p, X.ld, n, E->tree_d.p, &hdr->node_count, lr,
                            E->mc_F.p + (size_t)k * n));
   }
+  CHK(lanes.join());
   HIPCHK(hipMemcpyAsync(E->mc_out_pin, E->mc_out_d.p, per * (size_t)K, hipMemcpyDeviceToHost,
                         E->st));
   CHK(sync(E));
   // (A class rebuilt on the host-driven path below gathers its own root.)
   E->root_set = -1;
-  E->root_codes_ready = false;
   for (int32_t k = 0; k < K; ++k) {
     TreeOut o = out(k);
     const char *base = E->mc_out_pin + (size_t)k * per;
@@ -3593,6 +3762,13 @@ void bsscl_engine_destroy(bsscl_engine *E) {
   E->mc_out_d.release();
   E->mc_feat_d.release();
   if (E->mc_out_pin) (void)hipHostFree(E->mc_out_pin);
+  for (TreeLane &l : E->mc_lane) {
+    lane_buffers(l, l, [](auto &b, auto &) { b.release(); });
+    if (l.table_pin) (void)hipHostFree(l.table_pin);
+    if (l.done) (void)hipEventDestroy(l.done);
+    if (l.st) (void)hipStreamDestroy(l.st);
+  }
+  if (E->mc_fork) (void)hipEventDestroy(E->mc_fork);
   E->level_args_d.release();
   E->lvl_d.release();
   E->table_d.release();

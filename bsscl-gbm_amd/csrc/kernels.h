@@ -315,6 +315,12 @@ hipError_t launch_gather_gh(hipStream_t st, const double *F, const uint8_t *y,
                             int64_t pad_to, NodeSeg *segs, int32_t *hist_node,
                             const LevelPlan *plan_src = nullptr,
                             LevelPlan *plan_dst = nullptr);
+// The second part for a multiclass round's class.
+hipError_t launch_gather_quantized(hipStream_t st, const double *g, const double *h,
+                                   const int32_t *rows32, int64_t m, double g_mul, double h_mul,
+                                   DevScale dev, GH *gh_c, int64_t pad_to, NodeSeg *segs,
+                                   int32_t *hist_node, const LevelPlan *plan_src,
+                                   LevelPlan *plan_dst);
 // Level kernels take their work counts from a device LevelPlan; the grid
 // argument (blocks, tasks or parents) is an upper bound, and blocks loop
 // over the work with a grid stride, so any bound >= 1 gives the same result.

@@ -761,6 +761,50 @@ __global__ __launch_bounds__(256) void k_gather_gh(
   gh_c[k] = q;
 }
 
+// The same from a class's gradients and hessians.  (Quantizing every row
+// first, gathering those and copying the plan took three launches a tree.)
+__global__ __launch_bounds__(256) void k_gather_quantized(
+    const double *__restrict__ g, const double *__restrict__ h,
+    const int32_t *__restrict__ rows32, int64_t m, double g_mul, double h_mul, DevScale dev,
+    GH *__restrict__ gh_c, int64_t pad_to, NodeSeg *__restrict__ segs,
+    int32_t *__restrict__ hist_node, const LevelPlan *__restrict__ plan_src,
+    LevelPlan *__restrict__ plan_dst) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (dev.max) {
+    g_mul = dev_fixed_mul(dev.max[0], dev.bits);
+    h_mul = dev_fixed_mul(dev.max[1], dev.bits);
+  }
+  if (k == 0) {
+    *plan_dst = *plan_src;
+    NodeSeg r;
+    r.start = 0;
+    r.count = m;
+    r.valid = 1;
+    r.is_small = 1;
+    segs[0] = r;
+    hist_node[0] = 0;
+  }
+  if (k >= pad_to) return;
+  GH q = make_longlong2(0, 0);
+  if (k < m) {
+    const int32_t i = rows32[k];
+    q = make_longlong2(__double2ll_rn(g[i] * g_mul), __double2ll_rn(h[i] * h_mul));
+  }
+  gh_c[k] = q;
+}
+
+hipError_t launch_gather_quantized(hipStream_t st, const double *g, const double *h,
+                                   const int32_t *rows32, int64_t m, double g_mul, double h_mul,
+                                   DevScale dev, GH *gh_c, int64_t pad_to, NodeSeg *segs,
+                                   int32_t *hist_node, const LevelPlan *plan_src,
+                                   LevelPlan *plan_dst) {
+  if (pad_to <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_gather_quantized, dim3((unsigned)((pad_to + 255) / 256)), dim3(256), 0, st,
+                     g, h, rows32, m, g_mul, h_mul, dev, gh_c, pad_to, segs, hist_node, plan_src,
+                     plan_dst);
+  return hipGetLastError();
+}
+
 hipError_t launch_gather_codes(hipStream_t st, const uint8_t *codes, int64_t ld,
                                const int32_t *feat, int32_t F_sel, const int32_t *rows32,
                                int64_t m, uint8_t *codes_c, int64_t ld_c, int64_t pad_to) {

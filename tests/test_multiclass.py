@@ -367,6 +367,30 @@ def test_multiclass_round_paths_agree(engine, monkeypatch, K, subsample):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,K,depth", [(70_001, 5, 6), (3000, 3, 8), (900, 16, 3), (4000, 4, 9)])
+def test_multiclass_lanes_agree(monkeypatch, n, K, depth):
+    """The classes' trees built in two lanes beside each other are those
+    built one after the other, at odd and even class counts, up to the depth
+    that lanes take (8) and past it, and in a fit after a larger one on the
+    same engine."""
+    from bsscl_gbm import HybridHistGBMNumbaV1_0_1
+    print(f"[case] multiclass lanes n={n} K={K} depth={depth}", flush=True)
+    X, y = _mc_data(n, 11, K, seed=90 + K)
+    fits = []
+    for lanes in ("1", "2", "2"):
+        monkeypatch.setenv("BSSCL_TEST_MC_LANES", lanes)
+        fits.append(HybridHistGBMNumbaV1_0_1(verbose=False, n_estimators=6, max_depth=depth,
+                                             n_bins=100, random_state=4).fit(X, y))
+    for got in fits[1:]:
+        assert got.train_loss_history_ == fits[0].train_loss_history_
+        for k in range(K):
+            for a, b in zip(fits[0].mc_trees[k], got.mc_trees[k]):
+                assert a[5] == b[5]
+                for i in (0, 1, 2, 3, 4, 6):
+                    np.testing.assert_array_equal(a[i][:a[5]], b[i][:a[5]])
+
+
+@pytest.mark.gpu
 def test_multiclass_round_ahead_handed_back(engine):
     """An early-stopped multiclass fit leaves a round taken ahead by the
     engine; the fit hands it back before closing its sampler, and the next

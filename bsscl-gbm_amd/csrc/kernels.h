@@ -102,7 +102,7 @@ struct PlanArgs {
   // min_samples_leaf rows (est:614-615, 678-683).  Then the level's other
   // candidates with a split count as kept splits ranked above a candidate.
   int32_t all_kept;
-  int32_t part_rows;      // rows per thread of a partition tile (4, 8 or 16)
+  int32_t part_rows;      // rows per thread of a partition tile (4 or 8)
   // In place and grouped levels: blocks 1.. of the planner launch count the
   // level's partition tiles (plan_count_role) while block 0 plans.
   int32_t fused_count;
@@ -174,7 +174,7 @@ struct TreeNodeDev {
   double value;
 };
 
-// Partition tiles are runs of 256 * R rows (R = 4, 8 or 16 rows per thread,
+// Partition tiles are runs of 256 * R rows (R = 4 or 8 rows per thread,
 // chosen per tree) starting at a 16-row boundary (tiles of one parent are
 // consecutive; rows outside the parent's segment are masked).
 constexpr int kPartThreads = 256;

@@ -1371,7 +1371,7 @@ hipError_t launch_hist(hipStream_t st, const uint8_t *codes_c, int64_t ld_c,
 
 // ---------------------------------------------------------------------------
 // Partition (est:662-674, made stable): count, scan, scatter.  A tile is 256
-// threads x R rows (R = 4, 8 or 16, chosen per tree: 1024 to 4096 rows)
+// threads x R rows (R = 4 or 8, chosen per tree: 1024 or 2048 rows)
 // starting at a 16-row boundary; rows of the tile outside its group's
 // segment are masked.  A thread reads its R rows' codes of a feature as one
 // R-byte load.  A group (PartGroup) sends each row by up to two splits to
@@ -1383,7 +1383,6 @@ constexpr int kPartBlock = 256;
 template <int R> struct CodesR;  // R consecutive codes as one load
 template <> struct CodesR<4> { using T = uint32_t; };
 template <> struct CodesR<8> { using T = uint2; };
-template <> struct CodesR<16> { using T = uint4; };
 
 template <int R>
 union CodeWords {
@@ -1457,6 +1456,21 @@ __device__ __forceinline__ Route<R> route_load(const uint8_t *__restrict__ codes
   return q;
 }
 
+// Bit k: code k of c is above bin.  (Two codes to a 32-bit add, which carries
+// into bit 8 of its half when code + 255 - bin does not fit a byte.)
+template <int R>
+__device__ __forceinline__ uint32_t codes_above(const CodeWords<R> &c, uint32_t bin) {
+  const uint32_t add = (255u - min(bin, 255u)) * 0x00010001u;
+  uint32_t m = 0u;
+#pragma unroll
+  for (int k = 0; k < R / 4; ++k) {
+    const uint32_t even = (c.w[k] & 0x00ff00ffu) + add, odd = ((c.w[k] >> 8) & 0x00ff00ffu) + add;
+    const uint32_t t = ((even >> 8) & 0x00010001u) | ((odd >> 7) & 0x00020002u);
+    m |= ((t | (t >> 14)) & 15u) << (4 * k);
+  }
+  return m;
+}
+
 // Bit k of run[r]: row row+k lies in the tile's part of the group and goes
 // to run r (side 1 when the group's split sends it right, then right when
 // its side's parent's split does: code > bin).  Rows of a side without a
@@ -1464,22 +1478,17 @@ __device__ __forceinline__ Route<R> route_load(const uint8_t *__restrict__ codes
 template <int R>
 __device__ __forceinline__ void route_masks(const Route<R> &q, const PartGroup &G, int64_t row,
                                             uint32_t (&run)[4]) {
-  const bool has_a = G.par[0] >= 0, has_b = G.par[1] >= 0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) run[r] = 0u;
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const int sh = 8 * (k & 3);
-    const bool in = (row + k >= q.lo) && (row + k < q.hi);
-    const bool side = G.fpos >= 0 && ((q.c0.w[k >> 2] >> sh) & 255u) > (uint32_t)G.bin;
-    const bool right = side ? ((q.cb.w[k >> 2] >> sh) & 255u) > q.bin_b
-                            : ((q.ca.w[k >> 2] >> sh) & 255u) > q.bin_a;
-    const uint32_t bit = ((in && (side ? has_b : has_a)) ? 1u : 0u) << k;
-    run[0] |= (!side && !right) ? bit : 0u;
-    run[1] |= (!side && right) ? bit : 0u;
-    run[2] |= (side && !right) ? bit : 0u;
-    run[3] |= (side && right) ? bit : 0u;
-  }
+  const uint32_t side = G.fpos >= 0 ? codes_above<R>(q.c0, (uint32_t)G.bin) : 0u;
+  const uint32_t right = (side & codes_above<R>(q.cb, q.bin_b)) |
+                         (~side & codes_above<R>(q.ca, q.bin_a));
+  const int klo = (int)min<int64_t>(R, max<int64_t>(0, q.lo - row));
+  const int khi = (int)min<int64_t>(R, max<int64_t>(0, q.hi - row));
+  uint32_t in = ((1u << khi) - 1u) & ~((1u << klo) - 1u);
+  in &= (G.par[0] >= 0 ? ~side : 0u) | (G.par[1] >= 0 ? side : 0u);
+  run[0] = in & ~side & ~right;
+  run[1] = in & ~side & right;
+  run[2] = in & side & ~right;
+  run[3] = in & side & right;
 }
 
 // The side parents of a group (start 0 and no split when a side has none).
@@ -1508,7 +1517,7 @@ __global__ __launch_bounds__(kPartBlock) void k_part_count(
     const Route<R> rt = route_load<R>(codes_c, ld_c, t, G, Pa, Pb, row);
     uint32_t run[4];
     route_masks<R>(rt, G, row, run);
-    // Four counts as 16-bit fields (a tile has at most 4096 rows).
+    // Four counts as 16-bit fields (a tile has at most 2048 rows).
     const uint32_t a = wave_sum((uint32_t)__builtin_popcount(run[0]) |
                                 ((uint32_t)__builtin_popcount(run[1]) << 16));
     const uint32_t b = wave_sum((uint32_t)__builtin_popcount(run[2]) |
@@ -1540,7 +1549,6 @@ hipError_t launch_part_count(hipStream_t st, const uint8_t *codes_c,
   switch (part_rows) {
     case 4: BSSCL_COUNT(4); break;
     case 8: BSSCL_COUNT(8); break;
-    case 16: BSSCL_COUNT(16); break;
     default: return hipErrorInvalidValue;
   }
 #undef BSSCL_COUNT
@@ -1561,15 +1569,21 @@ __device__ __forceinline__ void wave_side_counts(const int32_t *__restrict__ til
 // keeping the input order within each run.  A row's slot (the tile's rows
 // of run 0, then run 1, 2, 3) is a block-wide exclusive scan of per-thread
 // counts plus its rank among the thread's R rows; inv[slot] is the row it
-// came from.  The output is cut into R-byte chunks aligned in the
+// came from.  The output is cut into chunks of four rows aligned in the
 // destination.  Features move four at a time: each tile row's four codes go
-// to LDS as one 32-bit word (a 4x4 byte transpose of the thread's loads),
-// and each output chunk reads its R source rows' words and transposes them
-// back into one R-byte store per feature (byte stores only for the chunks
-// at the ends of a run, which it shares with the neighbouring tiles).
-// (g,h) and row ids are gathered through inv and stored as consecutive
-// elements.
-constexpr int kChunkSlots = 2;  // output chunks a thread may own (<= 264 per tile)
+// to LDS as one 32-bit word (4x4 byte transposes of the thread's loads), and
+// each output chunk reads its four source rows' words and transposes them
+// back into one 32-bit store per feature, neighbouring lanes to neighbouring
+// words (byte stores only for the chunks at the ends of a run, which it
+// shares with the neighbouring tiles).  (g,h) and row ids are gathered
+// through inv and stored as consecutive elements.
+// What bounds it: the bytes, moved in many short runs.  5M rows x 35 features
+// (510 MB) take 125 us a level (4.1 TB/s).  16-row threads that gathered
+// their 16-byte chunks byte by byte (64 LDS byte reads a thread and batch,
+// four banks for a wave) took 178; with these words and chunks they take
+// 140.  The routing as byte masks (codes_above) instead of a compare per row
+// and run is 14 us of the 8-row tiles'.
+constexpr int kChunkRows = 4;
 constexpr int kQuad = 4;        // features per LDS pass (one 32-bit word per row)
 
 // 4x4 byte transpose: byte j of r_i is byte i of w_j.
@@ -1585,18 +1599,9 @@ __device__ __forceinline__ void transpose4(uint32_t w0, uint32_t w1, uint32_t w2
   r2 = (lo01 >> 16) | (lo23 & 0xffff0000u);
   r3 = (hi01 >> 16) | (hi23 & 0xffff0000u);
 }
-// Waves per SIMD the register budget must allow (4: 128 VGPRs, which the
-// four-run routing needs without spilling).  16-row tiles move one feature
-// per barrier through LDS bytes instead of four through words: the word
-// transposes of 16 rows need more registers than that.
-template <int R> struct ScatterWaves { static constexpr int value = 4; };
-// Features a 16-row tile stages per barrier: each thread's next Q codes
-// loads are in flight while it gathers the current ones.  At 10M x 50
-// (35 features) one feature per barrier kept about 16 KB of loads in flight
-// per CU and moved 2.9 TB/s; Q = 2, 4 and 8 ran the round in 2.49, 2.46 and
-// 2.56 ms against 2.54 (Q = 8: 74 KB of LDS, two blocks per CU).
-template <int R> struct ScatterQ { static constexpr int value = 1; };
-template <> struct ScatterQ<16> { static constexpr int value = 4; };
+// Waves per SIMD the register budget must allow (128 VGPRs, which the
+// four-run routing needs without spilling; LDS allows as many).
+constexpr int kScatterWaves = 4;
 
 // One of four values by a run index r in 0..3, as selects of values (an
 // array indexed by r would live in scratch memory).
@@ -1605,8 +1610,8 @@ __device__ __forceinline__ T sel4(int r, T a, T b, T c, T d) {
   return r == 0 ? a : r == 1 ? b : r == 2 ? c : d;
 }
 
-template <int R, int Q = ScatterQ<R>::value>
-__global__ __launch_bounds__(kPartBlock) __attribute__((amdgpu_waves_per_eu(ScatterWaves<R>::value)))
+template <int R>
+__global__ __launch_bounds__(kPartBlock) __attribute__((amdgpu_waves_per_eu(kScatterWaves)))
 void k_part_scatter(
     const uint8_t *__restrict__ codes_src, uint8_t *__restrict__ codes_dst,
     int64_t ld_c, const GH *__restrict__ gh_src, GH *__restrict__ gh_dst,
@@ -1624,12 +1629,14 @@ void k_part_scatter(
   __shared__ unsigned long long tmp[kPartBlock / 64];
   __shared__ unsigned long long red[kPartBlock / 64][4];
   constexpr int kTile = kPartBlock * R;
-  __shared__ uint16_t inv[kTile];
-  constexpr bool kQuads = R < 16;
-  // Four features' codes per tile row (16-row tiles: Q features' codes per
-  // thread), double buffered.
-  __shared__ __align__(16) uint32_t rows4[2][kQuads ? kTile : 1];
-  __shared__ typename CodesR<R>::T cs[2][kQuads ? 1 : Q * kPartBlock];
+  // Four features' codes per tile row, double buffered; until the second
+  // batch its buffer holds inv, which is read before the first batch's
+  // barrier only.
+  __shared__ __align__(16) uint32_t rows4[2][kTile];
+  uint16_t *inv = reinterpret_cast<uint16_t *>(rows4[1]);
+  // Output chunks a thread may own (a run has at most len / 4 + 1.5).
+  constexpr int kSlots = R / kChunkRows + 1;
+  static_assert(kSlots * kPartBlock >= kTile / kChunkRows + 6, "every chunk has an owner");
   const int32_t n_tiles = plan->n_tiles;
   const int tid = (int)threadIdx.x;
   for (int32_t ti = (int32_t)blockIdx.x; ti < n_tiles; ti += (int32_t)gridDim.x) {
@@ -1668,7 +1675,7 @@ void k_part_scatter(
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[tid >> 6][r] = acc[r];
     }
-    // This thread's counts as four 16-bit fields (a tile has at most 4096 rows).
+    // This thread's counts as four 16-bit fields (a tile has at most 2048 rows).
     const unsigned long long packed = (unsigned long long)__builtin_popcount(run[0]) |
                                       ((unsigned long long)__builtin_popcount(run[1]) << 16) |
                                       ((unsigned long long)__builtin_popcount(run[2]) << 32) |
@@ -1709,19 +1716,30 @@ void k_part_scatter(
     off[3] = off[2] + len[2];
     const int vtot = off[3] + len[3];
     {
-      int rk[4] = {0, 0, 0, 0};
+      const uint32_t side = run[2] | run[3], right = run[1] | run[3];
+      const uint32_t in = run[0] | run[1] | side | right;
+      int slot[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) slot[r] = off[r] + tpre[r];
 #pragma unroll
       for (int k = 0; k < R; ++k) {
+        const bool sk = (side >> k) & 1u, rk = (right >> k) & 1u;
+        const int to = sk ? (rk ? slot[3] : slot[2]) : (rk ? slot[1] : slot[0]);
+        if ((in >> k) & 1u) inv[to] = (uint16_t)(R * tid + k);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if ((run[r] >> k) & 1u) {
-            inv[off[r] + tpre[r] + rk[r]] = (uint16_t)(R * tid + k);
-            ++rk[r];
-          }
-        }
+        for (int r = 0; r < 4; ++r) slot[r] += (int)((run[r] >> k) & 1u);
       }
     }
     __syncthreads();
+    CodeWords<R> cur[kQuad];
+    auto load = [&](int f0) {
+#pragma unroll
+      for (int u = 0; u < kQuad; ++u)
+        cur[u] = f0 + u < F_sel
+                     ? load_codes<R>(codes_src + (int64_t)(f0 + u) * ld_c, row, lo, hi)
+                     : zero_codes<R>();
+    };
+    load(f_first);
     // (g,h) and row ids: slot s -> its destination row.  (An empty run's
     // offset equals the next one's, so the count below skips it.)
     for (int sl = first_part ? tid : vtot; sl < vtot; sl += kPartBlock) {
@@ -1732,173 +1750,76 @@ void k_part_scatter(
       gh_dst[d] = gh_src[src];
       if (rid_dst) rid_dst[d] = rid_src[src];
     }
-    // Output chunks: each run's aligned R-byte chunks, runs in order.
+    // Output chunks: each run's aligned chunks, runs in order.
     int cum[4], n_chunks = 0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       cum[r] = n_chunks;
-      n_chunks += len[r] ? (int)((base[r] + len[r] + R - 1) / R - base[r] / R) : 0;
+      n_chunks += len[r] ? (int)((base[r] + len[r] + kChunkRows - 1) / kChunkRows -
+                                 base[r] / kChunkRows)
+                         : 0;
     }
-    if constexpr (!kQuads) {
-      // 16-row tiles.  Per owned chunk: its destination row, the slot (inv
-      // index) of its first byte and the bytes [klo, khi) that lie in its
-      // run (all 16 for a full chunk); each batch of Q features reads the
-      // chunk's 16 tile rows from inv once.
-      int64_t cdst[kChunkSlots];
-      int32_t cinv[kChunkSlots], kr[kChunkSlots];
-      bool cown[kChunkSlots];
+    // Per owned chunk: its destination row (rows fit 32 bits) and the tile
+    // rows it copies (0xffff: outside the run, not written).
+    uint32_t cdst[kSlots], csrc[kSlots][kChunkRows / 2];
 #pragma unroll
-      for (int q = 0; q < kChunkSlots; ++q) {
-        const int c = tid + q * kPartBlock;
-        cown[q] = c < n_chunks;
-        const int r = (c >= cum[1] ? 1 : 0) + (c >= cum[2] ? 1 : 0) + (c >= cum[3] ? 1 : 0);
-        const int64_t D = sel4(r, base[0], base[1], base[2], base[3]);
-        const int L = sel4(r, len[0], len[1], len[2], len[3]);
-        const int S = sel4(r, off[0], off[1], off[2], off[3]);
-        const int64_t c0 =
-            (D & ~int64_t(R - 1)) + R * (int64_t)(c - sel4(r, cum[0], cum[1], cum[2], cum[3]));
-        cdst[q] = c0;
-        cinv[q] = S + (int)(c0 - D);
-        const int klo = (int)max<int64_t>(0, D - c0);
-        const int khi = (int)min<int64_t>(R, D + L - c0);
-        kr[q] = klo | (khi << 8);
-      }
-      CodeWords<R> nxt[Q];
+    for (int q = 0; q < kSlots; ++q) {
+      const int c = tid + q * kPartBlock;
+      const int r = (c >= cum[1] ? 1 : 0) + (c >= cum[2] ? 1 : 0) + (c >= cum[3] ? 1 : 0);
+      const int64_t D = sel4(r, base[0], base[1], base[2], base[3]);
+      const int L = sel4(r, len[0], len[1], len[2], len[3]);
+      const int S = sel4(r, off[0], off[1], off[2], off[3]);
+      const int64_t c0 = (D & ~int64_t(kChunkRows - 1)) +
+                         kChunkRows * (int64_t)(c - sel4(r, cum[0], cum[1], cum[2], cum[3]));
+      cdst[q] = (uint32_t)c0;
 #pragma unroll
-      for (int u = 0; u < Q; ++u)
-        nxt[u] = f_first + u < F_sel
-                     ? load_codes<R>(codes_src + (int64_t)(f_first + u) * ld_c, row, lo, hi)
-                     : zero_codes<R>();
-      for (int f0 = f_first, b = 0; f0 < F_sel; f0 += Q, b ^= 1) {
+      for (int k = 0; k < kChunkRows; k += 2) {
+        uint32_t pairv = 0u;
 #pragma unroll
-        for (int u = 0; u < Q; ++u) cs[b][u * kPartBlock + tid] = nxt[u].v;
-#pragma unroll
-        for (int u = 0; u < Q; ++u)
-          if (f0 + Q + u < F_sel)
-            nxt[u] = load_codes<R>(codes_src + (int64_t)(f0 + Q + u) * ld_c, row, lo, hi);
-        __syncthreads();
-        const int nf = min(Q, F_sel - f0);
-#pragma unroll
-        for (int q = 0; q < kChunkSlots; ++q) {
-          if (!cown[q]) continue;
-          const int klo = kr[q] & 255, khi = kr[q] >> 8;
-          if (klo == 0 && khi == R) {
-            uint32_t src[R];
-#pragma unroll
-            for (int k = 0; k < R; ++k) src[k] = inv[cinv[q] + k];
-#pragma unroll
-            for (int u = 0; u < Q; ++u) {
-              if (u >= nf) break;
-              const uint8_t *tb = reinterpret_cast<const uint8_t *>(cs[b] + u * kPartBlock);
-              CodeWords<R> o;
-#pragma unroll
-              for (int k = 0; k < R / 4; ++k)
-                o.w[k] = (uint32_t)tb[src[4 * k]] | ((uint32_t)tb[src[4 * k + 1]] << 8) |
-                         ((uint32_t)tb[src[4 * k + 2]] << 16) |
-                         ((uint32_t)tb[src[4 * k + 3]] << 24);
-              *reinterpret_cast<typename CodesR<R>::T *>(codes_dst + (int64_t)(f0 + u) * ld_c +
-                                                         cdst[q]) = o.v;
-            }
-          } else {
-            for (int u = 0; u < nf; ++u) {
-              const uint8_t *tb = reinterpret_cast<const uint8_t *>(cs[b] + u * kPartBlock);
-              uint8_t *dcol = codes_dst + (int64_t)(f0 + u) * ld_c;
-              for (int k = klo; k < khi; ++k) dcol[cdst[q] + k] = tb[inv[cinv[q] + k]];
-            }
-          }
+        for (int h = 0; h < 2; ++h) {
+          const int64_t dr = c0 + k + h;
+          const bool in = c < n_chunks && dr >= D && dr < D + L;
+          const uint32_t src = in ? (uint32_t)inv[S + (int)(dr - D)] : 0xffffu;
+          pairv |= src << (16 * h);
         }
+        csrc[q][k >> 1] = pairv;
       }
-    } else {
-      // Per owned chunk: its destination row and, per byte, the tile row it
-      // copies (0xffff: outside the run, not written).
-      int64_t cdst[kChunkSlots];
-      uint32_t csrc[kChunkSlots][R / 2];  // R x u16 tile rows
-      bool cfull[kChunkSlots], cown[kChunkSlots];
+    }
+    // Batches of four features: one barrier each, the next batch's loads in
+    // flight meanwhile, then the owned chunks gathered and stored.
+    for (int f0 = f_first, b = 0; f0 < F_sel; f0 += kQuad, b ^= 1) {
 #pragma unroll
-      for (int q = 0; q < kChunkSlots; ++q) {
-        const int c = tid + q * kPartBlock;
-        cown[q] = c < n_chunks;
-        const int r = (c >= cum[1] ? 1 : 0) + (c >= cum[2] ? 1 : 0) + (c >= cum[3] ? 1 : 0);
-        const int64_t D = sel4(r, base[0], base[1], base[2], base[3]);
-        const int L = sel4(r, len[0], len[1], len[2], len[3]);
-        const int S = sel4(r, off[0], off[1], off[2], off[3]);
-        const int64_t c0 =
-            (D & ~int64_t(R - 1)) + R * (int64_t)(c - sel4(r, cum[0], cum[1], cum[2], cum[3]));
-        cdst[q] = c0;
+      for (int g = 0; g < R / 4; ++g) {
+        uint4 r;
+        transpose4(cur[0].w[g], cur[1].w[g], cur[2].w[g], cur[3].w[g], r.x, r.y, r.z, r.w);
+        *reinterpret_cast<uint4 *>(&rows4[b][R * tid + 4 * g]) = r;
+      }
+      load(f0 + kQuad);
+      __syncthreads();
+      const int nf = min(kQuad, F_sel - f0);
+      uint8_t *dst = codes_dst + (int64_t)f0 * ld_c;
+#pragma unroll
+      for (int q = 0; q < kSlots; ++q) {
+        if (tid + q * kPartBlock >= n_chunks) continue;
+        uint32_t sv[kChunkRows], sw[kChunkRows], o[kQuad];
         bool full = true;
 #pragma unroll
-        for (int k = 0; k < R; k += 2) {
-          uint32_t pairv = 0u;
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int64_t dr = c0 + k + h;
-            const bool in = cown[q] && dr >= D && dr < D + L;
-            full = full && in;
-            const uint32_t src = in ? (uint32_t)inv[S + (int)(dr - D)] : 0xffffu;
-            pairv |= src << (16 * h);
-          }
-          csrc[q][k >> 1] = pairv;
+        for (int k = 0; k < kChunkRows; ++k) {
+          sv[k] = (csrc[q][k >> 1] >> (16 * (k & 1))) & 0xffffu;
+          full = full && sv[k] != 0xffffu;
+          sw[k] = rows4[b][sv[k] < (uint32_t)kTile ? sv[k] : 0u];
         }
-        cfull[q] = full;
-      }
-      // Four features per batch, as one word of four codes per tile row,
-      // double buffered in LDS (one barrier per batch, the next batch's
-      // loads in flight meanwhile), then the owned chunks gathered and stored.
-      CodeWords<R> cur[kQuad];
-#pragma unroll
-      for (int u = 0; u < kQuad; ++u) {
-        if (f_first + u < F_sel) {
-          cur[u] = load_codes<R>(codes_src + (int64_t)(f_first + u) * ld_c, row, lo, hi);
-        } else {
-#pragma unroll
-          for (int k = 0; k < R / 4; ++k) cur[u].w[k] = 0u;
-        }
-      }
-      for (int f0 = f_first, b = 0; f0 < F_sel; f0 += kQuad, b ^= 1) {
-#pragma unroll
-        for (int g = 0; g < R / 4; ++g) {
-          uint4 r;
-          transpose4(cur[0].w[g], cur[1].w[g], cur[2].w[g], cur[3].w[g], r.x, r.y, r.z, r.w);
-          *reinterpret_cast<uint4 *>(&rows4[b][R * tid + 4 * g]) = r;
-        }
+        transpose4(sw[0], sw[1], sw[2], sw[3], o[0], o[1], o[2], o[3]);
 #pragma unroll
         for (int u = 0; u < kQuad; ++u) {
-          if (f0 + kQuad + u < F_sel) {
-            cur[u] = load_codes<R>(codes_src + (int64_t)(f0 + kQuad + u) * ld_c, row, lo, hi);
+          if (u >= nf) break;
+          uint8_t *dcol = dst + (int64_t)u * ld_c + cdst[q];
+          if (full) {
+            *reinterpret_cast<uint32_t *>(dcol) = o[u];
           } else {
 #pragma unroll
-            for (int k = 0; k < R / 4; ++k) cur[u].w[k] = 0u;
-          }
-        }
-        __syncthreads();
-        const int nf = min(kQuad, F_sel - f0);
-#pragma unroll
-        for (int q = 0; q < kChunkSlots; ++q) {
-          if (!cown[q]) continue;
-          CodeWords<R> o[kQuad];
-#pragma unroll
-          for (int g = 0; g < R / 4; ++g) {
-            uint32_t sw[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const uint32_t sv = (csrc[q][(4 * g + j) >> 1] >> (16 * ((4 * g + j) & 1))) & 0xffffu;
-              sw[j] = rows4[b][sv < (uint32_t)kTile ? sv : 0u];
-            }
-            transpose4(sw[0], sw[1], sw[2], sw[3], o[0].w[g], o[1].w[g], o[2].w[g], o[3].w[g]);
-          }
-#pragma unroll
-          for (int u = 0; u < kQuad; ++u) {
-            if (u >= nf) break;
-            uint8_t *dcol = codes_dst + (int64_t)(f0 + u) * ld_c;
-            if (cfull[q]) {
-              *reinterpret_cast<typename CodesR<R>::T *>(dcol + cdst[q]) = o[u].v;
-            } else {
-#pragma unroll
-              for (int k = 0; k < R; ++k) {
-                const uint32_t sv = (csrc[q][k >> 1] >> (16 * (k & 1))) & 0xffffu;
-                if (sv != 0xffffu) dcol[cdst[q] + k] = (uint8_t)(o[u].w[k >> 2] >> (8 * (k & 3)));
-              }
-            }
+            for (int k = 0; k < kChunkRows; ++k)
+              if (sv[k] != 0xffffu) dcol[k] = (uint8_t)(o[u] >> (8 * k));
           }
         }
       }
@@ -1921,16 +1842,14 @@ hipError_t launch_part_scatter(hipStream_t st, const uint8_t *codes_src,
   // (Whole batches of four features per part.)
   const int32_t f_part = (F_sel + 4 * parts - 1) / (4 * parts) * 4;
   const unsigned n_parts = (unsigned)std::max(1, (F_sel + f_part - 1) / f_part);
-#define BSSCL_SCATTER(R, Q)                                                                   \
-  hipLaunchKernelGGL((k_part_scatter<R, Q>), dim3((unsigned)max_tiles, n_parts), dim3(kPartBlock), 0, st, \
-                     codes_src, codes_dst, ld_c, gh_src, gh_dst, rid_src, rid_dst, parents,      \
-                     groups, tiles, plan, tile_begin, tile_cnt, parent_nleft, segs,            \
-                     hist_node,                                                                \
+#define BSSCL_SCATTER(R)                                                                         \
+  hipLaunchKernelGGL(k_part_scatter<R>, dim3((unsigned)max_tiles, n_parts), dim3(kPartBlock), 0, \
+                     st, codes_src, codes_dst, ld_c, gh_src, gh_dst, rid_src, rid_dst, parents,  \
+                     groups, tiles, plan, tile_begin, tile_cnt, parent_nleft, segs, hist_node,   \
                      min_samples_leaf, F_sel, f_part)
   switch (part_rows) {
-    case 4: BSSCL_SCATTER(4, ScatterQ<4>::value); break;
-    case 8: BSSCL_SCATTER(8, ScatterQ<8>::value); break;
-    case 16: BSSCL_SCATTER(16, ScatterQ<16>::value); break;
+    case 4: BSSCL_SCATTER(4); break;
+    case 8: BSSCL_SCATTER(8); break;
     default: return hipErrorInvalidValue;
   }
 #undef BSSCL_SCATTER
@@ -2751,7 +2670,7 @@ __device__ void plan_count_role(const uint8_t *__restrict__ codes_c, int64_t ld_
       const Route<R> rt = route_load<R>(codes_c, ld_c, T, G, Pa, Pb, row);
       route_masks<R>(rt, G, row, run);
     }
-    // Four counts as 16-bit fields (a tile has at most 4096 rows).
+    // Four counts as 16-bit fields (a tile has at most 2048 rows).
     const uint32_t ca = wave_sum((uint32_t)__builtin_popcount(run[0]) |
                                  ((uint32_t)__builtin_popcount(run[1]) << 16));
     const uint32_t cb = wave_sum((uint32_t)__builtin_popcount(run[2]) |
@@ -2817,20 +2736,12 @@ __global__ __launch_bounds__(kPlanBlock) void k_plan_lds(
     const int32_t c_nc = a.level == 0 ? 1 : level_in[1];
     if (a.fused_count && c_nc > 0 && c_nc <= kPlanLdsC) {
       const bool g = a.mode == kLevelGrouped;
-      switch (a.part_rows) {
-        case 4:
-          plan_count_role<4>(codes_c, ld_c, segs, cand, F_sel, prev_parents, c_first, c_nc, g, a,
-                             tile_cnt, stmp, s_ctb, s_cbest, s_cred);
-          break;
-        case 8:
-          plan_count_role<8>(codes_c, ld_c, segs, cand, F_sel, prev_parents, c_first, c_nc, g, a,
-                             tile_cnt, stmp, s_ctb, s_cbest, s_cred);
-          break;
-        default:
-          plan_count_role<16>(codes_c, ld_c, segs, cand, F_sel, prev_parents, c_first, c_nc, g,
-                              a, tile_cnt, stmp, s_ctb, s_cbest, s_cred);
-          break;
-      }
+      if (a.part_rows == 4)
+        plan_count_role<4>(codes_c, ld_c, segs, cand, F_sel, prev_parents, c_first, c_nc, g, a,
+                           tile_cnt, stmp, s_ctb, s_cbest, s_cred);
+      else
+        plan_count_role<8>(codes_c, ld_c, segs, cand, F_sel, prev_parents, c_first, c_nc, g, a,
+                           tile_cnt, stmp, s_ctb, s_cbest, s_cred);
     }
     return;
   }
@@ -3518,7 +3429,7 @@ hipError_t launch_plan_lds(hipStream_t st, NodeOut *nodes, LevelPlan *plan,
                            PlanArgs a, const uint8_t *codes_c, int64_t ld_c,
                            int32_t *tile_cnt, const int32_t *level_in, int32_t *level_out,
                            int32_t count_blocks) {
-  if (a.fused_count && (a.part_rows != 4 && a.part_rows != 8 && a.part_rows != 16))
+  if (a.fused_count && a.part_rows != 4 && a.part_rows != 8)
     return hipErrorInvalidValue;
   const unsigned grid = 1u + (a.fused_count ? (unsigned)std::max(1, count_blocks) : 0u);
   hipLaunchKernelGGL(k_plan_lds, dim3(grid), dim3(kPlanBlock), 0, st, nodes, plan, prev_parents,

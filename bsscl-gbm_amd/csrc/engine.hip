@@ -1450,7 +1450,11 @@ void read_hist_tuning(bsscl_engine *E, int64_t m, int32_t F_sel) {
   // The root: at least 10240 rows per tile (1M x 28, 73 tiles and half the
   // partials of 5120-row tiles: 2440 -> 2480 trees/s; at 10M x 50 the block
   // target decides, 227 tiles either way).
-  E->hist_rows_per_flush = env_int("BSSCL_HIST_ROWS_PER_FLUSH", 256, 1 << 22, 10240);
+  // Up to 256k rows such tiles leave the root too few blocks: 2560 there
+  // (the smallest tile, 4096 rows, is then the line; 100,000 x 100, 300
+  // rounds 73.9 -> 73.1 ms, 285k x 30 with validation 36.2 -> 35.5).
+  E->hist_rows_per_flush =
+      env_int("BSSCL_HIST_ROWS_PER_FLUSH", 256, 1 << 22, m <= (1 << 18) ? 2560 : 10240);
   // Below the root, smaller tiles (more blocks for the smaller levels, more
   // partials to sum): 1M x 28, 2560 rows took the five planned levels'
   // histograms and reductions from 120 to 114 us per round.

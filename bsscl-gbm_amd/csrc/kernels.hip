@@ -3587,7 +3587,10 @@ __global__ __launch_bounds__(kUpdBlock) void k_update_F(
 #pragma unroll
       for (int r = 0; r < kUpdRows; ++r)
         if (in[r]) {
-          f[r] = __dadd_rn(f[r], __dmul_rn(lr, nd[r].value));
+          // (Plain operators: the pragma keeps them apart, while an inlined
+          // __dadd_rn of a __dmul_rn is contracted to one fma.)
+          const double v = lr * nd[r].value;
+          f[r] = f[r] + v;
           F[i[r]] = f[r];
         }
     }
@@ -4347,8 +4350,7 @@ __global__ __launch_bounds__(256) void k_predict(
   double F = 0.0;
   for (int32_t t = 0; t < n_trees; ++t) {
     const TreeNodeDev *tree = nodes + offsets[t];
-    // (Plain operators: the pragma keeps them apart, while an inlined
-    // __dadd_rn of a __dmul_rn is contracted to one fma.)
+    // (Rounded apart as in k_update_F.)
     const double v = lr * tree[traverse(tree, codes, ld, i)].value;
     F = F + v;
   }
@@ -4533,7 +4535,9 @@ __global__ __launch_bounds__(256) void k_mc_apply(const uint8_t *__restrict__ co
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   // A device replay that failed left node_count at 0: F stays as it is.
   if (i >= n || (node_count_d && *node_count_d <= 0)) return;
-  Fk[i] = __dadd_rn(Fk[i], __dmul_rn(lr, tree[traverse(tree, codes, ld, i)].value));
+  // (Rounded apart as in k_update_F.)
+  const double v = lr * tree[traverse(tree, codes, ld, i)].value;
+  Fk[i] = Fk[i] + v;
 }
 
 // Per block: the sum of log(clip(softmax(F_i))[y_i], 1e-15, 1 - 1e-15)

@@ -313,6 +313,7 @@ constexpr int kMcLanesMax = 2;
 constexpr int kXferPins = 6;
 constexpr int kOutPins = 3;
 constexpr size_t kOutPinBytes = 16u << 20;
+constexpr size_t kOneChunkBytes = 16u << 20;  // host rows that predict_rows takes at once
 }  // namespace
 
 // What the enqueued work of one tree writes, and its stream.  A multiclass
@@ -3534,11 +3535,16 @@ int predict_to_device(bsscl_engine *E, int32_t slot, const int16_t *features,
 // stream bins, walks and reads back chunk c - 1 and the host copies chunk
 // c - 2's probabilities out.  The upload sets the rate (57 GB/s here), so a
 // chunk only has to be short enough that the last one's tail is short, and
-// long enough to fill the chip: an eighth of X between 8 and 64 MB.  Up to
-// 16 MB go as one chunk.  1M x 28 float32, 100 trees: 3.6 ms in one chunk,
-// 2.65 so (2.12 of them the upload); 10M x 50, 500 trees: 44.0 ms in 256 MB
-// chunks read back at the end, 39.2 so.  (More copy threads, or a thread for
-// the results alone, change neither.)
+// long enough to fill the chip: an eighth of X between 8 and 64 MB, rounded
+// up to whole 1,024 rows so that eight chunks are not nine.  1M x 28 float32,
+// 100 trees: 3.6 ms in one chunk, 2.6 so (2.12 of them the upload); 10M x 50,
+// 500 trees: 44.0 ms in 256 MB chunks read back at the end, 39.2 so.  (More
+// copy threads, or a thread for the results alone, change neither, and chunks
+// evened out, whose last one is longer, make 10M x 50 2-3% slower.)  Up to
+// 16 MB go as one chunk, whatever their row count: a tail of some hundred
+// rows behind so short an upload costs every launch and event again (1,500 x
+// 28 in 1,024 + 476 rows 0.19 ms, in one chunk 0.12; 10,000 x 20, 10 trees
+// 0.42 and 0.14).
 int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, int32_t F,
                  const double *edges_2d, int32_t edge_stride, const int32_t *bin_counts,
                  const int32_t *nan_bin_id, const PackedTrees &P, double lr, double base_score,
@@ -3549,16 +3555,23 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
   HIPCHK(hipSetDevice(E->device));
   const size_t row_b = (size_t)F * (x_is_f64 ? 8 : 4), total_b = row_b * (size_t)n;
   const size_t out_w = P.K > 1 ? (size_t)P.K : 2;  // doubles per row
-  size_t chunk_b = std::min<size_t>(std::max<size_t>(total_b / 8, 8u << 20), 64u << 20);
-  if (total_b <= (16u << 20)) chunk_b = total_b;
-  // (A chunk's probabilities fit a pinned buffer.)
-  int64_t rows_c = (int64_t)std::min(chunk_b / row_b, kOutPinBytes / (8 * out_w));
-  // (Test hook BSSCL_TEST_PREDICT_CHUNK_ROWS: another count.)
-  if (const char *t = std::getenv("BSSCL_TEST_PREDICT_CHUNK_ROWS"))
-    rows_c = std::min<int64_t>(std::strtoll(t, nullptr, 10), rows_c);
-  rows_c = std::min<int64_t>(std::max<int64_t>(1024, rows_c / 1024 * 1024), round_up(n, 1024));
-  if (rows_c >= n) rows_c = n;
-  const bool one_chunk = rows_c >= n;
+  // (A chunk's probabilities fit a pinned buffer.  Test hook
+  // BSSCL_TEST_PREDICT_CHUNK_ROWS: chunks of at most so many rows.)
+  int64_t rows_max = (int64_t)(kOutPinBytes / (8 * out_w)) / 1024 * 1024;
+  const char *hook = std::getenv("BSSCL_TEST_PREDICT_CHUNK_ROWS");
+  if (hook)
+    rows_max =
+        std::min(rows_max, std::max<int64_t>(1024, std::strtoll(hook, nullptr, 10) / 1024 * 1024));
+  int64_t rows_c = n;
+  if (total_b > kOneChunkBytes || n > rows_max) {
+    const size_t chunk_b = std::min<size_t>(std::max<size_t>(total_b / 8, 8u << 20), 64u << 20);
+    rows_c = round_up((int64_t)std::max<size_t>(1, chunk_b / row_b), 1024);
+    rows_c = std::min(n, std::min(rows_max, rows_c));
+  }
+  // A request of up to 1 MB goes through the arena on the engine's stream
+  // alone; from there on the rows stream carries X while the engine's takes
+  // the model up, in one chunk too (65,000 x 28: 0.34 ms, 0.36 behind X).
+  const bool small = rows_c >= n && total_b <= kXferSmall;
   // One chunk's codes, in the layout of a matrix of rows_c rows.
   Matrix view;
   view.n = rows_c;
@@ -3570,7 +3583,7 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
   CHK(E->proba_d.ensure(out_w * (size_t)rows_c));
   const size_t xbytes = (size_t)rows_c * row_b;
   CHK(E->xchunk.ensure(xbytes));
-  if (!one_chunk) CHK(E->xchunk2.ensure(xbytes));
+  if (rows_c < n) CHK(E->xchunk2.ensure(xbytes));
   CHK(ensure_out_pins(E, std::min(kOutPinBytes, out_w * 8 * (size_t)rows_c)));
   for (hipEvent_t &ev : E->pipe_ev)
     if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -3592,16 +3605,11 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
     const int b = (int)(c & 1);
     unsigned char *xb = b ? E->xchunk2.p : E->xchunk.p;
     const size_t xc = (size_t)rows * row_b;
-    if (one_chunk) {
-      // Nothing to overlap: through the arena when small, else as pieces.
+    if (small) {
       char *stage = nullptr;
-      if (xc <= (1u << 20)) {
-        CHK(take_pinned(E, xc, &stage));
-        std::memcpy(stage, xs, xc);
-        HIPCHK(hipMemcpyAsync(xb, stage, xc, hipMemcpyHostToDevice, E->st));
-      } else {
-        CHK(host_upload_async(E, E->st, xb, xs, xc));
-      }
+      CHK(take_pinned(E, xc, &stage));
+      std::memcpy(stage, xs, xc);
+      HIPCHK(hipMemcpyAsync(xb, stage, xc, hipMemcpyHostToDevice, E->st));
     } else {
       // (Its buffer is free once chunk c - 2 has been binned.)
       if (c >= 2) HIPCHK(hipStreamWaitEvent(E->st_rows, E->pipe_ev[2 + b], 0));
@@ -3612,10 +3620,10 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
       CHK(upload_ensemble(E, view, P, lr, rows_c, &en));
       CHK(upload_edges(E, F, edges_2d, edge_stride, bin_counts, nan_bin_id, &de));
     }
-    if (!one_chunk) HIPCHK(hipStreamWaitEvent(E->st, E->pipe_ev[b], 0));
+    if (!small) HIPCHK(hipStreamWaitEvent(E->st, E->pipe_ev[b], 0));
     HIPCHK(launch_bin(E->st, xb, x_is_f64, rows, F, de.edges, edge_stride, de.nb, de.nan_id,
                       has_any_nan, E->pcodes.p, view.ld, tiers, levels));
-    if (!one_chunk) HIPCHK(hipEventRecord(E->pipe_ev[2 + b], E->st));
+    if (!small) HIPCHK(hipEventRecord(E->pipe_ev[2 + b], E->st));
     if (P.K == 1) {
       CHK(run_ensemble(E, en, E->pcodes.p, view.ld, rows, E->out_d.p, rows_c, E->proba_d.p,
                        base_score));

@@ -933,9 +933,27 @@ int next_piece(bsscl_engine *E, char **pin, hipEvent_t *ev) {
   return BSSCL_OK;
 }
 
+// Waits for whatever the engine's streams still hold, on the error returns of
+// calls that use several of them: nothing then lands in, or reads from, a
+// buffer after the call.
+void drain_streams(bsscl_engine *E) {
+  for (hipStream_t s : {E->st_rows, E->st_xfer, E->st})
+    if (s) (void)hipStreamSynchronize(s);
+}
+
+// Drains them unless `ok` was set.
+struct DrainOnError {
+  bsscl_engine *e;
+  bool ok = false;
+  ~DrainOnError() {
+    if (!ok) drain_streams(e);
+  }
+};
+
 // Enqueues dst (device) = src (host, pageable) after the work already on
 // stream `st`, and returns once the last piece has been copied into its
-// pinned buffer; later work on `st` sees the whole copy.
+// pinned buffer; later work on `st` sees the whole copy.  (Test hook
+// BSSCL_TEST_UPLOAD_FAIL=k: an error after piece k.)
 int host_upload_async(bsscl_engine *E, hipStream_t st, void *dst, const void *src, size_t bytes) {
   if (bytes <= kXferSmall) {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
@@ -945,9 +963,11 @@ int host_upload_async(bsscl_engine *E, hipStream_t st, void *dst, const void *sr
   CopyPool &pool = CopyPool::get();
   HIPCHK(hipEventRecord(E->xfer_fork, st));
   HIPCHK(hipStreamWaitEvent(E->st_xfer, E->xfer_fork, 0));
+  const char *fail = std::getenv("BSSCL_TEST_UPLOAD_FAIL");
   const size_t piece = xfer_piece(bytes);
   hipEvent_t last = nullptr;
   bool second = false;
+  DrainOnError guard{E};  // (the pieces on st_xfer are not on `st` yet)
   for (size_t off = 0; off < bytes; off += piece, second = !second) {
     const size_t len = std::min(piece, bytes - off);
     char *pin;
@@ -958,8 +978,11 @@ int host_upload_async(bsscl_engine *E, hipStream_t st, void *dst, const void *sr
     HIPCHK(hipMemcpyAsync(static_cast<char *>(dst) + off, pin, len, hipMemcpyHostToDevice, on));
     HIPCHK(hipEventRecord(ev, on));
     if (second) last = ev;
+    if (fail && off / piece == std::strtoull(fail, nullptr, 10))
+      return set_error(BSSCL_EDEVICE, "host upload: BSSCL_TEST_UPLOAD_FAIL");
   }
   if (last) HIPCHK(hipStreamWaitEvent(st, last, 0));
+  guard.ok = true;
   return BSSCL_OK;
 }
 
@@ -987,6 +1010,7 @@ int host_download(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
   const size_t n = (bytes + piece - 1) / piece;
   char *pin[kXferPins];
   hipEvent_t ev[kXferPins];
+  DrainOnError guard{E};
   auto enqueue = [&](size_t c) -> int {
     CHK(next_piece(E, &pin[c % kXferPins], &ev[c % kXferPins]));
     hipStream_t on = c & 1 ? E->st_xfer : E->st;
@@ -1004,6 +1028,7 @@ int host_download(bsscl_engine *E, void *dst, const void *src, size_t bytes) {
     pool.copy(static_cast<char *>(dst) + c * piece, pin[c % kXferPins],
               std::min(piece, bytes - c * piece));
   }
+  guard.ok = true;
   return BSSCL_OK;
 }
 
@@ -3644,9 +3669,8 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
   }
   for (int64_t c = std::max<int64_t>(0, n_chunks - 2); c < n_chunks && rc == BSSCL_OK; ++c)
     rc = finish(c);
-  if (rc != BSSCL_OK) {  // the buffers can be used again once both streams drain
-    (void)hipStreamSynchronize(E->st_rows);
-    (void)hipStreamSynchronize(E->st);
+  if (rc != BSSCL_OK) {
+    drain_streams(E);
     return rc;
   }
   // (The last chunk's event followed everything on both streams: they need

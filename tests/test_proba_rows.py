@@ -81,3 +81,19 @@ def test_multiclass_chunks_equal_the_whole_matrix(engine, monkeypatch, case):
     np.testing.assert_array_equal(got, want)
     assert launches == (1 if case == "one_chunk" else 6)
     np.testing.assert_array_equal(eng.get_codes(1, n, F), codes)
+
+
+@pytest.mark.parametrize("piece", [0, 1, 2])
+def test_failed_upload_leaves_nothing_behind(model, monkeypatch, piece):
+    """A call whose upload fails after some of its pieces, on either copy
+    stream, returns the error with its streams idle: the next call, whose
+    rows take the same buffers at once, gets its own probabilities."""
+    print(f"[case] upload fails after piece {piece}", flush=True)
+    rng = np.random.default_rng(3)
+    X = rng.standard_normal((300_001, 20)).astype(np.float32)
+    want = model.predict_proba(X)
+    monkeypatch.setenv("BSSCL_TEST_UPLOAD_FAIL", str(piece))
+    with pytest.raises(RuntimeError, match="BSSCL_TEST_UPLOAD_FAIL"):
+        model.predict_proba(-X)
+    monkeypatch.delenv("BSSCL_TEST_UPLOAD_FAIL")
+    np.testing.assert_array_equal(model.predict_proba(X), want)

@@ -259,13 +259,11 @@ namespace {
 constexpr int32_t kNoAllocMaxNodes = 1 << 17;   // nodes of all trees of a call
 constexpr int32_t kNoAllocMaxTrees = 1 << 14;
 constexpr int32_t kNoAllocMaxCols = 4096;       // columns the walk can renumber
-// What launch_walk_pack and launch_walk read beside the nodes, one class.
-struct WalkLists {
-  int32_t first[kNoAllocMaxTrees + 8], count[kNoAllocMaxTrees + 8];
-  int32_t class_slots[2];
-  int32_t cols[kWalkMaxCols + 1];
-  uint8_t remap[kNoAllocMaxCols];
-};
+// What launch_walk_pack and launch_walk read beside the nodes, one class: first
+// node and node count of every slot, the class's slots, the staged columns,
+// every column's index among them.
+constexpr size_t kNoAllocLists =
+    (2 * (kNoAllocMaxTrees + kWalkMaxTpl) + 2 + kWalkMaxCols) * 4 + kNoAllocMaxCols;
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t kScrNodes = 0;
 constexpr size_t kScrFeat = kScrNodes + align256(sizeof(TreeNodeDev) * kNoAllocMaxNodes);
@@ -275,7 +273,7 @@ constexpr size_t kScrLeft = kScrVal + align256(sizeof(double) * kNoAllocMaxNodes
 constexpr size_t kScrRight = kScrLeft + align256(sizeof(int32_t) * kNoAllocMaxNodes);
 constexpr size_t kScrOffs = kScrRight + align256(sizeof(int32_t) * kNoAllocMaxNodes);
 constexpr size_t kScrLists = kScrOffs + align256(sizeof(int32_t) * (kNoAllocMaxTrees + 1));
-constexpr size_t kScratchBytes = kScrLists + align256(sizeof(WalkLists));
+constexpr size_t kScratchBytes = kScrLists + align256(kNoAllocLists);
 // The packed arrays are dead once the traversal nodes are made: the walk's
 // values and words take their place.
 constexpr size_t kScrWalk = kScrFeat;
@@ -553,7 +551,6 @@ struct bsscl_engine {
   // An ensemble's nodes and lists (upload_ensemble), and its packed form for
   // the walk in LDS.
   TempBuf<char> ens_d;
-  std::vector<uint8_t> child_marks;  // host work space of its checks
   TempBuf<uint32_t> walk_words;
   TempBuf<double> walk_vals;
   DevBuf<double> partials_d, loss_d, out_d, proba_d;
@@ -3337,20 +3334,31 @@ int check_classes(const PackedTrees &P) {
 struct TreeShape {
   int32_t max_nodes = 1;
   bool proper = true;
-  std::vector<uint8_t> used;  // by engine column
-  int32_t n_used = 0;
-  void use(int32_t col) {
-    n_used += used[(size_t)col] ? 0 : 1;
-    used[(size_t)col] = 1;
+  uint8_t *used;  // by engine column, cleared
+  int32_t n_cols, n_used = 0;
+  uint8_t has_parent[kWalkMaxNodes];  // the current tree's nodes
+  TreeShape(uint8_t *used_cols, int32_t cols) : used(used_cols), n_cols(cols) {}
+  void tree(int32_t nodes) {
+    max_nodes = std::max(max_nodes, nodes);
+    std::memset(has_parent, 0, (size_t)std::min(nodes, kWalkMaxNodes));
+  }
+  // A split of the current tree (checked), on engine column col.
+  void split(int32_t left, int32_t right, int32_t col) {
+    if (max_nodes > kWalkMaxNodes) return;  // no walk in LDS
+    uint8_t &l = has_parent[left], &r = has_parent[right];
+    proper = proper && !l && !r && left != right;
+    l = r = 1;
+    n_used += used[col] ? 0 : 1;
+    used[col] = 1;
   }
   // The used columns in ascending order (at least one) and every column's
   // index among them.
   void columns(int32_t *cols, uint8_t *remap) const {
     int32_t k = 0;
     cols[0] = 0;
-    for (size_t c = 0; c < used.size(); ++c) {
+    for (int32_t c = 0; c < n_cols; ++c) {
       remap[c] = (uint8_t)k;
-      if (used[c]) cols[k++] = (int32_t)c;
+      if (used[c]) cols[k++] = c;
     }
   }
 };
@@ -3391,8 +3399,8 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   Ensemble &en = *out;
   en.K = P.K;
   en.lr = lr;
-  TreeShape sh;
-  sh.used.assign((size_t)M.cols(), 0);
+  std::vector<uint8_t> used((size_t)M.cols(), 0);
+  TreeShape sh(used.data(), M.cols());
   // Built in pinned memory and copied from there: nodes, tree offsets, then
   // the walk's lists (first node and node count of every slot, the classes'
   // slots, the staged columns, every column's index among them).
@@ -3406,8 +3414,6 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   CHK(take_pinned(E, bytes_max, &stage));
   TreeNodeDev *nodes = reinterpret_cast<TreeNodeDev *>(stage);
   int32_t *offs = reinterpret_cast<int32_t *>(stage + off_b);
-  std::vector<uint8_t> &child = E->child_marks;
-  child.assign(std::max<size_t>(total, 1), 0);
   en.first_tree.assign((size_t)P.K + 1, 0);
   size_t base = 0;   // class k's first node
   int32_t tree = 0;  // and tree
@@ -3419,7 +3425,7 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
     for (int32_t t = 0; t < nt; ++t) {
       const int32_t a = offsets[t], b = offsets[t + 1];
       offs[(size_t)tree++] = (int32_t)base + a;
-      sh.max_nodes = std::max(sh.max_nodes, b - a);
+      sh.tree(b - a);
       for (int32_t i = a; i < b; ++i) {
         TreeNodeDev d;
         d.value = P.values[k][i];
@@ -3429,15 +3435,12 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
           if (d.feature >= M.F || l < 0 || r < 0 || l >= b - a || r >= b - a || l <= i - a ||
               r <= i - a)
             return set_error(BSSCL_EINVAL, "predict: malformed tree " + std::to_string(t));
-          uint8_t &lc = child[base + (size_t)(a + l)], &rc = child[base + (size_t)(a + r)];
-          sh.proper = sh.proper && !lc && !rc && l != r;
-          lc = rc = 1;
           int64_t thr = P.thresholds[k][i];
           split_to_engine(M, d.feature, thr);
           d.threshold = (int32_t)std::max<int64_t>(-1, std::min<int64_t>(thr, 1 << 20));
           d.left = l;
           d.right = r;
-          sh.use(d.feature);
+          sh.split(l, r, d.feature);
         } else {
           d.feature = -1;
           d.threshold = 0;
@@ -4742,26 +4745,25 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
                                        " nodes exceed the fixed scratch (at most " +
                                        std::to_string(kNoAllocMaxNodes) + ")");
   // The same checks as bsscl_predict: every traversal stays in its tree.
-  TreeShape sh;
-  sh.used.assign((size_t)M.cols(), 0);
-  std::vector<uint8_t> child((size_t)std::max(total, 1), 0);
+  // (All work space is on the stack; a matrix of more columns than it holds is
+  // walked in HBM.)
+  uint8_t used[kNoAllocMaxCols] = {};
+  TreeShape sh(used, M.cols());
+  const bool few_cols = M.cols() <= kNoAllocMaxCols;
   for (int32_t t = 0; t < n_trees; ++t) {
     const int32_t a = offsets[t], b = offsets[t + 1];
     if (a < 0 || b <= a || b > total) return set_error(BSSCL_EINVAL, "predict_noalloc: bad offsets");
-    sh.max_nodes = std::max(sh.max_nodes, b - a);
+    sh.tree(b - a);
     for (int32_t i = a; i < b; ++i) {
       if (features[i] < 0) continue;
       const int32_t l = left[i], r = right[i];
       if (features[i] >= M.F || l < 0 || r < 0 || l >= b - a || r >= b - a || l <= i - a ||
           r <= i - a)
         return set_error(BSSCL_EINVAL, "predict_noalloc: malformed tree " + std::to_string(t));
-      uint8_t &lc = child[(size_t)(a + l)], &rc = child[(size_t)(a + r)];
-      sh.proper = sh.proper && !lc && !rc && l != r;
-      lc = rc = 1;
       int32_t col = features[i];
       int64_t thr = thresholds[i];
       split_to_engine(M, col, thr);
-      sh.use(col);
+      if (few_cols) sh.split(l, r, col);
     }
   }
   HIPCHK(hipSetDevice(E->device));
@@ -4792,27 +4794,36 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
                              reinterpret_cast<const int32_t *>(S + kScrRight), total,
                              M.F, M.tiers, nodes));
   }
-  // The walk in LDS where its lists and packed trees fit the scratch (host
-  // lists on the stack; the copy has finished when the call returns).
+  // The walk in LDS where its packed trees fit the scratch (host lists on the
+  // stack, the used part of them copied; the copy has finished when the call
+  // returns).
   WalkPlan plan;
-  if (n_trees > 0 && M.cols() <= kNoAllocMaxCols && plan_walk(sh, M.n, &plan) &&
+  if (n_trees > 0 && few_cols && plan_walk(sh, M.n, &plan) &&
       round_up(n_trees, plan.tpl) * plan.slot <= kNoAllocWalkSlots) {
-    WalkLists L;
+    alignas(8) unsigned char lists[kNoAllocLists];
     const int32_t n_slots = (int32_t)round_up(n_trees, plan.tpl);
+    int32_t *first = reinterpret_cast<int32_t *>(lists);
+    int32_t *count = first + n_slots, *slots = count + n_slots, *cols = slots + 2;
+    uint8_t *remap = reinterpret_cast<uint8_t *>(cols + plan.n_cols);
     for (int32_t t = 0; t < n_slots; ++t) {
-      L.first[t] = t < n_trees ? offsets[t] : 0;
-      L.count[t] = t < n_trees ? offsets[t + 1] - offsets[t] : 0;
+      first[t] = t < n_trees ? offsets[t] : 0;
+      count[t] = t < n_trees ? offsets[t + 1] - offsets[t] : 0;
     }
-    L.class_slots[0] = 0;
-    L.class_slots[1] = n_slots;
-    sh.columns(L.cols, L.remap);
-    WalkLists *D = reinterpret_cast<WalkLists *>(S + kScrLists);
+    slots[0] = 0;
+    slots[1] = n_slots;
+    sh.columns(cols, remap);
+    const size_t bytes = (size_t)(remap - lists) + (size_t)M.cols();
+    HIPCHK(hipMemcpyAsync(S + kScrLists, lists, bytes, hipMemcpyHostToDevice, E->st));
+    auto dev = [&](const void *host) {
+      return S + kScrLists + (static_cast<const unsigned char *>(host) - lists);
+    };
     double *vals = reinterpret_cast<double *>(S + kScrWalk);
     uint32_t *words = reinterpret_cast<uint32_t *>(vals + kNoAllocWalkSlots);
-    HIPCHK(hipMemcpyAsync(D, &L, sizeof(L), hipMemcpyHostToDevice, E->st));
-    HIPCHK(launch_walk_pack(E->st, nodes, D->first, D->count, n_slots, D->remap, learning_rate,
-                            plan, words, vals));
-    const WalkArgs a{M.codes.p, M.ld, M.n, D->cols, plan.n_cols, words, vals, D->class_slots,
+    HIPCHK(launch_walk_pack(E->st, nodes, reinterpret_cast<const int32_t *>(dev(first)),
+                            reinterpret_cast<const int32_t *>(dev(count)), n_slots, dev(remap),
+                            learning_rate, plan, words, vals));
+    const WalkArgs a{M.codes.p, M.ld, M.n, reinterpret_cast<const int32_t *>(dev(cols)),
+                     plan.n_cols, words, vals, reinterpret_cast<const int32_t *>(dev(slots)),
                      plan.slot, plan.per_group, out_F_dev, M.n, nullptr, 0.0};
     HIPCHK(launch_walk(E->st, plan, a, 1));
     HIPCHK(hipStreamSynchronize(E->st));

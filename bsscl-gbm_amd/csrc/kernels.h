@@ -496,8 +496,9 @@ __device__ __forceinline__ double2 binary_proba(double F, double base_score) {
 hipError_t launch_binary_proba(hipStream_t st, const double *F, int64_t n, double base,
                                double *out);
 
-// Ensemble prediction in LDS (walk.hip), for trees of at most 1023 nodes
-// that split on at most kWalkMaxCols distinct columns.
+// Ensemble prediction in LDS (walk.hip), for trees of at most kWalkMaxNodes
+// nodes that split on at most kWalkMaxCols distinct columns.
+constexpr int32_t kWalkMaxNodes = 1023;
 constexpr int32_t kWalkMaxCols = 208;  // 256 rows' codes and a group of trees: 64 KB of LDS
 // From kWalkRows4 rows of at most kWalkCols4 columns on (1,024 rows' codes
 // and a group of trees: 64 KB) a lane walks four rows, else one.

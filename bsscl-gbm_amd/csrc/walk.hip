@@ -44,6 +44,7 @@ namespace bsscl {
 namespace {
 
 constexpr int kGroupNodes = 1024;  // node slots staged at a time
+static_assert(kWalkMaxNodes == kGroupNodes - 1, "slot 1 of a tree holds no node");
 constexpr int kValsAt = kGroupNodes * 4;  // LDS byte offsets
 constexpr int kCodesAt = kValsAt + kGroupNodes * 8;
 
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_walk_split(WalkArgs a) {
 #pragma clang fp contract(on)
 
 bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
-  if (n_cols < 1 || n_cols > kWalkMaxCols || max_nodes >= kGroupNodes) return false;
+  if (n_cols < 1 || n_cols > kWalkMaxCols || max_nodes > kWalkMaxNodes) return false;
   WalkPlan &p = *plan;
   p.slot = 4;
   while (p.slot <= max_nodes) p.slot *= 2;  // (slot 1 holds no node)

@@ -98,3 +98,36 @@ def test_predict_noalloc_refuses(engine):
     host = np.zeros(64)
     with pytest.raises(ValueError, match="not device memory"):
         engine.predict_noalloc(1, _subset(packed, 2), 2, 0.1, host.ctypes.data)
+
+
+# (rows, columns, bins, splits per tree): the walk by one wave per row tile
+# and by four rows a lane, codes in two tiers, trees that need a large window,
+# and what the fixed scratch does not hold packed (walked in HBM): many small
+# trees beside one of 62 splits, more columns than the lists number.
+CASES = {
+    "65537_rows": (65_537, 20, 250, [62] * 30 + [3]),
+    "400000_rows": (400_000, 8, 250, [30] * 9),
+    "two_tiers": (70_001, 12, 400, [62, 9] * 6),
+    "large_trees": (3000, 12, 250, [300, 5, 511, 0]),
+    "leaves": (300, 3, 250, [0]),
+    "unpacked_small_trees": (2000, 12, 250, [62] + [1] * 16_383),
+    "many_columns": (300, 4200, 250, [62] * 5),
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_predict_noalloc_walks(engine, case):
+    from test_walk import _pack, _tree
+    n, F, bins, splits = CASES[case]
+    print(f"[case] predict_noalloc {case}: {n} x {F}, {len(splits)} trees", flush=True)
+    rng = np.random.default_rng(n)
+    codes = rng.integers(0, bins, (n, F)).astype(np.uint8 if bins < 256 else np.uint16)
+    p = _pack([_tree(rng, s, F, bins) for s in splits])
+    engine.load_codes(1, codes)
+    out = DeviceBuffer(n)
+    try:
+        engine.predict_noalloc(1, p, len(splits), 0.1, out.p.value)
+        got = out.read()
+    finally:
+        out.close()
+    np.testing.assert_array_equal(got, om.predict_all_trees(codes, p, len(splits), 0.1))

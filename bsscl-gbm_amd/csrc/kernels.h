@@ -526,7 +526,7 @@ hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int3
 struct WalkArgs {
   const uint8_t *codes;  // feature-major, ld a multiple of 256
   int64_t ld, n;
-  const int32_t *cols;  // the staged columns (null: 0 .. n_cols - 1)
+  const int32_t *cols;  // the staged columns, ascending
   int32_t n_cols;
   const uint32_t *words;  // launch_walk_pack's outputs, slot entries a tree
   const double *vals;

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64) void k_walk_pack(
           order[pair] = none ? nd.right : nd.left;
           order[pair + 1] = none ? nd.left : nd.right;
           const uint32_t thr = none ? 255u : (uint32_t)min(nd.threshold, 255);
-          const uint32_t col = remap ? (uint32_t)remap[nd.feature] : (uint32_t)nd.feature;
+          const uint32_t col = (uint32_t)remap[nd.feature];
           word = (thr << 24) | (col << win) | (base + 4u * (uint32_t)pair);
         }
         w[i] = word;
@@ -146,7 +146,7 @@ __global__ __launch_bounds__((1 << kTileLog2) / kRpl) void k_walk(WalkArgs a) {
   for (int k = tid; k < a.n_cols * (kTile / 16); k += kThreads) {
     const int c = k / (kTile / 16), ch = k % (kTile / 16);
     const int64_t r = row0 + 16 * ch;
-    const int64_t col = a.cols ? a.cols[c] : c;
+    const int64_t col = a.cols[c];
     if (r < a.ld)
       lds_put(kCodesAt + (c << kTileLog2) + 16 * ch,
               *reinterpret_cast<const Quad *>(a.codes + col * a.ld + r));
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_walk_split(WalkArgs a) {
   const int32_t cls = (int32_t)blockIdx.y;
   const int64_t row0 = (int64_t)blockIdx.x * 64;
   for (int k = (int)threadIdx.x; k < a.n_cols * 4; k += 64 * kSplitWaves) {
-    const int64_t col = a.cols ? a.cols[k >> 2] : k >> 2;
+    const int64_t col = a.cols[k >> 2];
     lds_put(kCodes + 16 * k,
             *reinterpret_cast<const Quad *>(a.codes + col * a.ld + row0 + 16 * (k & 3)));
   }

@@ -1038,7 +1038,6 @@ int bin_layout(int32_t F, const double *edges_2d, int32_t edge_stride, const int
   *tiers = 1;
   *has_any_nan = 0;
   int32_t most = 2;
-  bool ascend = true;
   for (int32_t j = 0; j < F; ++j) {
     if (bin_counts[j] < 1 || bin_counts[j] >= edge_stride)
       return set_error(BSSCL_EINVAL, "bin_features: bin_counts must be in [1, edge_stride)");
@@ -1048,14 +1047,17 @@ int bin_layout(int32_t F, const double *edges_2d, int32_t edge_stride, const int
     *tiers = std::max(*tiers, tiers_for_bins(bin_counts[j]));
     if (nan_bin_id[j] >= 0) *has_any_nan = 1;
     most = std::max(most, bin_counts[j]);
+  }
+  *levels = 0;
+  if (most > 1 << kBinMaxLevels) return BSSCL_OK;
+  for (int32_t j = 0; j < F; ++j) {
     const double *e = edges_2d + (size_t)j * edge_stride;
     bool up = true;
     for (int32_t k = 0; k < bin_counts[j]; ++k) up &= e[k] <= e[k + 1];
-    ascend = ascend && up;
+    if (!up) return BSSCL_OK;
   }
   *levels = 1;
-  while (*levels <= kBinMaxLevels && (1 << *levels) < most) ++*levels;
-  if (!ascend || *levels > kBinMaxLevels) *levels = 0;
+  while ((1 << *levels) < most) ++*levels;
   return BSSCL_OK;
 }
 

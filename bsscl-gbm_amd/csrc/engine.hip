@@ -632,7 +632,7 @@ struct bsscl_engine {
   size_t ktime_used = 0;                                   // words
   std::vector<std::pair<size_t, size_t>> ktime_launches;  // (first word, blocks)
   double wall_khz = 0.0;
-  double stats[21] = {0};
+  double stats[22] = {0};
 };
 
 namespace bsscl {
@@ -773,17 +773,20 @@ int upload(bsscl_engine *E, DevBuf<T> &dst, const T *src, size_t count) {
   return BSSCL_OK;
 }
 
-// `bytes` of the pinned arena for a copy on E->st, waiting for its earlier
-// copies when they leave no room.
+// `bytes` (at most kArenaPiece) of the pinned arena for a copy on E->st,
+// waiting for its earlier copies when they leave no room.  Larger ones go
+// through host_upload_async: pinned memory that follows the largest model or
+// table would stay with the engine (64 rows against 21 MB of edges: the first
+// call took 9 ms, 7 of them pinning 42 MB).
+constexpr size_t kArenaBytes = 16u << 20;  // as the tree builder's first call takes
+constexpr size_t kArenaPiece = kArenaBytes / 2;
 int take_pinned(bsscl_engine *E, size_t bytes, char **out) {
-  // (16 MB, as the tree builder's first call takes: growing it later would
-  // free and pin again, about 1 ms.)
-  const size_t want = std::max<size_t>(2 * bytes + 512, 16u << 20);
-  *out = bytes + 512 <= E->pin.cap ? E->pin.take<char>(bytes) : nullptr;
+  *out = E->pin.take<char>(bytes);
   if (*out) return BSSCL_OK;
   CHK(sync(E));
-  CHK(E->pin.reserve(std::max(E->pin.cap, want)));
+  CHK(E->pin.reserve(std::max(E->pin.cap, kArenaBytes)));
   *out = E->pin.take<char>(bytes);
+  if (!*out) return set_error(BSSCL_EINTERNAL, "pinned staging");
   return BSSCL_OK;
 }
 
@@ -1062,7 +1065,7 @@ int bin_layout(int32_t F, const double *edges_2d, int32_t edge_stride, const int
 }
 
 // A binning call's edges [F][edge_stride], bin counts and NaN bins on the
-// device (E->edges_d), in one copy from pinned memory on E->st.
+// device (E->edges_d), on E->st: small ones in one copy from pinned memory.
 struct DevEdges {
   const double *edges;
   const int32_t *nb, *nan_id;
@@ -1071,13 +1074,19 @@ struct DevEdges {
 int upload_edges(bsscl_engine *E, int32_t F, const double *edges_2d, int32_t edge_stride,
                  const int32_t *bin_counts, const int32_t *nan_bin_id, DevEdges *out) {
   const size_t eb = (size_t)F * edge_stride * 8, fb = (size_t)F * 4;
-  char *stage = nullptr;
-  CHK(take_pinned(E, eb + 2 * fb, &stage));
-  std::memcpy(stage, edges_2d, eb);
-  std::memcpy(stage + eb, bin_counts, fb);
-  std::memcpy(stage + eb + fb, nan_bin_id, fb);
   CHK(E->edges_d.ensure(eb + 2 * fb));
-  HIPCHK(hipMemcpyAsync(E->edges_d.p, stage, eb + 2 * fb, hipMemcpyHostToDevice, E->st));
+  if (eb + 2 * fb <= kArenaPiece) {
+    char *stage = nullptr;
+    CHK(take_pinned(E, eb + 2 * fb, &stage));
+    std::memcpy(stage, edges_2d, eb);
+    std::memcpy(stage + eb, bin_counts, fb);
+    std::memcpy(stage + eb + fb, nan_bin_id, fb);
+    HIPCHK(hipMemcpyAsync(E->edges_d.p, stage, eb + 2 * fb, hipMemcpyHostToDevice, E->st));
+  } else {
+    CHK(host_upload_async(E, E->st, E->edges_d.p, edges_2d, eb));
+    CHK(host_upload_async(E, E->st, E->edges_d.p + eb, bin_counts, fb));
+    CHK(host_upload_async(E, E->st, E->edges_d.p + eb + fb, nan_bin_id, fb));
+  }
   out->edges = reinterpret_cast<const double *>(E->edges_d.p);
   out->nb = reinterpret_cast<const int32_t *>(E->edges_d.p + eb);
   out->nan_id = out->nb + F;
@@ -3403,17 +3412,24 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   en.lr = lr;
   std::vector<uint8_t> used((size_t)M.cols(), 0);
   TreeShape sh(used.data(), M.cols());
-  // Built in pinned memory and copied from there: nodes, tree offsets, then
-  // the walk's lists (first node and node count of every slot, the classes'
-  // slots, the staged columns, every column's index among them).
+  // Built in pinned memory, a large one in its own, and copied from there:
+  // nodes, tree offsets, then the walk's lists (first node and node count of
+  // every slot, the classes' slots, the staged columns, every column's index
+  // among them).
   const size_t off_b = std::max<size_t>(total, 1) * sizeof(TreeNodeDev);
   const size_t list_b = off_b + (trees + 1) * 4;
   const size_t slots_max = trees + (size_t)P.K * (kWalkMaxGroup + kWalkMaxTpl);
   const size_t cols_max = (size_t)M.cols();
   const size_t bytes_max =
       list_b + (2 * slots_max + 2 * (size_t)P.K + cols_max + 1) * 4 + cols_max;
+  std::vector<char> large;
   char *stage = nullptr;
-  CHK(take_pinned(E, bytes_max, &stage));
+  if (bytes_max <= kArenaPiece) {
+    CHK(take_pinned(E, bytes_max, &stage));
+  } else {
+    large.resize(bytes_max);
+    stage = large.data();
+  }
   TreeNodeDev *nodes = reinterpret_cast<TreeNodeDev *>(stage);
   int32_t *offs = reinterpret_cast<int32_t *>(stage + off_b);
   en.first_tree.assign((size_t)P.K + 1, 0);
@@ -3489,7 +3505,10 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
     sh.columns(cols, remap);
   }
   CHK(E->ens_d.ensure(bytes));
-  HIPCHK(hipMemcpyAsync(E->ens_d.p, stage, bytes, hipMemcpyHostToDevice, E->st));
+  if (large.empty())
+    HIPCHK(hipMemcpyAsync(E->ens_d.p, stage, bytes, hipMemcpyHostToDevice, E->st));
+  else
+    CHK(host_upload(E, E->ens_d.p, stage, bytes));
   auto dev = [&](const void *host) {
     return E->ens_d.p + (static_cast<const char *>(host) - stage);
   };
@@ -5032,7 +5051,8 @@ int bsscl_engine_stats(bsscl_engine *E, double *out, int32_t cap, int32_t *n_out
     HIPCHK(hipStreamSynchronize(E->st));
     CHK(prof_slots_collect(E));
   }
-  const int32_t n = std::min<int32_t>(cap, 21);
+  E->stats[21] = (double)E->pin.cap;
+  const int32_t n = std::min<int32_t>(cap, 22);
   for (int32_t i = 0; i < n; ++i) out[i] = E->stats[i];
   *n_out = n;
   return BSSCL_OK;

@@ -452,6 +452,7 @@ void bsscl_sampler_destroy(bsscl_sampler *s);
  *        root gather) ran as a captured HIP graph
  *   [19] boosting rounds whose tree kernels ran as a captured HIP graph
  *   [20] graphs captured
+ *   [21] bytes of pinned staging memory the engine holds for small uploads
  * and returns the number written in *n_out.  A histogram launch's time runs
  * from its first block's start to its last block's end, stamped by the
  * kernel on the device's constant-rate clock; prediction times come from

@@ -100,3 +100,27 @@ def test_walk_shared_child_takes_general_path(engine):
     engine.load_codes(1, codes)
     np.testing.assert_array_equal(engine.predict(1, 500, p, 1, 0.5),
                                   om.predict_all_trees(codes, p, 1, 0.5))
+
+
+def test_large_models_and_edges_pin_no_more(engine):
+    """Host tables of any size leave the engine's pinned staging memory at
+    its 16 MB, and give the same codes and sums."""
+    from bsscl_gbm import _native
+    rng = np.random.default_rng(8)
+    n, F, nb, T = 500, 40, 60_000, 15_000
+    eng = _native.Engine(0)
+    try:
+        E = np.sort(rng.standard_normal((F, nb + 1)), axis=1)  # 19 MB
+        X = rng.standard_normal((n, F)).astype(np.float32)
+        counts, nan_id = np.full(F, nb, np.int32), np.full(F, -1, np.int32)
+        eng.bin_features(1, X, E, counts, nan_id)
+        want = om.bin_features(X, E, counts, nan_id, "standard")
+        np.testing.assert_array_equal(eng.get_codes(1, n, F, u16=True), want)
+        codes = rng.integers(0, 200, (n, F)).astype(np.uint8)
+        p = _pack([_tree(rng, 14, F, 200) for _ in range(T)])  # 435,000 nodes, 14 MB
+        eng.load_codes(1, codes)
+        np.testing.assert_array_equal(eng.predict(1, n, p, T, 0.1),
+                                      om.predict_all_trees(codes, p, T, 0.1))
+        assert eng.stats()["staging_bytes"] <= 16 << 20
+    finally:
+        eng.close()

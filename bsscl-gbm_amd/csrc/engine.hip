@@ -260,10 +260,10 @@ constexpr int32_t kNoAllocMaxNodes = 1 << 17;   // nodes of all trees of a call
 constexpr int32_t kNoAllocMaxTrees = 1 << 14;
 constexpr int32_t kNoAllocMaxCols = 4096;       // columns the walk can renumber
 // What launch_walk_pack and launch_walk read beside the nodes, one class: first
-// node and node count of every slot, the class's slots, the staged columns,
-// every column's index among them.
+// node and node count of every slot, the class's slots, the depth, the staged
+// columns, every column's index among them.
 constexpr size_t kNoAllocLists =
-    (2 * (kNoAllocMaxTrees + kWalkMaxTpl) + 2 + kWalkMaxCols) * 4 + kNoAllocMaxCols;
+    (2 * (kNoAllocMaxTrees + kWalkMaxTpl) + 3 + kWalkMaxCols) * 4 + kNoAllocMaxCols;
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t kScrNodes = 0;
 constexpr size_t kScrFeat = kScrNodes + align256(sizeof(TreeNodeDev) * kNoAllocMaxNodes);
@@ -3392,6 +3392,7 @@ struct Ensemble {
   const TreeNodeDev *nodes = nullptr;
   const int32_t *offsets = nullptr;
   const int32_t *cols = nullptr, *class_slots = nullptr;
+  int32_t *depth = nullptr;
 };
 
 // Checks the trees for matrices with M's features and tiers, uploads them
@@ -3414,14 +3415,14 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   TreeShape sh(used.data(), M.cols());
   // Built in pinned memory, a large one in its own, and copied from there:
   // nodes, tree offsets, then the walk's lists (first node and node count of
-  // every slot, the classes' slots, the staged columns, every column's index
-  // among them).
+  // every slot, the classes' slots, the depth, the staged columns, every
+  // column's index among them).
   const size_t off_b = std::max<size_t>(total, 1) * sizeof(TreeNodeDev);
   const size_t list_b = off_b + (trees + 1) * 4;
   const size_t slots_max = trees + (size_t)P.K * (kWalkMaxGroup + kWalkMaxTpl);
   const size_t cols_max = (size_t)M.cols();
   const size_t bytes_max =
-      list_b + (2 * slots_max + 2 * (size_t)P.K + cols_max + 1) * 4 + cols_max;
+      list_b + (2 * slots_max + 2 * (size_t)P.K + 1 + cols_max + 1) * 4 + cols_max;
   std::vector<char> large;
   char *stage = nullptr;
   if (bytes_max <= kArenaPiece) {
@@ -3486,7 +3487,8 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
                                      P.n_trees[k], p.tpl);
     count = first + n_slots;
     slots = count + n_slots;
-    cols = slots + 2 * (size_t)P.K;
+    slots[2 * (size_t)P.K] = 0;  // the depth that packing finds
+    cols = slots + 2 * (size_t)P.K + 1;
     remap = reinterpret_cast<uint8_t *>(cols + std::max(1, sh.n_used));
     bytes = (size_t)(reinterpret_cast<char *>(remap) - stage) + cols_max;
     std::memset(first, 0, 2 * n_slots * 4);
@@ -3516,13 +3518,14 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   en.offsets = reinterpret_cast<const int32_t *>(dev(offs));
   if (!en.walk) return BSSCL_OK;
   en.class_slots = reinterpret_cast<const int32_t *>(dev(slots));
+  en.depth = reinterpret_cast<int32_t *>(dev(slots + 2 * (size_t)P.K));
   en.cols = reinterpret_cast<const int32_t *>(dev(cols));
   CHK(E->walk_words.ensure(n_slots * (size_t)en.plan.slot));
   CHK(E->walk_vals.ensure(n_slots * (size_t)en.plan.slot));
   HIPCHK(launch_walk_pack(E->st, en.nodes, reinterpret_cast<const int32_t *>(dev(first)),
                           reinterpret_cast<const int32_t *>(dev(count)), (int32_t)n_slots,
                           reinterpret_cast<const uint8_t *>(dev(remap)), lr, en.plan,
-                          E->walk_words.p, E->walk_vals.p));
+                          E->walk_words.p, E->walk_vals.p, en.depth));
   return BSSCL_OK;
 }
 
@@ -3536,7 +3539,7 @@ int run_ensemble(bsscl_engine *E, const Ensemble &en, const uint8_t *codes, int6
   if (en.walk) {
     CHK(prof_kernel(E, 4, &start, &stop));
     WalkArgs a{codes,        ld,         n,          en.cols,
-               en.plan.n_cols, E->walk_words.p, E->walk_vals.p, en.class_slots,
+               en.plan.n_cols, E->walk_words.p, E->walk_vals.p, en.class_slots, en.depth,
                en.plan.slot, en.plan.per_group, out, out_stride,
                reinterpret_cast<double2 *>(proba), base_score};
     HIPCHK(launch_walk(E->st, en.plan, a, en.K, start, stop));
@@ -4824,7 +4827,8 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
     alignas(8) unsigned char lists[kNoAllocLists];
     const int32_t n_slots = (int32_t)round_up(n_trees, plan.tpl);
     int32_t *first = reinterpret_cast<int32_t *>(lists);
-    int32_t *count = first + n_slots, *slots = count + n_slots, *cols = slots + 2;
+    int32_t *count = first + n_slots, *slots = count + n_slots, *depth = slots + 2;
+    int32_t *cols = depth + 1;
     uint8_t *remap = reinterpret_cast<uint8_t *>(cols + plan.n_cols);
     for (int32_t t = 0; t < n_slots; ++t) {
       first[t] = t < n_trees ? offsets[t] : 0;
@@ -4832,6 +4836,7 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
     }
     slots[0] = 0;
     slots[1] = n_slots;
+    *depth = 0;
     sh.columns(cols, remap);
     const size_t bytes = (size_t)(remap - lists) + (size_t)M.cols();
     HIPCHK(hipMemcpyAsync(S + kScrLists, lists, bytes, hipMemcpyHostToDevice, E->st));
@@ -4842,10 +4847,11 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
     uint32_t *words = reinterpret_cast<uint32_t *>(vals + kNoAllocWalkSlots);
     HIPCHK(launch_walk_pack(E->st, nodes, reinterpret_cast<const int32_t *>(dev(first)),
                             reinterpret_cast<const int32_t *>(dev(count)), n_slots, dev(remap),
-                            learning_rate, plan, words, vals));
+                            learning_rate, plan, words, vals,
+                            reinterpret_cast<int32_t *>(dev(depth))));
     const WalkArgs a{M.codes.p, M.ld, M.n, reinterpret_cast<const int32_t *>(dev(cols)),
                      plan.n_cols, words, vals, reinterpret_cast<const int32_t *>(dev(slots)),
-                     plan.slot, plan.per_group, out_F_dev, M.n, nullptr, 0.0};
+                     reinterpret_cast<const int32_t *>(dev(depth)), plan.slot, plan.per_group, out_F_dev, M.n, nullptr, 0.0};
     HIPCHK(launch_walk(E->st, plan, a, 1));
     HIPCHK(hipStreamSynchronize(E->st));
     return BSSCL_OK;

@@ -520,9 +520,11 @@ struct WalkPlan {
 // from a multiple of per_group on, their count rounded up to a multiple of
 // tpl (the rest of them with count 0 in launch_walk_pack).
 bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan);
+// Raises *depth to the levels of splits of the deepest tree, where they matter.
 hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int32_t *first,
                             const int32_t *count, int32_t n_slots, const uint8_t *remap,
-                            double lr, const WalkPlan &p, uint32_t *words, double *vals);
+                            double lr, const WalkPlan &p, uint32_t *words, double *vals,
+                            int32_t *depth);
 struct WalkArgs {
   const uint8_t *codes;  // feature-major, ld a multiple of 256
   int64_t ld, n;
@@ -531,6 +533,7 @@ struct WalkArgs {
   const uint32_t *words;  // launch_walk_pack's outputs, slot entries a tree
   const double *vals;
   const int32_t *class_slots;  // class k has slots [class_slots[2k], class_slots[2k + 1])
+  const int32_t *depth;        // launch_walk_pack's
   int32_t slot, per_group;
   double *out;  // F of class k at out + k * out_stride
   int64_t out_stride;

@@ -124,3 +124,24 @@ def test_large_models_and_edges_pin_no_more(engine):
         assert eng.stats()["staging_bytes"] <= 16 << 20
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("n", [300, 70_001, 400_003])
+@pytest.mark.parametrize("splits", [9, 20, 21, 62, 130, 300, 511])
+@pytest.mark.parametrize("stay", [0.5, 0.97])
+def test_walk_of_chains(engine, n, splits, stay):
+    """Trees deep on one side: walks that end early and walks that go to the
+    bottom, in every launch shape, on both sides of the steps a wave takes
+    before it looks for the end."""
+    print(f"[case] walk of chains: {n} rows, {splits} splits, {stay}", flush=True)
+    rng = np.random.default_rng(splits)
+    codes = rng.integers(0, 200, (n, 9)).astype(np.uint8)
+    trees = []
+    for k in range(5):
+        f, t, v, l, r = _tree(rng, splits if k % 2 == 0 else 5, 9, 200, skew=True)
+        t[f >= 0] = int(200 * (1 - stay)) - 1  # the deeper side is the right one
+        trees.append((f, t, v, l, r))
+    p = _pack(trees)
+    engine.load_codes(1, codes)
+    np.testing.assert_array_equal(engine.predict(1, n, p, 5, 0.1),
+                                  om.predict_all_trees(codes, p, 5, 0.1))

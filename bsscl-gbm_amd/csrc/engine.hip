@@ -259,11 +259,10 @@ namespace {
 constexpr int32_t kNoAllocMaxNodes = 1 << 17;   // nodes of all trees of a call
 constexpr int32_t kNoAllocMaxTrees = 1 << 14;
 constexpr int32_t kNoAllocMaxCols = 4096;       // columns the walk can renumber
-// What launch_walk_pack and launch_walk read beside the nodes, one class: first
-// node and node count of every slot, the class's slots, the depth, the staged
-// columns, every column's index among them.
+// What the walk's lists of one class take (walk_lists_bytes).
 constexpr size_t kNoAllocLists =
-    (2 * (kNoAllocMaxTrees + kWalkMaxTpl) + 3 + kWalkMaxCols) * 4 + kNoAllocMaxCols;
+    (4 * kNoAllocMaxTrees + 3 * (kWalkMaxGroup + kWalkMaxTpl) + 4 + kWalkMaxCols) * 4 +
+    kNoAllocMaxCols;
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t kScrNodes = 0;
 constexpr size_t kScrFeat = kScrNodes + align256(sizeof(TreeNodeDev) * kNoAllocMaxNodes);
@@ -3391,9 +3390,93 @@ struct Ensemble {
   std::vector<int32_t> first_tree;
   const TreeNodeDev *nodes = nullptr;
   const int32_t *offsets = nullptr;
-  const int32_t *cols = nullptr, *class_slots = nullptr;
-  int32_t *depth = nullptr;
+  const int32_t *cols = nullptr, *ranges = nullptr, *groups = nullptr;
+  const int32_t *depth = nullptr;
 };
+
+// The lists that launch_walk_pack and launch_walk read beside the nodes, one
+// after the other from `first` to `end` (trees_max entries at most, see
+// walk_lists_bytes).
+struct WalkLists {
+  int32_t *first, *count, *dest, *ranges, *depth, *groups, *cols;
+  uint8_t *remap, *end;
+  int32_t n = 0;      // entries
+  int64_t slots = 0;  // node slots of all packed trees
+};
+
+// What they take at most for so many trees of K classes and engine columns.
+constexpr size_t walk_lists_bytes(size_t trees, size_t K, size_t cols) {
+  const size_t entries = trees + K * (kWalkMaxGroup + kWalkMaxTpl);
+  return (3 * entries + 2 * K + 1 + trees + std::min<size_t>(cols, kWalkMaxCols) + 1) * 4 + cols;
+}
+
+// Writes them at `at` for the plan's layout; tree(k, t) is class k's tree t as
+// {first node, nodes}.
+template <typename TreeFn>
+WalkLists walk_lists(void *at, const WalkPlan &p, const TreeShape &sh, int32_t K,
+                     const int32_t *n_trees, TreeFn tree) {
+  WalkLists L;
+  int64_t n = 0;
+  for (int32_t k = 0; k < K; ++k)
+    n = p.own ? n + n_trees[k] : round_up(round_up(n, p.per_group) + n_trees[k], p.tpl);
+  L.n = (int32_t)n;
+  L.first = static_cast<int32_t *>(at);
+  L.count = L.first + n;
+  L.dest = L.count + n;
+  L.ranges = L.dest + n;
+  L.depth = L.ranges + 2 * (size_t)K;
+  L.groups = L.depth + 1;
+  *L.depth = 0;  // what packing finds
+  int32_t n_groups = 0;
+  if (p.own) {
+    int32_t e = 0;
+    for (int32_t k = 0; k < K; ++k) {
+      L.ranges[2 * k] = n_groups;
+      int32_t used = kWalkGroupSlots;  // of the current group
+      for (int32_t t = 0; t < n_trees[k]; ++t, ++e) {
+        const auto [first, count] = tree(k, t);
+        int32_t slot = 4;
+        while (slot <= count) slot *= 2;
+        used = (int32_t)round_up(used, slot);
+        if (used + slot > kWalkGroupSlots) {
+          used = 0;
+          L.groups[n_groups++] = 0;
+        }
+        int32_t &group = L.groups[n_groups - 1];
+        if (group == 1) group |= used << 16;
+        ++group;
+        L.first[e] = first;
+        L.count[e] = count;
+        L.dest[e] = (int32_t)((int64_t)(n_groups - 1) * kWalkGroupSlots + used);
+        used += slot;
+      }
+      L.ranges[2 * k + 1] = n_groups;
+    }
+    L.slots = (int64_t)n_groups * kWalkGroupSlots;
+  } else {
+    // The entries between the classes and up to a multiple of tpl are empty.
+    std::memset(L.first, 0, 2 * (size_t)n * 4);
+    int64_t e = 0;
+    for (int32_t k = 0; k < K; ++k) {
+      e = round_up(e, p.per_group);
+      L.ranges[2 * k] = (int32_t)e;
+      for (int32_t t = 0; t < n_trees[k]; ++t, ++e) {
+        const auto [first, count] = tree(k, t);
+        L.first[e] = first;
+        L.count[e] = count;
+      }
+      e = round_up(e, p.tpl);
+      L.ranges[2 * k + 1] = (int32_t)e;
+    }
+    for (int64_t i = 0; i < n; ++i) L.dest[i] = (int32_t)(i * p.slot);
+    L.slots = n * p.slot;
+  }
+  L.cols = L.groups + n_groups;
+  L.remap = reinterpret_cast<uint8_t *>(L.cols + p.n_cols);
+  sh.columns(L.cols, L.remap);
+  L.end = L.remap + sh.n_cols;
+  return L;
+}
 
 // Checks the trees for matrices with M's features and tiers, uploads them
 // with their lists in one copy and packs them for a walk of n rows.
@@ -3414,15 +3497,10 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   std::vector<uint8_t> used((size_t)M.cols(), 0);
   TreeShape sh(used.data(), M.cols());
   // Built in pinned memory, a large one in its own, and copied from there:
-  // nodes, tree offsets, then the walk's lists (first node and node count of
-  // every slot, the classes' slots, the depth, the staged columns, every
-  // column's index among them).
+  // nodes, tree offsets, then the walk's lists.
   const size_t off_b = std::max<size_t>(total, 1) * sizeof(TreeNodeDev);
   const size_t list_b = off_b + (trees + 1) * 4;
-  const size_t slots_max = trees + (size_t)P.K * (kWalkMaxGroup + kWalkMaxTpl);
-  const size_t cols_max = (size_t)M.cols();
-  const size_t bytes_max =
-      list_b + (2 * slots_max + 2 * (size_t)P.K + 1 + cols_max + 1) * 4 + cols_max;
+  const size_t bytes_max = list_b + walk_lists_bytes(trees, (size_t)P.K, (size_t)M.cols());
   std::vector<char> large;
   char *stage = nullptr;
   if (bytes_max <= kArenaPiece) {
@@ -3474,37 +3552,15 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   offs[(size_t)tree] = (int32_t)base;
   en.walk = tree > 0 && plan_walk(sh, n, &en.plan);
 
-  int32_t *first = reinterpret_cast<int32_t *>(stage + list_b);
-  int32_t *count = nullptr, *slots = nullptr, *cols = nullptr;
-  uint8_t *remap = nullptr;
-  size_t n_slots = 0, bytes = list_b;
+  WalkLists L;
+  size_t bytes = list_b;
   if (en.walk) {
-    // Each class's slots from a multiple of per_group on; the slots between
-    // the classes and up to a multiple of tpl are empty.
-    const WalkPlan &p = en.plan;
-    for (int32_t k = 0; k < P.K; ++k)
-      n_slots = (size_t)round_up(round_up((int64_t)n_slots, p.per_group) +
-                                     P.n_trees[k], p.tpl);
-    count = first + n_slots;
-    slots = count + n_slots;
-    slots[2 * (size_t)P.K] = 0;  // the depth that packing finds
-    cols = slots + 2 * (size_t)P.K + 1;
-    remap = reinterpret_cast<uint8_t *>(cols + std::max(1, sh.n_used));
-    bytes = (size_t)(reinterpret_cast<char *>(remap) - stage) + cols_max;
-    std::memset(first, 0, 2 * n_slots * 4);
-    size_t at = 0;
-    for (int32_t k = 0; k < P.K; ++k) {
-      at = (size_t)round_up((int64_t)at, p.per_group);
-      slots[2 * (size_t)k] = (int32_t)at;
-      const int32_t t0 = en.first_tree[(size_t)k];
-      for (int32_t t = 0; t < P.n_trees[k]; ++t, ++at) {
-        first[at] = offs[(size_t)(t0 + t)];
-        count[at] = P.offsets[k][t + 1] - P.offsets[k][t];
-      }
-      at = (size_t)round_up((int64_t)at, p.tpl);
-      slots[2 * (size_t)k + 1] = (int32_t)at;
-    }
-    sh.columns(cols, remap);
+    L = walk_lists(stage + list_b, en.plan, sh, P.K, P.n_trees, [&](int32_t k, int32_t t) {
+      return std::pair<int32_t, int32_t>(offs[(size_t)(en.first_tree[(size_t)k] + t)],
+                                         P.offsets[k][t + 1] - P.offsets[k][t]);
+    });
+    bytes = (size_t)(reinterpret_cast<char *>(L.end) - stage);
+    if (L.slots > INT32_MAX) en.walk = false;  // (places of trees are 32-bit)
   }
   CHK(E->ens_d.ensure(bytes));
   if (large.empty())
@@ -3517,15 +3573,16 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
   en.nodes = reinterpret_cast<const TreeNodeDev *>(E->ens_d.p);
   en.offsets = reinterpret_cast<const int32_t *>(dev(offs));
   if (!en.walk) return BSSCL_OK;
-  en.class_slots = reinterpret_cast<const int32_t *>(dev(slots));
-  en.depth = reinterpret_cast<int32_t *>(dev(slots + 2 * (size_t)P.K));
-  en.cols = reinterpret_cast<const int32_t *>(dev(cols));
-  CHK(E->walk_words.ensure(n_slots * (size_t)en.plan.slot));
-  CHK(E->walk_vals.ensure(n_slots * (size_t)en.plan.slot));
-  HIPCHK(launch_walk_pack(E->st, en.nodes, reinterpret_cast<const int32_t *>(dev(first)),
-                          reinterpret_cast<const int32_t *>(dev(count)), (int32_t)n_slots,
-                          reinterpret_cast<const uint8_t *>(dev(remap)), lr, en.plan,
-                          E->walk_words.p, E->walk_vals.p, en.depth));
+  auto dev_i = [&](const int32_t *host) { return reinterpret_cast<int32_t *>(dev(host)); };
+  en.ranges = dev_i(L.ranges);
+  en.groups = dev_i(L.groups);
+  en.depth = dev_i(L.depth);
+  en.cols = dev_i(L.cols);
+  CHK(E->walk_words.ensure((size_t)L.slots));
+  CHK(E->walk_vals.ensure((size_t)L.slots));
+  HIPCHK(launch_walk_pack(E->st, en.nodes, dev_i(L.first), dev_i(L.count), dev_i(L.dest), L.n,
+                          reinterpret_cast<const uint8_t *>(dev(L.remap)), lr, en.plan,
+                          E->walk_words.p, E->walk_vals.p, dev_i(L.depth)));
   return BSSCL_OK;
 }
 
@@ -3538,10 +3595,9 @@ int run_ensemble(bsscl_engine *E, const Ensemble &en, const uint8_t *codes, int6
   hipEvent_t start, stop;
   if (en.walk) {
     CHK(prof_kernel(E, 4, &start, &stop));
-    WalkArgs a{codes,        ld,         n,          en.cols,
-               en.plan.n_cols, E->walk_words.p, E->walk_vals.p, en.class_slots, en.depth,
-               en.plan.slot, en.plan.per_group, out, out_stride,
-               reinterpret_cast<double2 *>(proba), base_score};
+    const WalkArgs a{codes, ld, n, en.cols, en.plan.n_cols, E->walk_words.p, E->walk_vals.p,
+                     en.ranges, en.groups, en.depth, en.plan.slot, en.plan.per_group,
+                     out, out_stride, reinterpret_cast<double2 *>(proba), base_score};
     HIPCHK(launch_walk(E->st, en.plan, a, en.K, start, stop));
     return BSSCL_OK;
   }
@@ -4822,39 +4878,32 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
   // stack, the used part of them copied; the copy has finished when the call
   // returns).
   WalkPlan plan;
-  if (n_trees > 0 && few_cols && plan_walk(sh, M.n, &plan) &&
-      round_up(n_trees, plan.tpl) * plan.slot <= kNoAllocWalkSlots) {
+  if (n_trees > 0 && few_cols && plan_walk(sh, M.n, &plan)) {
+    static_assert(kNoAllocLists == walk_lists_bytes(kNoAllocMaxTrees, 1, kNoAllocMaxCols),
+                  "the lists fit the scratch");
     alignas(8) unsigned char lists[kNoAllocLists];
-    const int32_t n_slots = (int32_t)round_up(n_trees, plan.tpl);
-    int32_t *first = reinterpret_cast<int32_t *>(lists);
-    int32_t *count = first + n_slots, *slots = count + n_slots, *depth = slots + 2;
-    int32_t *cols = depth + 1;
-    uint8_t *remap = reinterpret_cast<uint8_t *>(cols + plan.n_cols);
-    for (int32_t t = 0; t < n_slots; ++t) {
-      first[t] = t < n_trees ? offsets[t] : 0;
-      count[t] = t < n_trees ? offsets[t + 1] - offsets[t] : 0;
+    const WalkLists L =
+        walk_lists(lists, plan, sh, 1, &n_trees, [&](int32_t, int32_t t) {
+          return std::pair<int32_t, int32_t>(offsets[t], offsets[t + 1] - offsets[t]);
+        });
+    if (L.slots <= kNoAllocWalkSlots) {
+      HIPCHK(hipMemcpyAsync(S + kScrLists, lists, (size_t)(L.end - lists), hipMemcpyHostToDevice,
+                            E->st));
+      auto dev = [&](const void *host) {
+        return S + kScrLists + (static_cast<const unsigned char *>(host) - lists);
+      };
+      auto dev_i = [&](const int32_t *host) { return reinterpret_cast<int32_t *>(dev(host)); };
+      double *vals = reinterpret_cast<double *>(S + kScrWalk);
+      uint32_t *words = reinterpret_cast<uint32_t *>(vals + kNoAllocWalkSlots);
+      HIPCHK(launch_walk_pack(E->st, nodes, dev_i(L.first), dev_i(L.count), dev_i(L.dest), L.n,
+                              dev(L.remap), learning_rate, plan, words, vals, dev_i(L.depth)));
+      const WalkArgs a{M.codes.p, M.ld, M.n, dev_i(L.cols), plan.n_cols, words, vals,
+                       dev_i(L.ranges), dev_i(L.groups), dev_i(L.depth), plan.slot,
+                       plan.per_group, out_F_dev, M.n, nullptr, 0.0};
+      HIPCHK(launch_walk(E->st, plan, a, 1));
+      HIPCHK(hipStreamSynchronize(E->st));
+      return BSSCL_OK;
     }
-    slots[0] = 0;
-    slots[1] = n_slots;
-    *depth = 0;
-    sh.columns(cols, remap);
-    const size_t bytes = (size_t)(remap - lists) + (size_t)M.cols();
-    HIPCHK(hipMemcpyAsync(S + kScrLists, lists, bytes, hipMemcpyHostToDevice, E->st));
-    auto dev = [&](const void *host) {
-      return S + kScrLists + (static_cast<const unsigned char *>(host) - lists);
-    };
-    double *vals = reinterpret_cast<double *>(S + kScrWalk);
-    uint32_t *words = reinterpret_cast<uint32_t *>(vals + kNoAllocWalkSlots);
-    HIPCHK(launch_walk_pack(E->st, nodes, reinterpret_cast<const int32_t *>(dev(first)),
-                            reinterpret_cast<const int32_t *>(dev(count)), n_slots, dev(remap),
-                            learning_rate, plan, words, vals,
-                            reinterpret_cast<int32_t *>(dev(depth))));
-    const WalkArgs a{M.codes.p, M.ld, M.n, reinterpret_cast<const int32_t *>(dev(cols)),
-                     plan.n_cols, words, vals, reinterpret_cast<const int32_t *>(dev(slots)),
-                     reinterpret_cast<const int32_t *>(dev(depth)), plan.slot, plan.per_group, out_F_dev, M.n, nullptr, 0.0};
-    HIPCHK(launch_walk(E->st, plan, a, 1));
-    HIPCHK(hipStreamSynchronize(E->st));
-    return BSSCL_OK;
   }
   HIPCHK(launch_predict(E->st, M.codes.p, M.ld, M.n, nodes, offs, n_trees, learning_rate,
                         out_F_dev));

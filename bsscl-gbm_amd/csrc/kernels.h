@@ -507,33 +507,42 @@ constexpr int32_t kWalkCols4 = 52;
 // Up to this many rows the waves of a block share out the trees.
 constexpr int64_t kWalkSplitRows = 65536;
 constexpr int32_t kWalkMaxGroup = 256, kWalkMaxTpl = 8;  // limits of per_group and tpl below
+constexpr int32_t kWalkGroupSlots = 1024;  // node slots staged in LDS at a time
 struct WalkPlan {
-  int32_t slot;       // node slots of a tree: a power of two above the largest tree's nodes
-  int32_t per_group;  // trees staged in LDS at a time
+  int32_t slot;       // node slots of the largest tree: a power of two above its nodes
+  int32_t per_group;  // trees of that size staged at a time
   int32_t n_cols;     // columns staged per row
   int32_t rpl, tpl;   // rows of a lane, trees walked at once
   bool split;         // a block's waves walk different trees
+  bool own;           // every tree has slots for its own nodes only
   int32_t win;        // log2 bytes of the window of LDS that a tree's offsets are relative to
 };
 // The plan for n rows, n_cols distinct columns and trees of at most
-// max_nodes nodes; false when they do not fit.  A class's trees take slots
-// from a multiple of per_group on, their count rounded up to a multiple of
-// tpl (the rest of them with count 0 in launch_walk_pack).
+// max_nodes nodes; false when they do not fit.
+//
+// Where the trees lie (dest, in node slots).  Equal slots: entry i at i *
+// slot; a class's entries from a multiple of per_group on, their number
+// rounded up to a multiple of tpl (the rest of them with count 0).  Own
+// slots: groups of kWalkGroupSlots; a tree takes the power of two above its
+// nodes (at least 4), from a multiple of it on, and lies in one group, the
+// first one at its start; groups[g] is the trees of group g, with the slot of
+// its second tree in the upper half.
 bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan);
 // Raises *depth to the levels of splits of the deepest tree, where they matter.
 hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int32_t *first,
-                            const int32_t *count, int32_t n_slots, const uint8_t *remap,
-                            double lr, const WalkPlan &p, uint32_t *words, double *vals,
-                            int32_t *depth);
+                            const int32_t *count, const int32_t *dest, int32_t n_entries,
+                            const uint8_t *remap, double lr, const WalkPlan &p, uint32_t *words,
+                            double *vals, int32_t *depth);
 struct WalkArgs {
   const uint8_t *codes;  // feature-major, ld a multiple of 256
   int64_t ld, n;
   const int32_t *cols;  // the staged columns, ascending
   int32_t n_cols;
-  const uint32_t *words;  // launch_walk_pack's outputs, slot entries a tree
+  const uint32_t *words;  // launch_walk_pack's outputs
   const double *vals;
-  const int32_t *class_slots;  // class k has slots [class_slots[2k], class_slots[2k + 1])
-  const int32_t *depth;        // launch_walk_pack's
+  const int32_t *ranges;  // class k has entries (own slots: groups) [ranges[2k], ranges[2k + 1])
+  const int32_t *groups;  // (own slots)
+  const int32_t *depth;   // launch_walk_pack's
   int32_t slot, per_group;
   double *out;  // F of class k at out + k * out_stride
   int64_t out_stride;

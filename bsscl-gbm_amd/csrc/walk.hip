@@ -28,7 +28,8 @@
 // rows x 100 columns x 300 trees about 100 us, 673 with the walk in HBM.
 //
 // A tree's node slots are a power of two: the root in slot 0, its number of
-// levels in slot 1's word, pairs of children from slot 2 on; trees never
+// levels in slot 1's word (own slots: in the upper half the slot of the tree
+// kTpl trees on), pairs of children from slot 2 on; trees never
 // cross a window of 1 << kWin bytes.  Node word:
 //   bits 2 .. kWin - 1  the left child's byte offset in the window (a
 //                       multiple of 8, so the right child's is "or 4")
@@ -44,7 +45,7 @@ namespace bsscl {
 
 namespace {
 
-constexpr int kGroupNodes = 1024;  // node slots staged at a time
+constexpr int kGroupNodes = kWalkGroupSlots;
 static_assert(kWalkMaxNodes == kGroupNodes - 1, "slot 1 of a tree holds no node");
 constexpr int kValsAt = kGroupNodes * 4;  // LDS byte offsets
 constexpr int kCodesAt = kValsAt + kGroupNodes * 8;
@@ -76,28 +77,33 @@ using Quad = __attribute__((ext_vector_type(4))) uint32_t;
 
 }  // namespace
 
-// One wave per tree slot: tree s holds nodes [first[s], first[s] + count[s])
-// of `nodes` (a child's index is relative to first[s]).  count 0 is padding:
-// one leaf of value 0.0, which adds +0.0 to a sum that is never -0.0.  A
-// tree that is a single leaf gets a root over two copies of it.  The host
-// has checked that the nodes form a tree, so at most slot - 1 are reached.
+// One wave per entry: tree s is nodes [first[s], first[s] + count[s]) of
+// `nodes` (a child's index is relative to first[s]) and goes to slot dest[s].
+// count 0 is padding: one leaf of value 0.0, which adds +0.0 to a sum that is
+// never -0.0.  A tree that is a single leaf gets a root over two copies of it.
+// The host has checked that the nodes form a tree, so no slot past count[s]
+// is reached.
 __global__ __launch_bounds__(64) void k_walk_pack(
     const TreeNodeDev *__restrict__ nodes, const int32_t *__restrict__ first,
-    const int32_t *__restrict__ count, const uint8_t *__restrict__ remap, double lr,
-    int32_t slot, int32_t per_group, int32_t win, uint32_t *__restrict__ words,
-    double *__restrict__ vals, int32_t *__restrict__ depth) {
+    const int32_t *__restrict__ count, const int32_t *__restrict__ dest,
+    const uint8_t *__restrict__ remap, double lr, int32_t win, int32_t link,
+    uint32_t *__restrict__ words, double *__restrict__ vals, int32_t *__restrict__ depth) {
   __shared__ int32_t order[kGroupNodes];
   const int32_t s = (int32_t)blockIdx.x, lane = (int32_t)threadIdx.x;
   const TreeNodeDev *tree = nodes + first[s];
-  const int32_t cnt = count[s];
-  uint32_t *w = words + (int64_t)s * slot;
-  double *v = vals + (int64_t)s * slot;
+  const int32_t cnt = count[s], slot = cnt + 1, to = dest[s];
+  uint32_t *w = words + to;
+  double *v = vals + to;
   // The tree's byte offset in its window.
-  const uint32_t base = ((uint32_t)(s % per_group) * (uint32_t)slot * 4u) & ((1u << win) - 1u);
+  const uint32_t base = ((uint32_t)to * 4u) & ((1u << win) - 1u);
+  // (Read only when that tree lies in the same group.)
+  const uint32_t on = link > 0 && s + link < (int32_t)gridDim.x
+                          ? (uint32_t)(dest[s + link] & (kGroupNodes - 1)) << 16
+                          : 0u;
   if (cnt <= 0 || tree[0].feature < 0) {
     if (lane < 4) {
       // The root and both leaves: always left, to the left leaf.
-      w[lane] = lane == 1 ? 1u : (255u << 24) | (base + 8u);
+      w[lane] = lane == 1 ? on | 1u : (255u << 24) | (base + 8u);
       v[lane] = cnt > 0 ? __dmul_rn(lr, tree[0].value) : 0.0;
     }
     return;
@@ -139,7 +145,7 @@ __global__ __launch_bounds__(64) void k_walk_pack(
     __syncthreads();
   }
   if (lane == 0) {
-    w[1] = (uint32_t)d;
+    w[1] = on | (uint32_t)d;
     if (d > kDeepSteps) atomicMax(depth, d);
   }
 }
@@ -165,8 +171,15 @@ __device__ __forceinline__ void walk_rows(const WalkArgs &a) {
       lds_put(kCodesAt + (c << kTileLog2) + 16 * ch,
               *reinterpret_cast<const Quad *>(a.codes + col * a.ld + r));
   }
-  const int32_t t_end = a.class_slots[2 * cls + 1];
-  int32_t g0 = a.class_slots[2 * cls];
+  // Trees too large for eight at a time lie in slots of their own size, so
+  // that small ones beside them do not fill a group each (their groups are
+  // numbered, g0; else g0 is a group's first entry).  With the largest tree's
+  // slots for all: 1M rows through one tree of 511 splits and 2,000 stumps
+  // 4.7 ms, 0.95 so; 1,000 rows through 10 of 511 and 290 of 7 159 us and 78;
+  // trees of one size are level to 4% slower.
+  constexpr bool kOwn = kRpl == 1 && kTpl < 8;
+  const int32_t t_end = a.ranges[2 * cls + 1];
+  int32_t g0 = a.ranges[2 * cls];
   const uint32_t lane_at = (uint32_t)(tid * kRpl);
   auto code_at = [&](uint32_t w) {
     return ((w & kColMask) >> (kWin - kTileLog2)) | lane_at;
@@ -174,12 +187,13 @@ __device__ __forceinline__ void walk_rows(const WalkArgs &a) {
   // The next group's words and values wait in registers while a group is
   // walked.
   Quad pw[kWordLoads], pv[kValLoads];
-  int32_t cnt = 0;
+  int32_t cnt = 0;  // own slots: the group's record
   auto prefetch = [&]() {
-    cnt = min(a.per_group, t_end - g0);
-    const int nw = cnt * a.slot / 4, nv = cnt * a.slot / 2;
-    const Quad *sw = reinterpret_cast<const Quad *>(a.words + (int64_t)g0 * a.slot);
-    const Quad *sv = reinterpret_cast<const Quad *>(a.vals + (int64_t)g0 * a.slot);
+    cnt = kOwn ? a.groups[g0] : min(a.per_group, t_end - g0);
+    const int nw = kOwn ? kGroupNodes / 4 : cnt * a.slot / 4, nv = 2 * nw;
+    const int64_t from = kOwn ? (int64_t)g0 * kGroupNodes : (int64_t)g0 * a.slot;
+    const Quad *sw = reinterpret_cast<const Quad *>(a.words + from);
+    const Quad *sv = reinterpret_cast<const Quad *>(a.vals + from);
 #pragma unroll
     for (int q = 0; q < kWordLoads; ++q)
       if (tid + q * kThreads < nw) pw[q] = sw[tid + q * kThreads];
@@ -192,8 +206,11 @@ __device__ __forceinline__ void walk_rows(const WalkArgs &a) {
   for (int r = 0; r < kRpl; ++r) F[r] = 0.0;
   if (g0 < t_end) prefetch();
   while (g0 < t_end) {
-    const int32_t here = cnt;
-    const int nw = here * a.slot / 4, nv = here * a.slot / 2;
+    const int32_t here = kOwn ? cnt & 0xffff : cnt;
+    uint32_t next_at[kTpl];  // own slots: where the next trees start
+    next_at[0] = 0u;
+    if constexpr (kTpl > 1) next_at[1] = here > 1 ? (uint32_t)cnt >> 16 : 0u;
+    const int nw = kOwn ? kGroupNodes / 4 : here * a.slot / 4, nv = 2 * nw;
     __syncthreads();  // the previous group's walks are done
 #pragma unroll
     for (int q = 0; q < kWordLoads; ++q)
@@ -202,17 +219,23 @@ __device__ __forceinline__ void walk_rows(const WalkArgs &a) {
     for (int q = 0; q < kValLoads; ++q)
       if (tid + q * kThreads < nv) lds_put(kValsAt + 16 * (tid + q * kThreads), pv[q]);
     __syncthreads();
-    g0 += a.per_group;
+    g0 += kOwn ? 1 : a.per_group;
     if (g0 < t_end) prefetch();
     for (int32_t t = 0; t < here; t += kTpl) {
       int32_t steps = 2;
       uint32_t w[kTpl][kRpl], p[kTpl][kRpl], win[kTpl];
 #pragma unroll
       for (int j = 0; j < kTpl; ++j) {
-        const uint32_t at = (uint32_t)((t + j) * a.slot * 4);
+        const uint32_t at = kOwn ? next_at[j] * 4u : (uint32_t)((t + j) * a.slot * 4);
         win[j] = at & ~((1u << kWin) - 1u);
         const Quad top = lds_get<Quad>(at);  // root, levels, left and right child
-        steps = max(steps, __builtin_amdgcn_readfirstlane((int)top.y));
+        const int32_t top_y = __builtin_amdgcn_readfirstlane((int)top.y);
+        steps = max(steps, kOwn ? top_y & 0xffff : top_y);
+        if constexpr (kOwn) {
+          // (After the last tree: the first of this step's again; an odd
+          // last one is walked beside another and added alone.)
+          next_at[j] = t + kTpl + j < here ? (uint32_t)top_y >> 16 : next_at[0];
+        }
         const uint32_t thr = top.x >> 24;
         uint32_t c4;
         if constexpr (kRpl == 4) c4 = lds_get<uint32_t>(kCodesAt + code_at(top.x));
@@ -266,7 +289,8 @@ __device__ __forceinline__ void walk_rows(const WalkArgs &a) {
       for (int j = 0; j < kTpl; ++j)
 #pragma unroll
         for (int r = 0; r < kRpl; ++r)
-          F[r] = __dadd_rn(F[r], lds_get<double>(kValsAt + 2 * p[j][r]));
+          if (!kOwn || j == 0 || t + j < here)
+            F[r] = __dadd_rn(F[r], lds_get<double>(kValsAt + 2 * p[j][r]));
     }
   }
 #pragma unroll
@@ -316,9 +340,9 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_walk_split(WalkArgs a) {
   auto code_at = [&](uint32_t w) {
     return kCodes + (((w & kColMask) >> (kWin - 6)) | (uint32_t)lane);
   };
-  const int32_t t_end = a.class_slots[2 * cls + 1];
+  const int32_t t_end = a.ranges[2 * cls + 1];
   double F = 0.0;
-  for (int32_t g = a.class_slots[2 * cls]; g < t_end; g += kSplitTrees) {
+  for (int32_t g = a.ranges[2 * cls]; g < t_end; g += kSplitTrees) {
     // This wave's trees: slots [t0, t0 + nt), nt a multiple of kTpl or 0.  A
     // tree's words are relative to its window, and a group of trees starts
     // at a window.
@@ -406,16 +430,17 @@ bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
     p.split = n <= kWalkSplitRows && p.tpl == 8;
   }
   p.per_group = kGroupNodes / p.slot;
+  p.own = p.rpl == 1 && p.tpl < 8;
   return true;
 }
 
 hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int32_t *first,
-                            const int32_t *count, int32_t n_slots, const uint8_t *remap,
-                            double lr, const WalkPlan &p, uint32_t *words, double *vals,
-                            int32_t *depth) {
-  if (n_slots <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_walk_pack, dim3((unsigned)n_slots), dim3(64), 0, st, nodes, first, count,
-                     remap, lr, p.slot, p.per_group, p.win, words, vals, depth);
+                            const int32_t *count, const int32_t *dest, int32_t n_entries,
+                            const uint8_t *remap, double lr, const WalkPlan &p, uint32_t *words,
+                            double *vals, int32_t *depth) {
+  if (n_entries <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_walk_pack, dim3((unsigned)n_entries), dim3(64), 0, st, nodes, first, count,
+                     dest, remap, lr, p.win, p.own ? p.tpl : 0, words, vals, depth);
   return hipGetLastError();
 }
 

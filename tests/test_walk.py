@@ -145,3 +145,34 @@ def test_walk_of_chains(engine, n, splits, stay):
     engine.load_codes(1, codes)
     np.testing.assert_array_equal(engine.predict(1, n, p, 5, 0.1),
                                   om.predict_all_trees(codes, p, 5, 0.1))
+
+
+MIXED = {
+    "large_then_stumps": [511] + [1] * 700,
+    "one_per_group": [511, 400, 300, 511],
+    "exact_groups": [255, 255, 127, 127, 127, 127, 511, 255, 62],
+    "odd_tails": [255, 1, 1, 0, 200, 3, 300, 0],
+    "leaves_between": [300, 0, 0, 0, 255, 0, 130, 0],
+    "up_to_256_slots": [127, 1, 100, 0, 63, 64, 127, 5, 2],
+}
+
+
+@pytest.mark.parametrize("n", [257, 66_000, 400_011])
+@pytest.mark.parametrize("case", list(MIXED))
+def test_walk_of_mixed_sizes(engine, case, n):
+    """Trees of more than 127 nodes lie beside small ones in slots of their
+    own size: group ends, odd tails, classes of different sizes."""
+    splits = MIXED[case]
+    print(f"[case] walk of mixed sizes {case}: {n} rows", flush=True)
+    rng = np.random.default_rng(len(splits) + n)
+    codes = rng.integers(0, 250, (n, 11)).astype(np.uint8)
+    p = _pack([_tree(rng, s, 11, 250) for s in splits])
+    q = _pack([_tree(rng, s, 11, 250) for s in splits[::-1][:5]])
+    T, U = len(splits), len(splits[::-1][:5])
+    engine.load_codes(1, codes)
+    want = om.predict_all_trees(codes, p, T, 0.1)
+    np.testing.assert_array_equal(engine.predict(1, n, p, T, 0.1), want)
+    proba = engine.predict_proba_mc(1, n, [q, None, p], [U, 0, T], 0.1)
+    F = np.stack([om.predict_all_trees(codes, q, U, 0.1), np.zeros(n), want], 1)
+    e = np.exp(F - F.max(1, keepdims=True))
+    np.testing.assert_allclose(proba, e / e.sum(1, keepdims=True), rtol=1e-13, atol=1e-300)

@@ -3374,9 +3374,9 @@ struct TreeShape {
 };
 
 // (Test hook BSSCL_TEST_PREDICT_GLOBAL=1: every row walks the trees in HBM.)
-bool plan_walk(const TreeShape &sh, int64_t n, WalkPlan *plan) {
+bool plan_walk(const TreeShape &sh, int64_t n, int32_t K, WalkPlan *plan) {
   return sh.proper && !std::getenv("BSSCL_TEST_PREDICT_GLOBAL") &&
-         walk_plan(n, std::max(1, sh.n_used), sh.max_nodes, plan);
+         walk_plan(n, K, std::max(1, sh.n_used), sh.max_nodes, plan);
 }
 
 // An ensemble on the device: the nodes in the engine's columns, class k's
@@ -3550,7 +3550,7 @@ int upload_ensemble(bsscl_engine *E, const Matrix &M, const PackedTrees &P, doub
     en.first_tree[(size_t)k + 1] = tree;
   }
   offs[(size_t)tree] = (int32_t)base;
-  en.walk = tree > 0 && plan_walk(sh, n, &en.plan);
+  en.walk = tree > 0 && plan_walk(sh, n, P.K, &en.plan);
 
   WalkLists L;
   size_t bytes = list_b;
@@ -3648,11 +3648,13 @@ int predict_to_device(bsscl_engine *E, int32_t slot, const int16_t *features,
 // 100 trees: 3.6 ms in one chunk, 2.6 so (2.12 of them the upload); 10M x 50,
 // 500 trees: 44.0 ms in 256 MB chunks read back at the end, 39.2 so.  (More
 // copy threads, or a thread for the results alone, change neither, and chunks
-// evened out, whose last one is longer, make 10M x 50 2-3% slower.)  Up to
-// 16 MB go as one chunk, whatever their row count: a tail of some hundred
-// rows behind so short an upload costs every launch and event again (1,500 x
-// 28 in 1,024 + 476 rows 0.19 ms, in one chunk 0.12; 10,000 x 20, 10 trees
-// 0.42 and 0.14).
+// evened out, whose last one is longer, make 10M x 50 2-3% slower.)  The walk
+// is planned for a chunk's rows and takes longer than one launch over all of
+// them (1M 0.27 ms against 0.12, 10M 12.1 against 8.5), behind the upload
+// either way.  Up to 16 MB go as one chunk, whatever their row count: a tail
+// of some hundred rows behind so short an upload costs every launch and event
+// again (1,500 x 28 in 1,024 + 476 rows 0.19 ms, in one chunk 0.12; 10,000 x
+// 20, 10 trees 0.42 and 0.14).
 int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, int32_t F,
                  const double *edges_2d, int32_t edge_stride, const int32_t *bin_counts,
                  const int32_t *nan_bin_id, const PackedTrees &P, double lr, double base_score,
@@ -4878,7 +4880,7 @@ int bsscl_predict_noalloc(bsscl_engine *E, int32_t slot, const int16_t *features
   // stack, the used part of them copied; the copy has finished when the call
   // returns).
   WalkPlan plan;
-  if (n_trees > 0 && few_cols && plan_walk(sh, M.n, &plan)) {
+  if (n_trees > 0 && few_cols && plan_walk(sh, M.n, 1, &plan)) {
     static_assert(kNoAllocLists == walk_lists_bytes(kNoAllocMaxTrees, 1, kNoAllocMaxCols),
                   "the lists fit the scratch");
     alignas(8) unsigned char lists[kNoAllocLists];

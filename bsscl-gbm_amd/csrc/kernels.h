@@ -504,8 +504,13 @@ constexpr int32_t kWalkMaxCols = 208;  // 256 rows' codes and a group of trees: 
 // and a group of trees: 64 KB) a lane walks four rows, else one.
 constexpr int64_t kWalkRows4 = 400000;
 constexpr int32_t kWalkCols4 = 52;
-// Up to this many rows the waves of a block share out the trees.
-constexpr int64_t kWalkSplitRows = 65536;
+// Up to this many rows, times classes, the waves of a block share out the
+// trees.  Shared and not, us: 28 columns, 100 trees 19 and 28 at 65,000 rows, 32
+// and 34 at 131,000, 48 and 51 at 200,000; 50 columns, 500 trees 136 and 153 at
+// 131,000; 12 columns, 20 trees 8 and 8 at 98,000, 11 and 9 at 131,000; 24
+// columns, 40 trees of 5 classes 12 and 16 at 16,000, 28 and 23 at 49,000; 30
+// splits, 16 classes 14 and 13 at 8,000, 82 and 58 at 65,000.
+constexpr int64_t kWalkSplitRows = 131072;
 constexpr int32_t kWalkMaxGroup = 256, kWalkMaxTpl = 8;  // limits of per_group and tpl below
 constexpr int32_t kWalkGroupSlots = 1024;  // node slots staged in LDS at a time
 struct WalkPlan {
@@ -517,7 +522,7 @@ struct WalkPlan {
   bool own;           // every tree has slots for its own nodes only
   int32_t win;        // log2 bytes of the window of LDS that a tree's offsets are relative to
 };
-// The plan for n rows, n_cols distinct columns and trees of at most
+// The plan for n rows, K classes, n_cols distinct columns and trees of at most
 // max_nodes nodes; false when they do not fit.
 //
 // Where the trees lie (dest, in node slots).  Equal slots: entry i at i *
@@ -527,7 +532,7 @@ struct WalkPlan {
 // nodes (at least 4), from a multiple of it on, and lies in one group, the
 // first one at its start; groups[g] is the trees of group g, with the slot of
 // its second tree in the upper half.
-bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan);
+bool walk_plan(int64_t n, int32_t K, int32_t n_cols, int32_t max_nodes, WalkPlan *plan);
 // Raises *depth to the levels of splits of the deepest tree, where they matter.
 hipError_t launch_walk_pack(hipStream_t st, const TreeNodeDev *nodes, const int32_t *first,
                             const int32_t *count, const int32_t *dest, int32_t n_entries,

@@ -311,10 +311,8 @@ __global__ __launch_bounds__((1 << kTileLog2) / kRpl) void k_walk(WalkArgs a) {
 
 // The walk of few rows: the kSplitWaves waves of a block take 64 rows through
 // eight trees each at a time, so a request of some rows is not one wave's
-// walk of every tree (28 columns, 100 trees: 11 us at 64 rows and 20 at 65,000,
-// against 27 and 28 in k_walk's blocks; 50 columns, 500 trees: 37 and 77
-// against 120 and 125; from about 100,000 rows on the rows alone fill the
-// chip).
+// walk of every tree (28 columns, 100 trees: 11 us at 64 rows, 27 in k_walk's
+// blocks; where rows and classes alone fill the chip: kWalkSplitRows).
 // The leaves' values wait in LDS, in place of the words they were reached
 // by, and the first wave adds them in tree order.
 constexpr int kSplitWaves = 8, kSplitTrees = 8 * kSplitWaves;
@@ -408,7 +406,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_walk_split(WalkArgs a) {
 }
 #pragma clang fp contract(on)
 
-bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
+bool walk_plan(int64_t n, int32_t K, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
   if (n_cols < 1 || n_cols > kWalkMaxCols || max_nodes > kWalkMaxNodes) return false;
   WalkPlan &p = *plan;
   p.slot = 4;
@@ -427,7 +425,7 @@ bool walk_plan(int64_t n, int32_t n_cols, int32_t max_nodes, WalkPlan *plan) {
   } else {
     p.rpl = 1;
     p.tpl = p.slot <= kGroupNodes / 8 ? 8 : p.slot <= kGroupNodes / 2 ? 2 : 1;
-    p.split = n <= kWalkSplitRows && p.tpl == 8;
+    p.split = n * K <= kWalkSplitRows && p.tpl == 8;
   }
   p.per_group = kGroupNodes / p.slot;
   p.own = p.rpl == 1 && p.tpl < 8;

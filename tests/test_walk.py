@@ -56,6 +56,8 @@ CASES = {
     "skewed": (1000, 12, 9, [62, 100], {"skew": True}),
     "right_before_left": (1000, 12, 9, [40], {"loose": True}),
     "tile256_edge": (65536 + 257, 28, 9, [62], {}),
+    "shared_edge": (131072, 9, 9, [62, 5], {}),
+    "not_shared": (131072 + 257, 28, 9, [62], {}),
     "rows4": (400001, 52, 9, [62, 3], {}),
     "rows4_too_wide": (400001, 53, 5, [62], {}),
     "rows4_tile_edge": (400384, 30, 3, [62], {}),
@@ -126,7 +128,7 @@ def test_large_models_and_edges_pin_no_more(engine):
         eng.close()
 
 
-@pytest.mark.parametrize("n", [300, 70_001, 400_003])
+@pytest.mark.parametrize("n", [300, 131_201, 400_003])
 @pytest.mark.parametrize("splits", [9, 20, 21, 62, 130, 300, 511])
 @pytest.mark.parametrize("stay", [0.5, 0.97])
 def test_walk_of_chains(engine, n, splits, stay):
@@ -157,7 +159,7 @@ MIXED = {
 }
 
 
-@pytest.mark.parametrize("n", [257, 66_000, 400_011])
+@pytest.mark.parametrize("n", [257, 131_300, 400_011])
 @pytest.mark.parametrize("case", list(MIXED))
 def test_walk_of_mixed_sizes(engine, case, n):
     """Trees of more than 127 nodes lie beside small ones in slots of their

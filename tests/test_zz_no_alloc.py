@@ -100,14 +100,14 @@ def test_predict_noalloc_refuses(engine):
         engine.predict_noalloc(1, _subset(packed, 2), 2, 0.1, host.ctypes.data)
 
 
-# (rows, columns, bins, splits per tree): the walk by one wave per row tile
-# and by four rows a lane, codes in two tiers, trees that need a large window,
+# (rows, columns, bins, splits per tree): the walk by one row and by four rows
+# a lane, codes in two tiers, trees that need a large window,
 # and what the fixed scratch does not hold packed (walked in HBM): many small
 # trees beside one of 62 splits, more columns than the lists number.
 CASES = {
-    "65537_rows": (65_537, 20, 250, [62] * 30 + [3]),
+    "131073_rows": (131_073, 20, 250, [62] * 30 + [3]),
     "400000_rows": (400_000, 8, 250, [30] * 9),
-    "two_tiers": (70_001, 12, 400, [62, 9] * 6),
+    "two_tiers": (140_001, 12, 400, [62, 9] * 6),
     "large_trees": (3000, 12, 250, [300, 5, 511, 0]),
     "leaves": (300, 3, 250, [0]),
     "unpacked_small_trees": (2000, 12, 250, [62] + [1] * 16_383),

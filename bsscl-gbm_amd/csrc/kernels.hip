@@ -3488,7 +3488,9 @@ __device__ __forceinline__ int32_t traverse(const TreeNodeDev *__restrict__ tree
 constexpr int kUpdTreeLds = 1024;
 
 #pragma clang fp contract(off)
+// (NumPy's clip keeps a NaN, and so does the mean.)
 __device__ __forceinline__ double row_loss(double f, uint8_t yi) {
+  if (isnan(f)) return f;
   const double fc = fmin(fmax(f, -500.0), 500.0);
   double p = 1.0 / (1.0 + exp(-fc));
   p = fmin(fmax(p, 1e-15), 1.0 - 1e-15);
@@ -3505,7 +3507,7 @@ __device__ __forceinline__ double row_loss_gh(double f, uint8_t yi, double w, do
   g = __dmul_rn(w, __dsub_rn(p, (double)yi));
   h = __dmul_rn(__dmul_rn(w, p), __dsub_rn(1.0, p));
   const double pc = fmin(fmax(p, 1e-15), 1.0 - 1e-15);
-  return yi ? log(pc) : log(1.0 - pc);
+  return isnan(f) ? f : yi ? log(pc) : log(1.0 - pc);
 }
 
 // Raises out[0], out[1] to the block's largest |g| and h (bit patterns of

@@ -58,3 +58,26 @@ def test_multiclass_scores_round_twice(monkeypatch, path):
         for t in m.mc_trees[k]:
             F[:, k] = F[:, k] + m.learning_rate * om.predict_tree(codes, t)
     np.testing.assert_array_equal(est_mod._engine(0).mc_scores(), F)
+
+
+@pytest.mark.parametrize("start", [np.nan, np.inf, -np.inf, 600.0])
+@pytest.mark.parametrize("path", ["pipelined", "host_replay"])
+def test_validation_loss_of_scores_past_the_clip(monkeypatch, path, start):
+    """A NaN score gives a NaN loss, as np.clip and the mean keep it;
+    infinities are clipped."""
+    from bsscl_gbm import HybridHistGBMNumbaV1_0_1, _native
+    print(f"[case] validation scores from {start}, {path}", flush=True)
+    _mode(monkeypatch, path)
+    begin = _native.Engine.boost_val_begin
+    monkeypatch.setattr(_native.Engine, "boost_val_begin",
+                        lambda self, y, base: begin(self, y, start))
+    X, y = make_data(3000, 6, seed=9)
+    m = HybridHistGBMNumbaV1_0_1(n_estimators=3, max_depth=3, random_state=1, verbose=False)
+    m.fit(X, y, eval_set=[(X[:700], y[:700])])
+    codes = om.bin_features(X[:700], m.bin_edges, m.feature_bin_counts, m._nan_bin_id, "standard")
+    F, want = np.full(700, start), []
+    for t in m.trees:
+        F = F + m.learning_rate * om.predict_tree(codes, t)
+        want.append(om.binary_logloss(y[:700], F))
+    np.testing.assert_allclose(m.val_loss_history_, want, rtol=1e-13, atol=0)
+    assert np.isfinite(m.train_loss_history_).all()

@@ -725,7 +725,8 @@ class HybridHistGBMNumbaV1_0_1:
         w0, w1, self.base_score_ = binary_start
         eng.boost_begin(y, w0, w1, self.base_score_)
         if n_val:
-            eng.boost_val_begin(y_val, self.base_score_)
+            # (NumPy's loss expression takes one label for all rows, too.)
+            eng.boost_val_begin(np.broadcast_to(y_val, n_val), self.base_score_)
         best_val_loss = np.inf
         rounds_no_improve = 0
         hook = getattr(self, '_round_hook', None)

@@ -81,3 +81,16 @@ def test_validation_loss_of_scores_past_the_clip(monkeypatch, path, start):
         want.append(om.binary_logloss(y[:700], F))
     np.testing.assert_allclose(m.val_loss_history_, want, rtol=1e-13, atol=0)
     assert np.isfinite(m.train_loss_history_).all()
+
+
+def test_one_validation_label_for_all_rows():
+    """A single label stands for every validation row; other lengths that
+    differ from the rows are refused."""
+    from bsscl_gbm import HybridHistGBMNumbaV1_0_1
+    X, y = make_data(2000, 5, seed=10)
+    kw = dict(n_estimators=4, max_depth=3, random_state=1, verbose=False)
+    one = HybridHistGBMNumbaV1_0_1(**kw).fit(X, y, eval_set=[(X[:50], [1])])
+    full = HybridHistGBMNumbaV1_0_1(**kw).fit(X, y, eval_set=[(X[:50], np.ones(50, int))])
+    assert one.val_loss_history_ == full.val_loss_history_
+    with pytest.raises(ValueError):
+        HybridHistGBMNumbaV1_0_1(**kw).fit(X, y, eval_set=[(X[:50], y[:49])])

@@ -451,6 +451,7 @@ struct bsscl_engine {
 
   // A multiclass round's further lanes (buffers are released with the engine).
   TreeLane mc_lane[kMcLanesMax - 1];
+  bool mc_one_lane = false;  // this run's second lane did not fit
   hipEvent_t mc_fork = nullptr;
 
   // Tree workspace.
@@ -3078,9 +3079,11 @@ int mc_tree_host(bsscl_engine *E, int32_t k, const std::vector<int32_t> &feats,
 // four hardware queues also serve the rows, the copies and the caller), and
 // so does the rows stream as the third (24.5).  A tree of more than
 // kLevelsPerCheck levels reads its plan back on the way and a profiled one is
-// timed by itself: one lane.  (Test hook BSSCL_TEST_MC_LANES=1: one lane.)
+// timed by itself: one lane, and so are the rounds of a run whose second lane
+// did not fit the memory.  (Test hook BSSCL_TEST_MC_LANES: 1 for one lane,
+// nomem for no memory.)
 int32_t mc_lanes(const bsscl_engine *E, int32_t K, const TreeParams &tp) {
-  if (E->prof > 0 || tp.max_depth > kLevelsPerCheck) return 1;
+  if (E->prof > 0 || tp.max_depth > kLevelsPerCheck || E->mc_one_lane) return 1;
   const char *t = std::getenv("BSSCL_TEST_MC_LANES");
   return t && t[0] == '1' ? 1 : std::min(K, kMcLanesMax);
 }
@@ -3113,6 +3116,17 @@ class TreeLanes {
     if (n_ > 1 && !E_->mc_fork)
       HIPCHK(hipEventCreateWithFlags(&E_->mc_fork, hipEventDisableTiming));
     return BSSCL_OK;
+  }
+  // Gives the further lanes' memory back and goes on with lane 0 alone.
+  void drop() {
+    use(0);
+    for (int32_t i = 1; i < n_; ++i) {
+      lane_buffers(lane(i), lane(i), [](auto &b, auto &) { b.release(); });
+      lane(i).node_alloc = lane(i).node_cap = 0;
+      lane(i).plan_d = nullptr;
+      lane(i).nodes_d = nullptr;
+    }
+    n_ = 1;
   }
   int fork() {
     if (n_ < 2) return BSSCL_OK;
@@ -3184,13 +3198,25 @@ int mc_trees_device(bsscl_engine *E, const std::vector<int32_t> &feats,
     bsscl_engine *e;
     ~RootReset() { e->root_set = -1; }
   } root_reset{E};
-  const int32_t n_lanes = shared_root ? mc_lanes(E, K, tp) : 1;
+  int32_t n_lanes = shared_root ? mc_lanes(E, K, tp) : 1;
   TreeLanes lanes(E, n_lanes);
   CHK(lanes.create());
   for (int32_t i = 0; i < n_lanes; ++i) {
     lanes.use(i);
-    CHK(E->tree_d.ensure((size_t)M));
-    CHK(prepare_tree_buffers(E, m, F_sel, std::max(1, tp.max_depth), tp.max_leaves));
+    int rc = E->tree_d.ensure((size_t)M);
+    if (rc == BSSCL_OK)
+      rc = prepare_tree_buffers(E, m, F_sel, std::max(1, tp.max_depth), tp.max_leaves);
+    const char *hook = std::getenv("BSSCL_TEST_MC_LANES");
+    if (i > 0 && hook && hook[0] == 'n') rc = BSSCL_ENOMEM;
+    if (i > 0 && rc == BSSCL_ENOMEM) {
+      // The trees fit one after the other.
+      (void)hipGetLastError();
+      lanes.drop();
+      E->mc_one_lane = true;
+      n_lanes = 1;
+      break;
+    }
+    CHK(rc);
   }
   lanes.use(0);
   PreRoot pre;
@@ -4446,6 +4472,7 @@ int bsscl_mc_begin(bsscl_engine *E, const int64_t *y, int64_t n, int32_t n_class
   E->mc_K = n_classes;
   E->mc_m = 0;
   E->mc_rows32 = nullptr;
+  E->mc_one_lane = false;
   // h = w p (1 - p) <= w / 4, floored at 1e-8 (est:3019).
   E->mc_hbound = std::max(0.25 * wmax, 1e-8);
   E->node_cap_floor = 0;  // a new fit starts from the node table its trees' shape asks for

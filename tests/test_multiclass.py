@@ -391,6 +391,25 @@ def test_multiclass_lanes_agree(monkeypatch, n, K, depth):
 
 
 @pytest.mark.gpu
+def test_multiclass_second_lane_without_memory(monkeypatch):
+    """A fit whose second lane does not fit the memory builds its trees in one
+    lane, the same ones, and the next fit has two again."""
+    from bsscl_gbm import HybridHistGBMNumbaV1_0_1
+    X, y = _mc_data(5000, 8, 4, seed=77)
+    fits = []
+    for lanes in ("1", "nomem", "2"):
+        monkeypatch.setenv("BSSCL_TEST_MC_LANES", lanes)
+        fits.append(HybridHistGBMNumbaV1_0_1(verbose=False, n_estimators=5, max_depth=5,
+                                             random_state=4).fit(X, y))
+    for got in fits[1:]:
+        assert got.train_loss_history_ == fits[0].train_loss_history_
+        for k in range(4):
+            for a, b in zip(fits[0].mc_trees[k], got.mc_trees[k]):
+                for i in (0, 1, 2, 3, 4, 6):
+                    np.testing.assert_array_equal(a[i][:a[5]], b[i][:a[5]])
+
+
+@pytest.mark.gpu
 def test_multiclass_round_ahead_handed_back(engine):
     """An early-stopped multiclass fit leaves a round taken ahead by the
     engine; the fit hands it back before closing its sampler, and the next

@@ -1484,9 +1484,11 @@ void read_hist_tuning(bsscl_engine *E, int64_t m, int32_t F_sel) {
   // The root: at least 10240 rows per tile (1M x 28, 73 tiles and half the
   // partials of 5120-row tiles: 2440 -> 2480 trees/s; at 10M x 50 the block
   // target decides, 227 tiles either way).
-  // Up to 256k rows such tiles leave the root too few blocks: 2560 there
-  // (the smallest tile, 4096 rows, is then the line; 100,000 x 100, 300
-  // rounds 73.9 -> 73.1 ms, 285k x 30 with validation 36.2 -> 35.5).
+  // Such tiles leave the root of a smaller tree too few blocks: 2560 up to
+  // 256k rows (the smallest tile, 4096 rows, is then the line).  Training of 60
+  // rounds with 10240 and 2560, 28 columns: 15,000 rows 12.1 and 11.5 ms,
+  // 75,000 13.3 and 12.9 (100 columns 15.1 and 14.8); level within 1% from
+  // 150,000 (14.0 and 14.0) to 375,000 (17.0 and 17.1).
   E->hist_rows_per_flush =
       env_int("BSSCL_HIST_ROWS_PER_FLUSH", 256, 1 << 22, m <= (1 << 18) ? 2560 : 10240);
   // Below the root, smaller tiles (more blocks for the smaller levels, more

@@ -199,7 +199,7 @@ def run_gpu(name, steps, warmup, rounds_only=False):
 
 
 CPU_PREDICT_ROWS = 200_000
-E2E_CALLS = 9  # timed predict_proba calls of a batch
+E2E_CALLS, E2E_WARMUP = 15, 5  # timed and earlier predict_proba calls of a batch
 
 
 def run_predict(model, name, repeats=3):
@@ -222,11 +222,11 @@ def run_predict(model, name, repeats=3):
     # its first calls meet several of them.  The walk's launches are counted
     # and timed in calls of their own.
     times = []
-    for _ in range(1 + E2E_CALLS):  # the first one warms up
+    for _ in range(E2E_WARMUP + E2E_CALLS):
         t = time.perf_counter()
         model.predict_proba(Xp)
         times.append(time.perf_counter() - t)
-    t_total = float(np.median(times[1:]))
+    t_total = float(np.median(times[E2E_WARMUP:]))
     eng.set_profiling(1)
     for _ in range(repeats):
         model.predict_proba(Xp)

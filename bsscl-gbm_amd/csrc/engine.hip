@@ -1523,7 +1523,8 @@ int prepare_tree_buffers(bsscl_engine *E, int64_t m, int32_t F_sel, int32_t leve
   // Partition tiles: eight rows per thread where that gives the root at
   // least 512 tiles, else four (wider tiles left CUs idle at 1M).  Sixteen at
   // 10M x 50: the scatter 140 us a level against 125, the planner's counts 12
-  // against 15, whole fits of 100 rounds 327 ms against 321.
+  // against 15 (whole fits are level within their spread: the rows stream
+  // beside the tree takes the difference).
   E->part_rows = m / (8 * (int64_t)kPartThreads) < 512 ? 4 : 8;
   E->part_tile = kPartThreads * E->part_rows;
   // A tile's features are shared out over blocks until about 1,024 blocks

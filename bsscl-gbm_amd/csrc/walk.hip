@@ -23,14 +23,14 @@
 //     take eight trees at a time instead.
 // LDS reads then set the rate, about four clocks each per CU: 7 clocks per
 // wave and step at 28 columns.  Measured (125-node trees of depth 6): 1M rows
-// x 28 columns x 100 trees 117 us, where lanes that stopped at
-// their leaf and column-strided codes (23 clocks a step) took 357; 100,000
-// rows x 100 columns x 300 trees about 100 us, 673 with the walk in HBM.
+// x 28 columns x 100 trees 117 us, where lanes that stopped at their leaf and
+// column-strided codes (23 clocks a step) took 357; 100,000 rows x 100 columns
+// x 300 trees 68 us (k_walk_split), 673 with the walk in HBM.
 //
 // A tree's node slots are a power of two: the root in slot 0, its number of
 // levels in slot 1's word (own slots: in the upper half the slot of the tree
-// kTpl trees on), pairs of children from slot 2 on; trees never
-// cross a window of 1 << kWin bytes.  Node word:
+// kTpl trees on), pairs of children from slot 2 on; trees never cross a window
+// of 1 << kWin bytes.  Node word:
 //   bits 2 .. kWin - 1  the left child's byte offset in the window (a
 //                       multiple of 8, so the right child's is "or 4")
 //   bits kWin .. 23     the column

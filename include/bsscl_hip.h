@@ -301,8 +301,8 @@ int bsscl_predict_proba(bsscl_engine *eng, int32_t slot, const int16_t *features
  * The whole of a binary model's predict_proba from host rows: binning X
  * (est:3289, as bsscl_bin_features with the same edges, bin counts and NaN
  * bins), the walk and the probabilities (est:3318-3336, as
- * bsscl_predict_proba), with identical results.  X streams through the
- * device in row chunks of 8 to 64 MB: a chunk's upload runs while the
+ * bsscl_predict_proba), with identical results.  Up to 16 MB of X go as one
+ * chunk, more in row chunks of 8 to 64 MB: a chunk's upload runs while the
  * device bins and walks the chunk before it.  Leaves matrix slots 0 and 1
  * as they were.
  */

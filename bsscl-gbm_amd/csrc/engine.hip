@@ -3705,7 +3705,9 @@ int predict_rows(bsscl_engine *E, const void *X, int32_t x_is_f64, int64_t n, in
   if (total_b > kOneChunkBytes || n > rows_max) {
     const size_t chunk_b = std::min<size_t>(std::max<size_t>(total_b / 8, 8u << 20), 64u << 20);
     rows_c = round_up((int64_t)std::max<size_t>(1, chunk_b / row_b), 1024);
-    rows_c = std::min(n, std::min(rows_max, rows_c));
+    // (64 MB are sixteen pieces of an upload, a little more one of some KB.)
+    rows_max = std::min(rows_max, (int64_t)((64u << 20) / row_b) / 1024 * 1024);
+    rows_c = std::min(n, std::max<int64_t>(1024, std::min(rows_max, rows_c)));
   }
   // A request of up to 1 MB goes through the arena on the engine's stream
   // alone; from there on the rows stream carries X while the engine's takes

@@ -39,6 +39,11 @@ class DeviceBuffer:
         self._copy(out.ctypes.data_as(ctypes.c_void_p), self.p, 2)  # device -> host
         return out
 
+    def free_memory(self):
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert self.hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
     def close(self):
         if self.p:
             self.hip.hipFree(self.p)
@@ -111,6 +116,7 @@ CASES = {
     "large_trees": (3000, 12, 250, [300, 5, 511, 0]),
     "leaves": (300, 3, 250, [0]),
     "unpacked_small_trees": (2000, 12, 250, [62] + [1] * 16_383),
+    "unpacked_large_trees": (2000, 12, 250, [0, 256] * 150),
     "many_columns": (300, 4200, 250, [62] * 5),
 }
 
@@ -127,6 +133,9 @@ def test_predict_noalloc_walks(engine, case):
     out = DeviceBuffer(n)
     try:
         engine.predict_noalloc(1, p, len(splits), 0.1, out.p.value)
+        free = out.free_memory()  # (the first call may have loaded kernels)
+        engine.predict_noalloc(1, p, len(splits), 0.1, out.p.value)
+        assert out.free_memory() == free
         got = out.read()
     finally:
         out.close()
